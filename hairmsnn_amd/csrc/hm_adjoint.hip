@@ -192,11 +192,7 @@ HM_D bool adj_vertex(const SceneView& sc, const AdjArgs& a, TraceStack& st, floa
 __global__ void __launch_bounds__(kTraceBlock, HM_ADJ_MIN_WAVES) k_adjoint(SceneView sc, AdjArgs a) {
   __shared__ int lds_stack[kStackLds * kTraceBlock];
   TraceStack st;
-  st.lds = lds_stack + threadIdx.x;
-  st.spill = a.spill + blockIdx.x * blockDim.x + threadIdx.x;
-  st.spill_stride = a.spill_stride;
-  st.spill_levels = a.spill_levels;
-  st.sp = 0;
+  st.init(lds_stack, a.spill + blockIdx.x * blockDim.x + threadIdx.x, a.spill_stride, a.spill_levels);
   const int npx = sc.width * sc.height;
   const long long total = (long long)npx * a.npass;
   float gg[3] = {0.f, 0.f, 0.f};

@@ -266,7 +266,7 @@ PassConfig Context::pt_pass_config() const {
     c.dl_zero = 0;
     c.dl_from = 1 << 30;
   }
-  c.trace_blocks = trace_blocks;
+  c.trace_blocks = ray_blocks;
   c.shade_blocks = std::max(64, num_cus * 8);
   return c;
 }
@@ -283,15 +283,10 @@ int Context::init(std::string& err) {
   HM_HIP(hipGetDeviceProperties(&prop, dev), err);
   num_cus = prop.multiProcessorCount;
   // traversal blocks resident per CU: 8 (8 waves per SIMD), fewer when the
-  // blocks' LDS stacks do not fit the CU's 160 KB together; the traversal
-  // grid is that many blocks per CU unless HM_TRACE_GRID_PER_CU says more
+  // blocks' LDS stacks do not fit the CU's 160 KB together
   const int lds_blocks = (160 * 1024) / (kStackLds * kTraceBlock * (int)sizeof(int));
-  const int resident = std::max(1, std::min(8, lds_blocks));
-#ifdef HM_TRACE_GRID_PER_CU
-  trace_blocks = std::max(64, num_cus * HM_TRACE_GRID_PER_CU);
-#else
-  trace_blocks = std::max(64, num_cus * resident);
-#endif
+  trace_blocks = std::max(64, num_cus * std::max(1, std::min(8, lds_blocks)));
+  ray_blocks = std::min(trace_blocks, std::max(64, num_cus * kRayBlocksPerCu));
 
   // ---- geometry ----
   if ((int)scene.dlight_from.size() > kMaxDirLights) {
@@ -1028,7 +1023,7 @@ int hmsnn_trace_rays_dev(hmsnn_ctx* ctx, const float* rays, int n, int any_hit, 
   int rc = c.ensure_path_buffers(false, err);
   if (rc) return fail(rc, err);
   rc = trace_rays(c.view, rays, n, any_hit, prim, t, u, c.pb.spill, c.pb.spill_stride, c.pb.spill_levels,
-                  c.trace_blocks, nullptr, c.stream, err);
+                  c.ray_blocks, nullptr, c.stream, err);
   if (rc) return fail(rc, err);
   hipError_t e = hipStreamSynchronize(c.stream);
   return e == hipSuccess ? HMSNN_OK : fail(HMSNN_EDEVICE, std::string("trace rays: ") + hipGetErrorString(e));

@@ -1,12 +1,11 @@
 // Device-side BVH view and traversal (closest hit and any hit).
 //
-// Layout in HBM: the Karras LBVH is built binary (64-byte nodes holding both
-// children's boxes) and then collapsed into wide nodes (BvhNodeWide, 4 or 8
-// children) that traversal reads; segments are 32-byte records in Morton
-// order. A child index >= 0 is an inner node, < 0 codes a leaf: a run of
+// Layout in HBM: the tree is built binary (64-byte nodes holding both
+// children's boxes) and then collapsed into four-wide nodes (BvhNodeWide)
+// that traversal reads; segments are 32-byte records in leaf order. A child index >= 0 is an inner node, < 0 codes a leaf: a run of
 // consecutive positions of the segment array (leaf_code).
 //
-// Traversal is one ray per lane (wave64). The stack's top kStackLds entries
+// Traversal is one ray per lane (wave64). The stack's lowest kStackLds entries
 // live in LDS, one column per lane (conflict-free), deeper entries spill to a
 // per-thread global area sized from the wide tree's depth at build time.
 #pragma once
@@ -24,23 +23,22 @@ struct BvhNode {
   int4 d;    // child0, child1, unused, unused
 };
 
-// Wide node of kBvhWidth children (4: 128 bytes, 8: 224 bytes): child boxes
-// as structure-of-arrays, so one node fetch is a run of 16-byte loads that
-// decides all children. child[k] >= 0 is an inner node, < 0 is ~segment
-// position (leaf), kEmptyChild an unused slot (its box is never tested).
-#ifndef HM_BVH_WIDTH
-#define HM_BVH_WIDTH 4
-#endif
-constexpr int kBvhWidth = HM_BVH_WIDTH;
-static_assert(kBvhWidth == 4 || kBvhWidth == 8, "4- or 8-wide nodes");
-struct __attribute__((aligned(16))) BvhNodeWide {
-  float lox[kBvhWidth], loy[kBvhWidth], loz[kBvhWidth];
-  float hix[kBvhWidth], hiy[kBvhWidth], hiz[kBvhWidth];
+// Four-wide node of one 128-byte line: per axis the four children's lower
+// planes, then their upper planes. A ray picks the 16-byte half that holds
+// the near planes of an axis by the sign of its direction, so the slab test
+// needs no min / max per plane. child[k] >= 0 is an inner node, < 0 codes a
+// leaf (leaf_code). An unused slot has an inverted box, which no ray enters;
+// its child code is leaf 0, so that even a ray with non-finite
+// components only tests a primitive that exists.
+constexpr int kBvhWidth = 4;
+struct __attribute__((aligned(128))) BvhNodeWide {
+  float x[2 * kBvhWidth], y[2 * kBvhWidth], z[2 * kBvhWidth];
   int child[kBvhWidth];
-  int pad[kBvhWidth == 4 ? 4 : 0];  // 4-wide: one 128-byte line; 8-wide: 224 bytes
+  int pad[4];
 };
-constexpr int kEmptyChild = 0x7fffffff;
-
+static_assert(sizeof(BvhNodeWide) == 128, "one cache line per node");
+constexpr int kEmptyChild = ~0;
+constexpr float kEmptyLo = 3e38f, kEmptyHi = -3e38f;
 
 struct BvhView {
   const BvhNodeWide* nodes;  // wide tree, root at 0
@@ -64,24 +62,18 @@ struct MeshView {
 };
 
 // Stack entries per lane kept in LDS (4 bytes x 256 lanes each per block).
-#ifndef HM_STACK_LDS
-#define HM_STACK_LDS 16
-#endif
-constexpr int kStackLds = HM_STACK_LDS;
+constexpr int kStackLds = 16;
 constexpr int kTraceBlock = 256;
+// Blocks per CU of a ray stream's grid. Each lane should get several rays, or
+// a wave has nothing to refill from: a million rays over 8, 6, 4, 3 and 2
+// blocks per CU measured 636, 659, 525, 535 and 679 us.
+constexpr int kRayBlocksPerCu = 4;
 
-// Launch bounds of the traversal kernels: 256 threads, and a floor of
-// HM_TRACE_MIN_WAVES waves per SIMD (the register budget follows from it).
-#ifndef HM_TRACE_MIN_WAVES
-#define HM_TRACE_MIN_WAVES 8
-#endif
-#define HM_TRACE_BOUNDS __launch_bounds__(kTraceBlock, HM_TRACE_MIN_WAVES)
-// Traversal kernels over round curves: the curve iteration needs more
-// registers than the segment test, fewer waves.
-#ifndef HM_CURVE_MIN_WAVES
-#define HM_CURVE_MIN_WAVES 4
-#endif
-#define HM_TRACE_BOUNDS_T(curves) __launch_bounds__(kTraceBlock, (curves) ? HM_CURVE_MIN_WAVES : HM_TRACE_MIN_WAVES)
+// Launch bounds of the traversal kernels: 256 threads and a floor of waves per
+// SIMD, which sets the register budget. Segments: 8 (the ray streams launch
+// four waves per SIMD, so that two streams' launches run side by side); the
+// round-curve iteration needs more registers.
+#define HM_TRACE_BOUNDS_T(curves) __launch_bounds__(kTraceBlock, (curves) ? 4 : 8)
 
 struct TraceCounters {
   uint32_t nodes;
@@ -94,6 +86,7 @@ struct TraceCounters {
 struct RayInv {
   float ox, oy, oz, dx, dy, dz;
   float ix, iy, iz, oix, oiy, oiz;
+  unsigned nx, ny, nz;  // byte offsets of the near planes in a node, per axis
 };
 
 HM_D float safe_inv(float d) {
@@ -107,93 +100,142 @@ HM_D RayInv make_ray(float ox, float oy, float oz, float dx, float dy, float dz)
   r.dx = dx; r.dy = dy; r.dz = dz;
   r.ix = safe_inv(dx); r.iy = safe_inv(dy); r.iz = safe_inv(dz);
   r.oix = ox * r.ix; r.oiy = oy * r.iy; r.oiz = oz * r.iz;
+  r.nx = __float_as_int(r.ix) < 0 ? 16u : 0u;
+  r.ny = __float_as_int(r.iy) < 0 ? 48u : 32u;
+  r.nz = __float_as_int(r.iz) < 0 ? 80u : 64u;
   return r;
 }
 
-// Slab test against [0, tmax]; returns the entry distance, or NaN on a miss
-// so that every ordered comparison with it is false (a +inf sentinel would
-// pass `t <= best_t` while nothing has been hit yet).
-HM_D float box_enter(const RayInv& r, float lx, float ly, float lz, float hx, float hy, float hz,
-                     float tmax) {
-  const float tx0 = fmaf(lx, r.ix, -r.oix), tx1 = fmaf(hx, r.ix, -r.oix);
-  const float ty0 = fmaf(ly, r.iy, -r.oiy), ty1 = fmaf(hy, r.iy, -r.oiy);
-  const float tz0 = fmaf(lz, r.iz, -r.oiz), tz1 = fmaf(hz, r.iz, -r.oiz);
-  const float tn = fmaxf(fmaxf(fminf(tx0, tx1), fminf(ty0, ty1)), fmaxf(fminf(tz0, tz1), 0.f));
-  const float tf = fminf(fminf(fmaxf(tx0, tx1), fmaxf(ty0, ty1)), fminf(fmaxf(tz0, tz1), tmax));
-  return tn <= tf ? tn : __builtin_nanf("");
-}
+typedef __attribute__((address_space(3))) char lds_char;
+typedef __attribute__((address_space(3))) int lds_int;
 
+// Traversal stack of one lane: kStackLds entries in LDS, entry k of lane
+// thread t of the block at byte 1024 k + 4 t (conflict-free), then
+// spill_levels entries in memory. The LDS pointer keeps its address space,
+// so the accesses are LDS instructions (through a generic pointer they were
+// flat ones, which go through the vector memory path that the node loads
+// need).
 struct TraceStack {
-  int* lds;       // this lane's column base: lds[k * kTraceBlock]
-  int* spill;     // global spill base for this thread
+  static constexpr int kLevel = kTraceBlock * (int)sizeof(int);
+  lds_char* lds;     // the block's stacks
+  int off;           // byte offset of the lane's next free entry
+  int* spill;        // this thread's spill column
   int spill_stride;
-  int spill_levels;  // capacity of the spill area (entries per thread)
-  int sp;
+  int spill_levels;
+  HM_D void init(int* block_stacks, int* spill_column, int stride, int levels) {
+    lds = (lds_char*)block_stacks;
+    off = 4 * (int)threadIdx.x;
+    spill = spill_column;
+    spill_stride = stride;
+    spill_levels = levels;
+  }
+  HM_D void clear() { off &= kLevel - 1; }
+  HM_D bool empty() const { return off < kLevel; }
+  HM_D lds_int* at(int o) const { return (lds_int*)(lds + o); }
+  // Whether every active lane has room for three more entries in LDS (and
+  // none in memory), decided for the whole wave.
+  HM_D bool room3() const { return __ballot(off >= kLevel * (kStackLds - 2)) == 0; }
+  HM_D bool in_lds() const { return __ballot(off >= kLevel * (kStackLds + 1)) == 0; }
+  // Writes v to the next entry and keeps it if `keep` (room3 holds).
+  HM_D void put(int v, bool keep) {
+    *at(off) = v;
+    off += keep ? kLevel : 0;
+  }
   HM_D void push(int v) {
-    if (sp < kStackLds) lds[sp * kTraceBlock] = v;
-    else if (sp - kStackLds < spill_levels) spill[(sp - kStackLds) * spill_stride] = v;
+    const int k = off / kLevel;
+    if (k < kStackLds) *at(off) = v;
+    else if (k - kStackLds < spill_levels) spill[(size_t)(k - kStackLds) * spill_stride] = v;
     else return;  // unreachable for a tree within the sized depth; drop rather than overrun
-    ++sp;
+    off += kLevel;
   }
   HM_D int pop() {
-    --sp;
-    return sp < kStackLds ? lds[sp * kTraceBlock] : spill[(sp - kStackLds) * spill_stride];
+    off -= kLevel;
+    const int k = off / kLevel;
+    return k < kStackLds ? *at(off) : spill[(size_t)(k - kStackLds) * spill_stride];
+  }
+  HM_D int pop_lds() {
+    off -= kLevel;
+    return *at(off);
   }
 };
 
 // Traversal: the current entry is an inner node (>= 0) or a leaf (~index <
-// 0); each iteration either visits one wide node (nearest hit child next,
-// the other hit children pushed far to near, leaves included) or tests one
-// segment. Keeping the two steps apart bounds the code a wave executes per
-// iteration to one node visit plus one segment test. The cap bounds the loop
-// for a malformed tree only: a valid tree visits each node and leaf at most
-// once per ray.
+// 0); a step either visits one wide node (nearest hit child next, the other
+// hit children pushed far to near, leaves included) or tests one primitive.
 constexpr int kNone = 0x7fffffff;
 
-// Entry distances of the child boxes against [0, tmax]; +inf for a miss or
-// an empty slot (so that sorting puts them last).
-HM_D void node_hits(const BvhNodeWide& n, const RayInv& r, float tmax, float t[kBvhWidth]) {
+// A node's children and the entry distances of their boxes against
+// [0, tmax]; t[k] is +inf where the ray misses child k.
+HM_D void node_boxes(const BvhView& bvh, const RayInv& r, int node, float tmax, float t[4], int c[4]) {
+  const char* base = (const char*)bvh.nodes;
+  const unsigned o = (unsigned)node * (unsigned)sizeof(BvhNodeWide);
+  const float4 nx = *(const float4*)(base + (o | r.nx)), fx = *(const float4*)(base + ((o | r.nx) ^ 16u));
+  const float4 ny = *(const float4*)(base + (o | r.ny)), fy = *(const float4*)(base + ((o | r.ny) ^ 16u));
+  const float4 nz = *(const float4*)(base + (o | r.nz)), fz = *(const float4*)(base + ((o | r.nz) ^ 16u));
+  const int4 ch = *(const int4*)(base + (o | 96u));
+  const float nxs[4] = {nx.x, nx.y, nx.z, nx.w}, fxs[4] = {fx.x, fx.y, fx.z, fx.w};
+  const float nys[4] = {ny.x, ny.y, ny.z, ny.w}, fys[4] = {fy.x, fy.y, fy.z, fy.w};
+  const float nzs[4] = {nz.x, nz.y, nz.z, nz.w}, fzs[4] = {fz.x, fz.y, fz.z, fz.w};
+  c[0] = ch.x; c[1] = ch.y; c[2] = ch.z; c[3] = ch.w;
 #pragma unroll
-  for (int k = 0; k < kBvhWidth; ++k) {
-    const float e = box_enter(r, n.lox[k], n.loy[k], n.loz[k], n.hix[k], n.hiy[k], n.hiz[k], tmax);
-    t[k] = (n.child[k] != kEmptyChild && e <= tmax) ? e : __builtin_inff();
+  for (int k = 0; k < 4; ++k) {
+    const float tn = fmaxf(fmaxf(fmaf(nxs[k], r.ix, -r.oix), fmaf(nys[k], r.iy, -r.oiy)),
+                           fmaxf(fmaf(nzs[k], r.iz, -r.oiz), 0.f));
+    const float tf = fminf(fminf(fmaf(fxs[k], r.ix, -r.oix), fmaf(fys[k], r.iy, -r.oiy)),
+                           fminf(fmaf(fzs[k], r.iz, -r.oiz), tmax));
+    t[k] = tn <= tf ? tn : __builtin_inff();
   }
 }
 
-HM_D void cswap(float& ta, int& ca, float& tb, int& cb) {
-  const bool s = tb < ta;
-  const float t = s ? tb : ta;
-  tb = s ? ta : tb;
-  ta = t;
-  const int c = s ? cb : ca;
-  cb = s ? ca : cb;
-  ca = c;
+// (entry distance, child) as one 64-bit value whose order as a double is
+// the order of the distances: a non-negative float's bits in the high word
+// make a non-negative finite double. One v_min_f64 / v_max_f64 (full rate on
+// CDNA) then moves distance and child together; comparing and selecting the
+// two words separately took five instructions per exchange instead of two.
+HM_D double hit_key(float t, int c) { return __hiloint2double(__float_as_int(t), c); }
+HM_D bool key_hit(double k) { return __int_as_float(__double2hiint(k)) < __builtin_inff(); }
+HM_D int key_child(double k) { return __double2loint(k); }
+HM_D void key_swap(double& a, double& b) {
+  double lo, hi;
+  asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+  asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+  a = lo;
+  b = hi;
 }
 
-// Per-lane traversal state, advanced one step (one wide node or one segment)
-// at a time so that a kernel can hand an idle lane a new ray while the rest of
-// its wave is still traversing.
+// Per-lane traversal state, advanced one step (one wide node or one
+// primitive) at a time.
 struct ClosestState {
   float best_t, best_u;
   int best_id;
   int cur;   // current entry: node (>= 0), ~leaf (< 0) or kNone when done
-  int iter;  // steps taken (cap for a malformed tree)
 };
 
+// Steps after which a query of a valid tree has certainly ended (each node and
+// leaf is visited at most once); bounds the loops for a malformed tree.
 HM_D int trace_cap(const BvhView& bvh) { return 2 * bvh.num_segs + 64; }
 
 // Starts a closest-hit query with (best_t, best_id) preset by the caller
 // (e.g. a hit on the head sphere).
 HM_D void closest_begin(const BvhView& bvh, TraceStack& st, ClosestState& s) {
-  st.sp = 0;
+  st.clear();
   s.cur = bvh.num_segs > 0 ? 0 : kNone;
-  s.iter = 0;
 }
 
 // Leaf tests: a leaf record is two float4s in Morton order whose second w
 // holds the primitive id. Hair: the record is the segment itself. Triangle
 // meshes: the record holds the triangle's box, the vertices are read by id.
+//
+// For the ray streams: a wave tests primitives when kPrims x (lanes waiting at
+// a primitive) >= kNodes x (lanes waiting at a node), and takes its rays in
+// chunks of kChunk. A segment test costs about a node step: a third of the
+// lanes at segments is worth it (shares 1/2, 1/4 and 1/8 of the node lanes:
+// 352, 357 and 375 us on a million mixed rays; 86.4, 88.8 and 93.7 ms on 16
+// passes of the headline frame). A round curve's iteration costs an order of
+// magnitude more, so two thirds of the lanes are waited for; and its rays
+// differ so much that a wave's share is dealt out in small chunks.
 struct SegLeaf {
+  static constexpr int kPrims = 2, kNodes = 1, kChunk = 32;
   HM_D bool operator()(const BvhView& bvh, const RayInv& r, int leaf, float* t, float* u, int* id) const {
     const float4 s0 = bvh.segs[2 * leaf];
     const float4 s1 = bvh.segs[2 * leaf + 1];
@@ -218,6 +260,7 @@ struct TriLeaf {
 // points (5 float4 per segment: q0..q3, then strand and end flags) are read
 // by id; caps: end caps on (the flags then say which ends have one).
 struct CurveLeaf {
+  static constexpr int kPrims = 1, kNodes = 2, kChunk = 8;
   const float4* crv;
   int caps;
   HM_D bool operator()(const BvhView& bvh, const RayInv& r, int leaf, float* t, float* u, int* id) const {
@@ -230,52 +273,51 @@ struct CurveLeaf {
 };
 
 // Closest hit over the tree's primitives: minimum (t, id) lexicographically.
-template <bool kCount, class Leaf = SegLeaf>
-HM_D void closest_step(const BvhView& bvh, const RayInv& r, TraceStack& st, ClosestState& s, TraceCounters& cnt,
-                       const Leaf& leaf_test = Leaf{}) {
-  if (s.cur < 0) {
-    const int code = ~s.cur, leaf = code & kLeafPosMask;
-    if (kCount) cnt.segs++;
-    float t, u;
-    int id;
-    if (leaf_test(bvh, r, leaf, &t, &u, &id)) {
-      if (t < s.best_t || (t == s.best_t && id < s.best_id)) {
-        s.best_t = t;
-        s.best_id = id;
-        s.best_u = u;
-      }
-    }
-    // the rest of a leaf run, one primitive per step
-    const int rest = leaf_rest(code);
-    s.cur = rest ? rest : (st.sp ? st.pop() : kNone);
+template <bool kCount>
+HM_D void closest_node(const BvhView& bvh, const RayInv& r, TraceStack& st, ClosestState& s, TraceCounters& cnt) {
+  if (kCount) cnt.nodes++;
+  float t[4];
+  int c[4];
+  node_boxes(bvh, r, s.cur, s.best_t, t, c);
+  // sorting network (Batcher): nearest first, misses (+inf) last
+  double e[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) e[k] = hit_key(t[k], c[k]);
+  key_swap(e[0], e[1]);
+  key_swap(e[2], e[3]);
+  key_swap(e[0], e[2]);
+  key_swap(e[1], e[3]);
+  key_swap(e[1], e[2]);
+  if (st.room3()) {
+#pragma unroll
+    for (int k = 3; k >= 1; --k) st.put(key_child(e[k]), key_hit(e[k]));
+    s.cur = key_child(e[0]);
+    if (!key_hit(e[0])) s.cur = st.empty() ? kNone : st.pop_lds();
   } else {
-    const BvhNodeWide n = bvh.nodes[s.cur];
-    if (kCount) cnt.nodes++;
-    float t[kBvhWidth];
-    node_hits(n, r, s.best_t, t);
-    int c[kBvhWidth];
 #pragma unroll
-    for (int k = 0; k < kBvhWidth; ++k) c[k] = n.child[k];
-    // sorting network (Batcher): nearest first, misses (+inf) last
-    if (kBvhWidth == 4) {
-      cswap(t[0], c[0], t[1], c[1]);
-      cswap(t[2], c[2], t[3], c[3]);
-      cswap(t[0], c[0], t[2], c[2]);
-      cswap(t[1], c[1], t[3], c[3]);
-      cswap(t[1], c[1], t[2], c[2]);
-    } else {
-      constexpr int net[19][2] = {{0, 1}, {2, 3}, {4, 5}, {6, 7}, {0, 2}, {1, 3}, {4, 6}, {5, 7}, {1, 2}, {5, 6},
-                                  {0, 4}, {1, 5}, {2, 6}, {3, 7}, {2, 4}, {3, 5}, {1, 2}, {3, 4}, {5, 6}};
-#pragma unroll
-      for (int q = 0; q < 19; ++q) cswap(t[net[q][0]], c[net[q][0]], t[net[q][1]], c[net[q][1]]);
-    }
-    const float inf = __builtin_inff();
-#pragma unroll
-    for (int k = kBvhWidth - 1; k >= 1; --k)
-      if (t[k] < inf) st.push(c[k]);
-    s.cur = t[0] < inf ? c[0] : (st.sp ? st.pop() : kNone);
+    for (int k = 3; k >= 1; --k)
+      if (key_hit(e[k])) st.push(key_child(e[k]));
+    s.cur = key_hit(e[0]) ? key_child(e[0]) : (st.empty() ? kNone : st.pop());
   }
-  if (++s.iter >= trace_cap(bvh)) s.cur = kNone;
+}
+
+template <bool kCount, class Leaf>
+HM_D void closest_leaf(const BvhView& bvh, const RayInv& r, TraceStack& st, ClosestState& s, TraceCounters& cnt,
+                       const Leaf& leaf_test) {
+  const int code = ~s.cur, leaf = code & kLeafPosMask;
+  if (kCount) cnt.segs++;
+  float t, u;
+  int id;
+  if (leaf_test(bvh, r, leaf, &t, &u, &id)) {
+    if (t < s.best_t || (t == s.best_t && id < s.best_id)) {
+      s.best_t = t;
+      s.best_id = id;
+      s.best_u = u;
+    }
+  }
+  // the rest of a leaf run, one primitive per step
+  s.cur = leaf_rest(code);
+  if (!s.cur) s.cur = st.empty() ? kNone : st.pop();
 }
 
 template <bool kCount, class Leaf = SegLeaf>
@@ -286,7 +328,10 @@ HM_D void trace_closest(const BvhView& bvh, const RayInv& r, TraceStack& st, flo
   s.best_id = best_id;
   s.best_u = best_u;
   closest_begin(bvh, st, s);
-  while (s.cur != kNone) closest_step<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
+  for (int left = trace_cap(bvh); s.cur != kNone && left > 0; --left) {
+    if (s.cur < 0) closest_leaf<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
+    else closest_node<kCount>(bvh, r, st, s, cnt);
+  }
   best_t = s.best_t;
   best_id = s.best_id;
   best_u = s.best_u;
@@ -296,49 +341,59 @@ HM_D void trace_closest(const BvhView& bvh, const RayInv& r, TraceStack& st, flo
 // taken in slot order.
 struct AnyState {
   int cur;
-  int iter;
   bool hit;
 };
 
 HM_D void any_begin(const BvhView& bvh, TraceStack& st, AnyState& s) {
-  st.sp = 0;
+  st.clear();
   s.cur = bvh.num_segs > 0 ? 0 : kNone;
-  s.iter = 0;
   s.hit = false;
 }
 
-template <bool kCount, class Leaf = SegLeaf>
-HM_D void any_step(const BvhView& bvh, const RayInv& r, TraceStack& st, AnyState& s, TraceCounters& cnt,
-                   const Leaf& leaf_test = Leaf{}) {
+template <bool kCount>
+HM_D void any_node(const BvhView& bvh, const RayInv& r, TraceStack& st, AnyState& s, TraceCounters& cnt) {
+  if (kCount) cnt.nodes++;
   const float tinf = __builtin_inff();
-  if (s.cur < 0) {
-    const int code = ~s.cur, leaf = code & kLeafPosMask;
-    if (kCount) cnt.segs++;
-    float t, u;
-    int id;
-    if (leaf_test(bvh, r, leaf, &t, &u, &id)) {
-      s.hit = true;
-      s.cur = kNone;
-    } else {
-      const int rest = leaf_rest(code);
-      s.cur = rest ? rest : (st.sp ? st.pop() : kNone);
-    }
-  } else {
-    const BvhNodeWide n = bvh.nodes[s.cur];
-    if (kCount) cnt.nodes++;
-    float t[kBvhWidth];
-    node_hits(n, r, tinf, t);
-    int next = kNone;
+  float t[4];
+  int c[4];
+  node_boxes(bvh, r, s.cur, tinf, t, c);
+  int next = kNone;
+  if (st.room3()) {
+    next = t[3] < tinf ? c[3] : kNone;
 #pragma unroll
-    for (int k = kBvhWidth - 1; k >= 0; --k) {
+    for (int k = 2; k >= 0; --k) {
+      const bool h = t[k] < tinf;
+      st.put(next, h && next != kNone);
+      next = h ? c[k] : next;
+    }
+    if (next == kNone && !st.empty()) next = st.pop_lds();
+  } else {
+#pragma unroll
+    for (int k = 3; k >= 0; --k) {
       if (t[k] < tinf) {
         if (next != kNone) st.push(next);
-        next = n.child[k];
+        next = c[k];
       }
     }
-    s.cur = next != kNone ? next : (st.sp ? st.pop() : kNone);
+    if (next == kNone && !st.empty()) next = st.pop();
   }
-  if (++s.iter >= trace_cap(bvh)) s.cur = kNone;
+  s.cur = next;
+}
+
+template <bool kCount, class Leaf>
+HM_D void any_leaf(const BvhView& bvh, const RayInv& r, TraceStack& st, AnyState& s, TraceCounters& cnt,
+                   const Leaf& leaf_test) {
+  const int code = ~s.cur, leaf = code & kLeafPosMask;
+  if (kCount) cnt.segs++;
+  float t, u;
+  int id;
+  if (leaf_test(bvh, r, leaf, &t, &u, &id)) {
+    s.hit = true;
+    s.cur = kNone;
+  } else {
+    s.cur = leaf_rest(code);
+    if (!s.cur) s.cur = st.empty() ? kNone : st.pop();
+  }
 }
 
 template <bool kCount, class Leaf = SegLeaf>
@@ -346,7 +401,10 @@ HM_D bool trace_any(const BvhView& bvh, const RayInv& r, TraceStack& st, TraceCo
                     const Leaf& leaf_test = Leaf{}) {
   AnyState s;
   any_begin(bvh, st, s);
-  while (s.cur != kNone) any_step<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
+  for (int left = trace_cap(bvh); s.cur != kNone && left > 0; --left) {
+    if (s.cur < 0) any_leaf<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
+    else any_node<kCount>(bvh, r, st, s, cnt);
+  }
   return s.hit;
 }
 

@@ -475,8 +475,8 @@ __global__ void k_collapse(CollapseArgs a) {
   BvhNodeWide o;
   for (int k = 0; k < kBvhWidth; ++k) {
     if (k < cnt) {
-      o.lox[k] = lo[k][0]; o.loy[k] = lo[k][1]; o.loz[k] = lo[k][2];
-      o.hix[k] = hi[k][0]; o.hiy[k] = hi[k][1]; o.hiz[k] = hi[k][2];
+      o.x[k] = lo[k][0]; o.y[k] = lo[k][1]; o.z[k] = lo[k][2];
+      o.x[4 + k] = hi[k][0]; o.y[4 + k] = hi[k][1]; o.z[4 + k] = hi[k][2];
       if (ch[k] >= 0) {
         const int j = atomicAdd(a.node_count, 1);
         a.next[atomicAdd(a.next_count, 1)] = make_int2(ch[k], j);
@@ -485,12 +485,12 @@ __global__ void k_collapse(CollapseArgs a) {
         o.child[k] = ch[k];
       }
     } else {
-      o.lox[k] = o.loy[k] = o.loz[k] = 0.f;
-      o.hix[k] = o.hiy[k] = o.hiz[k] = 0.f;
+      o.x[k] = o.y[k] = o.z[k] = kEmptyLo;
+      o.x[4 + k] = o.y[4 + k] = o.z[4 + k] = kEmptyHi;
       o.child[k] = kEmptyChild;
     }
   }
-  for (int k = 0; k < (int)(sizeof(o.pad) / sizeof(int)); ++k) o.pad[k] = 0;
+  for (int k = 0; k < 4; ++k) o.pad[k] = 0;
   a.out[f.y] = o;
 }
 

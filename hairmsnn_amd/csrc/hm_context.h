@@ -79,7 +79,8 @@ struct Context {
   float4* average = nullptr;
   int accum_id = 0;
   int seed_offset = 0;  // hmsnn_set_seed_offset
-  int trace_blocks = 2048;
+  int trace_blocks = 2048;  // largest traversal grid: stack spill is sized for it
+  int ray_blocks = 1024;    // grid of the ray streams (kRayBlocksPerCu per CU)
   int spill_levels = 0;
   unsigned long long* stats_dev = nullptr;
 

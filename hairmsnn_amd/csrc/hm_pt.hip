@@ -112,12 +112,7 @@ void launch_timed(PassTimer* tm, int kind, K kernel, dim3 grid, dim3 block, hipS
 
 __device__ __forceinline__ TraceStack make_stack(int* lds_base, const PathBuffers& pb) {
   TraceStack st;
-  st.lds = lds_base + threadIdx.x;
-  const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
-  st.spill = pb.spill + gtid;
-  st.spill_stride = pb.spill_stride;
-  st.spill_levels = pb.spill_levels;
-  st.sp = 0;
+  st.init(lds_base, pb.spill + blockIdx.x * blockDim.x + threadIdx.x, pb.spill_stride, pb.spill_levels);
   return st;
 }
 
@@ -425,18 +420,21 @@ __global__ void HM_TRACE_BOUNDS_T(kCurves) k_extend(SceneView sc, PathBuffers pb
   TraceCounters cnt{0, 0, 0};
   const int n = pb.counts[kCountStride * cur];
   const int* q = pb.queue[cur];
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+  auto load = [&](int i, float4& o, float4& d) {
     const int slot = kDense ? i : q[i];
-    const float4 o = pb.ray_o[slot], d = pb.ray_d[slot];
-    float t, u;
-    int prim;
-    if (kCount) cnt.rays++;
-    closest_hit<kCount, kCurves>(sc, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), st, t, prim, u, cnt);
+    o = pb.ray_o[slot];
+    d = pb.ray_d[slot];
+  };
+  auto store = [&](int i, float t, int prim, float u) {
+    const int slot = kDense ? i : q[i];
     pb.hit_t[slot] = t;
     pb.hit_prim[slot] = prim;
     pb.hit_u[slot] = u;
-  }
+  };
+  if constexpr (kCurves)
+    closest_stream<kCount>(sc, st, n, CurveLeaf{sc.curves, sc.curve_caps}, cnt, load, store);
+  else
+    closest_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store);
   if (kCount) flush_counters(cnt, &stats[0], &stats[1], &stats[4]);
 }
 
@@ -715,15 +713,18 @@ __global__ void HM_TRACE_BOUNDS_T(kCurves) k_shadow(SceneView sc, PathBuffers pb
   TraceStack st = make_stack(lds_stack, pb);
   TraceCounters cnt{0, 0, 0};
   const int n = pb.counts[kCountStride * 3];
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+  auto load = [&](int i, float4& o, float4& d) {
     const int e = pb.shadow_rays[i];
     const int slot = e >> 1;
-    const float4 o = (e & 1) ? pb.sh_o2[slot] : pb.sh_o1[slot];
-    const float4 d = (e & 1) ? pb.sh_d2[slot] : pb.sh_d1[slot];
-    if (kCount) cnt.rays++;
-    pb.sh_vis[e] = occluded<kCount, kCurves>(sc, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), st, cnt) ? 0 : 1;
-  }
+    o = (e & 1) ? pb.sh_o2[slot] : pb.sh_o1[slot];
+    d = (e & 1) ? pb.sh_d2[slot] : pb.sh_d1[slot];
+    return e;
+  };
+  auto store = [&](int e, bool hit) { pb.sh_vis[e] = hit ? 0 : 1; };
+  if constexpr (kCurves)
+    any_stream<kCount>(sc, st, n, CurveLeaf{sc.curves, sc.curve_caps}, cnt, load, store);
+  else
+    any_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store);
   if (kCount) flush_counters(cnt, &stats[2], &stats[3], &stats[5]);
 }
 
@@ -789,27 +790,26 @@ __global__ void HM_TRACE_BOUNDS_T(kCurves) k_trace_rays(SceneView sc, const floa
                                                             unsigned long long* stats) {
   __shared__ int lds_stack[kStackLds * kTraceBlock];
   TraceStack st;
-  st.lds = lds_stack + threadIdx.x;
-  st.spill = spill + blockIdx.x * blockDim.x + threadIdx.x;
-  st.spill_stride = spill_stride;
-  st.spill_levels = spill_levels;
-  st.sp = 0;
+  st.init(lds_stack, spill + blockIdx.x * blockDim.x + threadIdx.x, spill_stride, spill_levels);
   TraceCounters cnt{0, 0, 0};
-  const int stride = gridDim.x * blockDim.x;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
-    const float4 o = rays[2 * (size_t)i], d = rays[2 * (size_t)i + 1];
-    if (kCount) cnt.rays++;
-    if (any_hit) {
-      const bool occ = occluded<kCount, kCurves>(sc, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), st, cnt);
-      prim_out[i] = occ ? 1 : 0;
-    } else {
-      float t, u;
-      int prim;
-      closest_hit<kCount, kCurves>(sc, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), st, t, prim, u, cnt);
-      prim_out[i] = prim;
-      if (t_out) t_out[i] = t;
-      if (u_out) u_out[i] = u;
-    }
+  auto load = [&](int i, float4& o, float4& d) {
+    o = rays[2 * (size_t)i];
+    d = rays[2 * (size_t)i + 1];
+    return i;
+  };
+  auto store = [&](int i, float t, int prim, float u) {
+    prim_out[i] = prim;
+    if (t_out) t_out[i] = t;
+    if (u_out) u_out[i] = u;
+  };
+  auto store_any = [&](int i, bool hit) { prim_out[i] = hit ? 1 : 0; };
+  if constexpr (kCurves) {
+    const CurveLeaf leaf{sc.curves, sc.curve_caps};
+    if (any_hit) any_stream<kCount>(sc, st, n, leaf, cnt, load, store_any);
+    else closest_stream<kCount>(sc, st, n, leaf, cnt, load, store);
+  } else {
+    if (any_hit) any_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store_any);
+    else closest_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store);
   }
   if (kCount) flush_counters(cnt, &stats[0], &stats[1], &stats[4]);
 }

@@ -104,7 +104,7 @@ struct PassConfig {
   unsigned long long* stats = nullptr;
   PassTimer* timer = nullptr;
   int chunk = 0;  // camera_mode 1: paths per pass index (0 = all slots one pass)
-  int trace_blocks = 2048;
+  int trace_blocks = 1024;
   int shade_blocks = 2048;
   // camera_mode 0: one jittered camera ray per pixel (cuda/path_tracing.cu:32-42)
   // camera_mode 1: rays from the camera to sampled hair points, all slots

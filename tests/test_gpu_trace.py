@@ -178,3 +178,22 @@ def test_full_c1_bit_exact(gpu, builder):
     np.testing.assert_array_equal(u[hit], u_c[hit])
     occ_c = ol.intersect(seg, rays, any_hit=True, use_bvh=True)
     np.testing.assert_array_equal(occ, occ_c)
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 64, 65, 1000, 40_001])
+def test_ray_stream_lengths_bit_exact(gpu, n):
+    """Lists shorter than a wave, than a chunk of a wave's rays and longer than
+    one refill, rays that miss everything and rays that start inside the hair
+    among them: every ray's result is its own, whatever shares its wave."""
+    with c0_scene(gpu, width=128, height=128) as sc:
+        seg = sc.segments()
+        rays = make_rays(seg, 3 * n, 23)[::3].copy()
+        rays[::7, 4:7] *= -1.0  # some away from the hair
+        prim, t, u = sc.trace_rays(rays)
+        any_hit = sc.trace_rays(rays, any_hit=True)
+    prim_c, t_c, u_c = ol.intersect(seg, rays, use_bvh=True)
+    hit = prim_c >= 0
+    np.testing.assert_array_equal(prim, prim_c)
+    np.testing.assert_array_equal(t[hit], t_c[hit])
+    np.testing.assert_array_equal(u[hit], u_c[hit])
+    np.testing.assert_array_equal(any_hit, hit.astype(np.int32))
