@@ -12,7 +12,7 @@ Roofline: every pass kernel is timed alone with HIP events on its stream
 (extend: closest-hit traversal; shade: hit setup, light and BSDF samples,
 compaction; shadow: any-hit traversal), and the line's `roofline` is the
 one with the most time per pass. Algorithmic bytes: traversal = 4-wide nodes
-visited x 128 B + segments tested x 32 B + ray in / hit out (48 B closest,
+visited x 64 B + segments tested x 32 B + ray in / hit out (48 B closest,
 36 B any-hit), counted by the same traversal compiled with counters; shade =
 per vertex 56 B of path state read, per continuing vertex 60 B more read
 (hit, RNG, throughput, segment) and 92 B moved into the next wavefront, per
@@ -39,7 +39,7 @@ sys.path.insert(0, str(ROOT))
 METRIC = "paths/s @1024² 3.2M segs; HairMSNN β=1 vs plain PT time-to-equal-RMSE"
 HBM_PEAK_GBS = 8000.0
 SCENE = ROOT / "hairmsnn_amd" / "scenes" / "c1_curly.json"
-NODE_BYTES, SEG_BYTES, RAY_BYTES = 128, 32, 48  # 4-wide node, segment record, ray in + hit out
+NODE_BYTES, SEG_BYTES, RAY_BYTES = 64, 32, 48  # 4-wide node, segment record, ray in + hit out
 ANY_RAY_BYTES = 36  # shadow ray in (32 B) + visibility out
 # shade: path state read per vertex, more per continuing vertex, moved per
 # continuing vertex, per finished path, per shadow ray

@@ -437,6 +437,42 @@ static int ploc_build(BuildBuffers& b, DeviceArena& arena, int R, hipStream_t st
   return check_launch("ploc root", err);
 }
 
+// One axis of a wide node: corner and step, and per child the lower and upper
+// plane in steps (bytes), rounded outward in FP64 so that o + q * s holds the
+// box widened by 2^-21 of its coordinates (the rounding of node_boxes's step
+// term). Unused slots get the inverted box (255, 0).
+__device__ inline void quantise_axis(const float lo[][3], const float hi[][3], int axis, int cnt, float* o_out,
+                                     float* s_out, unsigned* lo_out, unsigned* hi_out) {
+  double l = 1e300, h = -1e300, m = 0.0;
+  for (int k = 0; k < cnt; ++k) {
+    l = fmin(l, (double)lo[k][axis]);
+    h = fmax(h, (double)hi[k][axis]);
+    m = fmax(m, fmax(fabs((double)lo[k][axis]), fabs((double)hi[k][axis])));
+  }
+  const double margin = m * 4.76837158203125e-7 + 1e-37;
+  // corner below every widened box; step so that 255 of them pass the highest
+  const float o = nextafterf((float)(l - margin), -3e38f);
+  float s = (float)fmax((h + margin - (double)o) / 255.0, 1e-37);
+  while ((double)o + 255.0 * (double)s < h + margin) s = nextafterf(s, 3e38f);
+  unsigned ql = 0, qh = 0;
+  for (int k = 0; k < kBvhWidth; ++k) {
+    int a = 255, b = 0;
+    if (k < cnt) {
+      const double dl = (double)lo[k][axis] - margin, dh = (double)hi[k][axis] + margin;
+      a = (int)fmin(255.0, fmax(0.0, floor((dl - (double)o) / (double)s)));
+      while (a > 0 && (double)o + a * (double)s > dl) --a;
+      b = (int)fmin(255.0, fmax(0.0, ceil((dh - (double)o) / (double)s)));
+      while (b < 255 && (double)o + b * (double)s < dh) ++b;
+    }
+    ql |= (unsigned)a << (8 * k);
+    qh |= (unsigned)b << (8 * k);
+  }
+  *o_out = o;
+  *s_out = s;
+  *lo_out = ql;
+  *hi_out = qh;
+}
+
 // One wide node per frontier entry: start from the binary node's two
 // children and open the inner child of largest surface area until there are
 // kBvhWidth (or only leaves remain).
@@ -475,8 +511,6 @@ __global__ void k_collapse(CollapseArgs a) {
   BvhNodeWide o;
   for (int k = 0; k < kBvhWidth; ++k) {
     if (k < cnt) {
-      o.x[k] = lo[k][0]; o.y[k] = lo[k][1]; o.z[k] = lo[k][2];
-      o.x[4 + k] = hi[k][0]; o.y[4 + k] = hi[k][1]; o.z[4 + k] = hi[k][2];
       if (ch[k] >= 0) {
         const int j = atomicAdd(a.node_count, 1);
         a.next[atomicAdd(a.next_count, 1)] = make_int2(ch[k], j);
@@ -485,12 +519,12 @@ __global__ void k_collapse(CollapseArgs a) {
         o.child[k] = ch[k];
       }
     } else {
-      o.x[k] = o.y[k] = o.z[k] = kEmptyLo;
-      o.x[4 + k] = o.y[4 + k] = o.z[4 + k] = kEmptyHi;
       o.child[k] = kEmptyChild;
     }
   }
-  for (int k = 0; k < 4; ++k) o.pad[k] = 0;
+  quantise_axis(lo, hi, 0, cnt, &o.ox, &o.sx, &o.lox, &o.hix);
+  quantise_axis(lo, hi, 1, cnt, &o.oy, &o.sy, &o.loy, &o.hiy);
+  quantise_axis(lo, hi, 2, cnt, &o.oz, &o.sz, &o.loz, &o.hiz);
   a.out[f.y] = o;
 }
 
