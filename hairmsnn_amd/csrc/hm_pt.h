@@ -54,14 +54,19 @@ struct SceneView {
   int mis;
 };
 
-constexpr int kDoneCount = 4;  // PathBuffers::counts index of the finished-path queue
-// PathBuffers::counts holds each queue length in a 256-byte line of its own:
-// counts[kCountStride * k] is the length of queue k (0 and 1 the two
-// wavefronts, 2 the shadow records, 3 the shadow rays, kDoneCount the
-// finished paths), so the appends to different queues do not contend for
-// one line.
+// PathBuffers::counts holds each queue length in a 256-byte line of its own,
+// so the appends to different queues do not contend for one line: the lengths
+// of the two wavefronts, then two sets of the lengths a shading step appends
+// to. Steps alternate between the sets, so one is cleared while the other is
+// still being read.
 constexpr int kCountStride = 64;
-constexpr int kCountInts = kCountStride * (kDoneCount + 1);
+constexpr int kShadowCount = 0;  // vertices with pending direct light
+constexpr int kRayCount = 1;     // shadow rays
+constexpr int kDoneCount = 2;    // finished paths (compacted wavefronts)
+constexpr int kNextCount = 3;    // continuing paths (compacted wavefronts)
+HM_HD constexpr int wave_count(int wave) { return kCountStride * wave; }
+HM_HD constexpr int append_count(int set, int which) { return kCountStride * (2 + 4 * set + which); }
+constexpr int kCountInts = kCountStride * 10;
 
 // Per-slot path state (structure of arrays in HBM). A slot is one pixel of
 // the current sample pass.
@@ -81,8 +86,8 @@ struct PathState {
 };
 
 // Scheduler words of the job schedule (pt_jobs_*): two copies of [0] next
-// job, [2] free path capacity, each copy in its own 64-byte line, then at
-// kJobCtlLive the number of iterations that found live paths.
+// job, each in its own 64-byte line, then at kJobCtlLive the number of
+// iterations that found live paths.
 constexpr int kJobCtlHalf = 8;
 constexpr int kJobCtlLive = 2 * kJobCtlHalf;
 constexpr int kJobCtl = kJobCtlLive + kJobCtlHalf;
@@ -127,7 +132,7 @@ struct PathBuffers {
   int* done_px;
   int* done_pass;
   long long* job_ctl;  // kJobCtl words
-  int* counts;  // [0], [1] continuation queues, [2] shadow slots, [3] shadow rays, [4] finished paths
+  int* counts;  // queue lengths (wave_count, append_count)
   int* spill;   // traversal stack spill
   int spill_stride;
   int spill_levels;
@@ -140,7 +145,8 @@ struct ShadeParams {
   int max_vertex;  // continuation allowed while depth + 1 <= max_vertex
   int trunc_beta;  // HairMSNN: terminate after the vertex when depth > trunc_beta
   int msnn;        // 1: HairMSNN G-buffer pass (training paths enabled)
-  int cur;         // current continuation queue index
+  int cur;         // current wavefront
+  int set;         // append_count set of this step
 };
 
 #if defined(__HIPCC__)
@@ -498,7 +504,7 @@ HM_D Continuation shade_vertex(const SceneView& sc, const Hit& h, uint32_t& rng,
 }
 
 // Writes a vertex's shadow records at index i of the pending-light arrays,
-// in the layout k_shadow and the resolve kernels read: (origin, 1 if the ray
+// in the layout k_trace and the resolve kernels read: (origin, 1 if the ray
 // exists), direction, contribution per ray, and the throughput.
 struct ShadowSink {
   float4 *o1, *d1, *c1, *o2, *d2, *c2, *beta;
@@ -588,6 +594,11 @@ HM_D bool occluded(const SceneView& sc, V3 o, V3 d, TraceStack& st, TraceCounter
 // enough lanes are ready for (the Leaf's kNodes); the others wait. A ray's own
 // steps and their order are those of trace_closest / trace_any, so its result
 // does not depend on the schedule.
+//
+// A launch takes the next wavefront's closest-hit rays and the light rays of
+// the vertices just shaded together: they do not depend on each other, and
+// a launch ends with its longest rays' chains of dependent node reads, 100 to
+// 150 us at any ray count, which the two then share.
 
 // The rays a wave takes from a list of n: chunks w, w + W, w + 2 W, ... of
 // kChunk consecutive rays (neighbours share nodes; interleaving spreads dense
@@ -596,7 +607,7 @@ template <int kChunk>
 struct RayQueue {
   long long n, stride, base;
   int pos;
-  HM_D RayQueue(int n_rays) : n(n_rays), pos(0) {
+  HM_D RayQueue(long long n_rays) : n(n_rays), pos(0) {
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6)));
     stride = (long long)gridDim.x * (kTraceBlock / 64) * kChunk;
     base = (long long)wave * kChunk;
@@ -628,12 +639,15 @@ HM_D bool leaf_turn(unsigned long long at_leaf, unsigned long long at_node) {
   return __popcll(at_leaf) * Leaf::kPrims >= __popcll(at_node) * Leaf::kNodes;
 }
 
-// Closest hits of n rays: load(i, o, d) gives ray i, store(i, t, prim, u)
-// takes its result (the sphere and the head mesh included, as closest_hit).
-template <bool kCount, class Leaf, class Load, class Store>
-HM_D void closest_stream(const SceneView& sc, TraceStack& st, int n, const Leaf& leaf, TraceCounters& cnt, Load load,
-                         Store store) {
-  RayQueue<Leaf::kChunk> rays(n);
+// Hits of n_closest + n_any rays: load(i, o, d) gives ray i; the first
+// n_closest are closest-hit queries (store_hit(i, t, prim, u), the sphere and
+// the head mesh included, as closest_hit), the others any-hit ones
+// (store_any(i, hit)). An any-hit query runs the same steps and ends at its
+// first hit. cnt: counters of the closest and of the any-hit rays.
+template <bool kCount, class Leaf, class Load, class StoreHit, class StoreAny>
+HM_D void trace_stream(const SceneView& sc, TraceStack& st, int n_closest, int n_any, const Leaf& leaf,
+                       TraceCounters cnt[2], Load load, StoreHit store_hit, StoreAny store_any) {
+  RayQueue<Leaf::kChunk> rays((long long)n_closest + n_any);
   ClosestState s;
   s.cur = kNone;
   s.best_t = s.best_u = 0.f;
@@ -646,12 +660,14 @@ HM_D void closest_stream(const SceneView& sc, TraceStack& st, int n, const Leaf&
     if (idle == ~0ull || (__popcll(idle) >= kRefillMin && !rays.empty())) {
       const int next = rays.take(idle);
       if (s.cur == kNone) {
-        if (idx >= 0) store(idx, s.best_t, s.best_id != kNone ? s.best_id : other, s.best_u);
+        if (idx >= n_closest) store_any(idx, s.best_id != kNone || other != kPrimMiss);
+        else if (idx >= 0) store_hit(idx, s.best_t, s.best_id != kNone ? s.best_id : other, s.best_u);
         idx = next;
         if (idx >= 0) {
+          const bool any = idx >= n_closest;
           float4 o, d;
           load(idx, o, d);
-          if (kCount) cnt.rays++;
+          if (kCount) cnt[any].rays++;
           s.best_t = __builtin_inff();
           s.best_u = 0.f;
           s.best_id = kNone;
@@ -665,71 +681,30 @@ HM_D void closest_stream(const SceneView& sc, TraceStack& st, int n, const Leaf&
             }
           }
           r = make_ray(o.x, o.y, o.z, d.x, d.y, d.z);
-          if (sc.mesh.num > 0) {
+          if (sc.mesh.num > 0 && !(any && other != kPrimMiss)) {
             float bu = 0.f;
             int tri = kNone;
-            trace_closest<kCount, TriLeaf>(sc.mesh.bvh, r, st, s.best_t, tri, bu, cnt, TriLeaf{sc.mesh.tri});
+            trace_closest<kCount, TriLeaf>(sc.mesh.bvh, r, st, s.best_t, tri, bu, cnt[any], TriLeaf{sc.mesh.tri});
             if (tri != kNone) other = kPrimMesh0 - tri;
           }
           closest_begin(sc.bvh, st, s);
+          if (any && other != kPrimMiss) s.cur = kNone;
         }
       }
       if (__ballot(idx >= 0) == 0) return;
     }
     const unsigned long long at_leaf = __ballot(s.cur < 0), at_node = __ballot(s.cur >= 0 && s.cur != kNone);
     if (leaf_turn<Leaf>(at_leaf, at_node)) {
-      if (s.cur < 0) closest_leaf<kCount, Leaf>(sc.bvh, r, st, s, cnt, leaf);
-    } else {
-      if (s.cur >= 0 && s.cur != kNone) closest_node<kCount>(sc.bvh, r, st, s, cnt);
-    }
-  }
-}
-
-// Any hits of n rays: load(i, o, d) gives ray i and returns the index that
-// store(index, hit) gets.
-template <bool kCount, class Leaf, class Load, class Store>
-HM_D void any_stream(const SceneView& sc, TraceStack& st, int n, const Leaf& leaf, TraceCounters& cnt, Load load,
-                     Store store) {
-  RayQueue<Leaf::kChunk> rays(n);
-  AnyState s;
-  s.cur = kNone;
-  s.hit = false;
-  RayInv r = make_ray(0.f, 0.f, 0.f, 1.f, 0.f, 0.f);
-  int idx = -1;
-  for (long long left = rays.most() * (trace_cap(sc.bvh) + 1); left > 0; --left) {
-    const unsigned long long idle = __ballot(s.cur == kNone);
-    if (idle == ~0ull || (__popcll(idle) >= kRefillMin && !rays.empty())) {
-      const int next = rays.take(idle);
-      if (s.cur == kNone) {
-        if (idx >= 0) store(idx, s.hit);
-        idx = next;
-        if (idx >= 0) {
-          float4 o, d;
-          idx = load(idx, o, d);
-          if (kCount) cnt.rays++;
-          bool blocked = false;
-          if (sc.sphere.enabled) {
-            float ts;
-            blocked = intersect_sphere(v3(o.x, o.y, o.z), v3(d.x, d.y, d.z),
-                                       v3(sc.sphere.cx, sc.sphere.cy, sc.sphere.cz), sc.sphere.r, &ts);
-          }
-          r = make_ray(o.x, o.y, o.z, d.x, d.y, d.z);
-          if (!blocked && sc.mesh.num > 0)
-            blocked = trace_any<kCount, TriLeaf>(sc.mesh.bvh, r, st, cnt, TriLeaf{sc.mesh.tri});
-          any_begin(sc.bvh, st, s);
-          if (blocked) {
-            s.hit = true;
-            s.cur = kNone;
-          }
-        }
+      if (s.cur < 0) {
+        if (kCount) cnt[idx >= n_closest].segs++;
+        closest_leaf<false, Leaf>(sc.bvh, r, st, s, cnt[0], leaf);
+        if (idx >= n_closest && s.best_id != kNone) s.cur = kNone;
       }
-      if (__ballot(idx >= 0) == 0) return;
-    }
-    const unsigned long long at_leaf = __ballot(s.cur < 0), at_node = __ballot(s.cur >= 0 && s.cur != kNone);
-    if (leaf_turn<Leaf>(at_leaf, at_node)) {
-      if (s.cur < 0) any_leaf<kCount, Leaf>(sc.bvh, r, st, s, cnt, leaf);
     } else {
-      if (s.cur >= 0 && s.cur != kNone) any_node<kCount>(sc.bvh, r, st, s, cnt);
+      if (s.cur >= 0 && s.cur != kNone) {
+        if (kCount) cnt[idx >= n_closest].nodes++;
+        closest_node<false>(sc.bvh, r, st, s, cnt[0]);
+      }
     }
   }
 }

@@ -2,11 +2,13 @@
 //
 // One sample pass over the image runs:
 //   camera   : seed each pixel's stream, jitter, primary ray   (path_tracing.cu:19-50)
+//   trace    : the camera rays' closest hits (BVH traversal)
 //   per vertex depth = 0 .. max_vertex:
-//     extend : closest hit for every live path (BVH traversal)
 //     shade  : hit setup, direct-lighting samples, Russian roulette and the
 //              continuation sample; survivors are compacted into the next queue
-//     shadow : any-hit tests for the pending light samples, then accumulate
+//     trace  : the survivors' closest hits and the any-hit tests of the
+//              pending light samples, in one launch
+//     resolve: the visible light samples' contributions
 //   accumulate: running sum and mean per pixel                   (utils.cuh:13-35)
 // Queues are compacted with ballots and popcounts and one atomic per block and
 // queue (shading) or per wave (the rest), each queue length in a cache line of
@@ -23,31 +25,6 @@
 namespace hm {
 
 namespace {
-
-// Appends to a queue from a 256-thread block: each lane with pred set gets a
-// position. The four waves' counts meet in LDS and one thread makes the
-// block's single atomic (one atomic per wave, every wave of a launch on the
-// same counter, serialised there). Every thread of the block calls it the
-// same number of times.
-__device__ __forceinline__ int block_append1(int* counter, bool pred) {
-  __shared__ int tot[4], base[4];
-  const unsigned long long mask = __ballot(pred);
-  const int w = threadIdx.x >> 6, lane = __lane_id();
-  if (lane == 0) tot[w] = __popcll(mask);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int sum = tot[0] + tot[1] + tot[2] + tot[3];
-    int b = sum > 0 ? atomicAdd(counter, sum) : 0;
-    for (int k = 0; k < 4; ++k) {
-      base[k] = b;
-      b += tot[k];
-    }
-  }
-  __syncthreads();
-  const int q = pred ? base[w] + __popcll(mask & ((1ull << lane) - 1ull)) : -1;
-  __syncthreads();  // base[] is read before the next call overwrites it
-  return q;
-}
 
 // Queue positions of one vertex after a shading step.
 struct Appended {
@@ -110,12 +87,6 @@ void launch_timed(PassTimer* tm, int kind, K kernel, dim3 grid, dim3 block, hipS
   hipExtLaunchKernelGGL(kernel, grid, block, 0, st, t0, t1, 0, args...);
 }
 
-__device__ __forceinline__ TraceStack make_stack(int* lds_base, const PathBuffers& pb) {
-  TraceStack st;
-  st.init(lds_base, pb.spill + blockIdx.x * blockDim.x + threadIdx.x, pb.spill_stride, pb.spill_levels);
-  return st;
-}
-
 // Wave-reduces the traversal counters and adds them to nodes/segs/rays.
 __device__ __forceinline__ void flush_counters(const TraceCounters& c, unsigned long long* nodes,
                                                unsigned long long* segs, unsigned long long* rays) {
@@ -152,15 +123,6 @@ __device__ __forceinline__ void camera_path(const SceneView& sc, const PathBuffe
   pb.rng[i] = rng;
 }
 
-__global__ void k_reset_counts(int* counts, int a, int b, int c) {
-  if (threadIdx.x == 0) {
-    counts[kCountStride * a] = 0;
-    counts[kCountStride * b] = 0;
-    counts[kCountStride * c] = 0;
-    counts[kCountStride * kDoneCount] = 0;
-  }
-}
-
 // Primary rays for every pixel of pass `accum_id` (path_tracing.cu:29-48).
 // HairMSNN training pixels (hair_msnn.cu:206-209) are flagged here.
 // NRC (nrc != 0): training pixels by the same rule (cuda/nrc.cu:371-377),
@@ -169,7 +131,7 @@ __global__ void k_camera(SceneView sc, PathBuffers pb, int accum_id, int msnn, c
                          int every_nth, int n_train, int nrc, int all_unbiased) {
   const int n = sc.width * sc.height;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) pb.counts[kCountStride * 0] = n;
+  if (i == 0) pb.counts[wave_count(0)] = n;
   if (i >= n) return;
   camera_path(sc, pb, i, i, accum_id);
   pb.queue[0][i] = i;
@@ -243,7 +205,7 @@ __device__ __forceinline__ void camera_train_point(const SceneView& sc, const Pa
 __global__ void k_camera_pixels(SceneView sc, PathBuffers pb, int accum_id, int n, int chunk, int every_nth,
                                 const int* train_idx, int* pix) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) pb.counts[kCountStride * 0] = n;
+  if (i == 0) pb.counts[wave_count(0)] = n;
   if (i >= n) return;
   camera_train_pixel(sc, pb, i, i, accum_id, chunk, every_nth, train_idx, pix);
   pb.queue[0][i] = i;
@@ -254,7 +216,7 @@ __global__ void k_camera_pixels(SceneView sc, PathBuffers pb, int accum_id, int 
 __global__ void k_camera_points(SceneView sc, PathBuffers pb, int accum_id, int n, int chunk, int grid_w,
                                 const float* pts) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) pb.counts[kCountStride * 0] = n;
+  if (i == 0) pb.counts[wave_count(0)] = n;
   if (i >= n) return;
   camera_train_point(sc, pb, i, i, accum_id, chunk, grid_w, pts);
   pb.queue[0][i] = i;
@@ -269,11 +231,11 @@ __global__ void k_camera_points(SceneView sc, PathBuffers pb, int accum_id, int 
 // record, direct light, continuation). No Russian roulette. The radiance of
 // a training pixel is frozen in L_short when its primary path queries the
 // cache and its suffix goes on.
-__global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb, int depth, int cur,
+__global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb, ShadeParams sp,
                                                    NrcPassArgs nr) {
-  const int nxt = cur ^ 1;
-  const int n = pb.counts[kCountStride * cur];
-  const int* q = pb.queue[cur];
+  const int depth = sp.depth, nxt = sp.cur ^ 1;
+  const int n = pb.counts[wave_count(sp.cur)];
+  const int* q = pb.queue[sp.cur];
   const int stride = gridDim.x * blockDim.x;
   const int nloop = (n + stride - 1) / stride * stride;
   const float kPiRef = 3.1415926f;  // Pi (utils.cuh:10)
@@ -402,8 +364,8 @@ __global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb,
       }
       pb.flags[slot] = fl;
     }
-    const Appended a = block_append(&pb.counts[kCountStride * nxt], nullptr, &pb.counts[kCountStride * 2],
-                                    &pb.counts[kCountStride * 3], cont, false, shadow, ray1, ray2);
+    const Appended a = block_append(&pb.counts[wave_count(nxt)], nullptr, &pb.counts[append_count(sp.set, kShadowCount)],
+                                    &pb.counts[append_count(sp.set, kRayCount)], cont, false, shadow, ray1, ray2);
     if (cont) pb.queue[nxt][a.next] = slot;
     if (shadow) pb.shadow_queue[a.shadow] = slot;
     if (ray1) pb.shadow_rays[a.ray1] = 2 * slot;
@@ -411,31 +373,56 @@ __global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb,
   }
 }
 
-// kDense: the wavefront is compacted (path i is at index i), no queue.
-template <bool kCount, bool kDense = false, bool kCurves = false>
-__global__ void HM_TRACE_BOUNDS_T(kCurves) k_extend(SceneView sc, PathBuffers pb, int cur,
-                                                        unsigned long long* stats) {
+// What a trace launch does: the closest hits of wavefront `wave` (what & 1)
+// and the shadow rays of append set `set` (what & 2). clear: empty the other
+// wavefront's and the other set's lengths, for the next shading step (their
+// readers have ended before this launch).
+struct TraceArgs {
+  int wave, set, what, clear;
+};
+
+// nb: the wavefront whose closest hits are traced, pb: the one whose light
+// samples are pending (the same buffers unless wavefronts are compacted).
+// kDense: compacted wavefronts (path i is at index i), no queue.
+template <bool kCount, bool kDense, bool kCurves>
+__global__ void HM_TRACE_BOUNDS_T(kCurves) k_trace(SceneView sc, PathBuffers pb, PathBuffers nb, TraceArgs a,
+                                                   unsigned long long* stats) {
   __shared__ int lds_stack[kStackLds * kTraceBlock];
-  TraceStack st = make_stack(lds_stack, pb);
-  TraceCounters cnt{0, 0, 0};
-  const int n = pb.counts[kCountStride * cur];
-  const int* q = pb.queue[cur];
+  TraceStack st;
+  st.init(lds_stack, pb.spill + blockIdx.x * blockDim.x + threadIdx.x, pb.spill_stride, pb.spill_levels);
+  TraceCounters cnt[2] = {{0, 0, 0}, {0, 0, 0}};
+  const int n_closest = (a.what & 1) ? pb.counts[wave_count(a.wave)] : 0;
+  const int n_any = (a.what & 2) ? pb.counts[append_count(a.set, kRayCount)] : 0;
+  if (a.clear && blockIdx.x == 0 && threadIdx.x < 5)
+    pb.counts[threadIdx.x < 4 ? append_count(a.set ^ 1, threadIdx.x) : wave_count(a.wave ^ 1)] = 0;
+  const int* q = pb.queue[a.wave];
   auto load = [&](int i, float4& o, float4& d) {
-    const int slot = kDense ? i : q[i];
-    o = pb.ray_o[slot];
-    d = pb.ray_d[slot];
+    if (i < n_closest) {
+      const int slot = kDense ? i : q[i];
+      o = nb.ray_o[slot];
+      d = nb.ray_d[slot];
+    } else {
+      const int e = pb.shadow_rays[i - n_closest], slot = e >> 1;
+      o = (e & 1) ? pb.sh_o2[slot] : pb.sh_o1[slot];
+      d = (e & 1) ? pb.sh_d2[slot] : pb.sh_d1[slot];
+    }
   };
-  auto store = [&](int i, float t, int prim, float u) {
+  auto store_hit = [&](int i, float t, int prim, float u) {
     const int slot = kDense ? i : q[i];
     pb.hit_t[slot] = t;
     pb.hit_prim[slot] = prim;
     pb.hit_u[slot] = u;
   };
+  auto store_any = [&](int i, bool hit) { pb.sh_vis[pb.shadow_rays[i - n_closest]] = hit ? 0 : 1; };
   if constexpr (kCurves)
-    closest_stream<kCount>(sc, st, n, CurveLeaf{sc.curves, sc.curve_caps}, cnt, load, store);
+    trace_stream<kCount>(sc, st, n_closest, n_any, CurveLeaf{sc.curves, sc.curve_caps}, cnt, load, store_hit,
+                         store_any);
   else
-    closest_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store);
-  if (kCount) flush_counters(cnt, &stats[0], &stats[1], &stats[4]);
+    trace_stream<kCount>(sc, st, n_closest, n_any, SegLeaf{}, cnt, load, store_hit, store_any);
+  if (kCount) {
+    flush_counters(cnt[0], &stats[0], &stats[1], &stats[4]);
+    flush_counters(cnt[1], &stats[2], &stats[3], &stats[5]);
+  }
 }
 
 #ifndef HM_SHADE_MIN_WAVES
@@ -444,7 +431,7 @@ __global__ void HM_TRACE_BOUNDS_T(kCurves) k_extend(SceneView sc, PathBuffers pb
 __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade(SceneView sc, PathBuffers pb, ShadeParams sp,
                                                                    GBufferOut gb) {
   const int nxt = sp.cur ^ 1;
-  const int n = pb.counts[kCountStride * (sp.cur)];
+  const int n = pb.counts[wave_count(sp.cur)];
   const int* q = pb.queue[sp.cur];
   const int stride = gridDim.x * blockDim.x;
   const int nloop = (n + stride - 1) / stride * stride;
@@ -517,11 +504,11 @@ __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade(SceneView sc,
         pb.rng[slot] = rng;
       }
     }
-    const Appended a = block_append(&pb.counts[kCountStride * nxt], nullptr, &pb.counts[kCountStride * 2],
-                                    &pb.counts[kCountStride * 3], cont, false, shadow, ray1, ray2);
+    const Appended a = block_append(&pb.counts[wave_count(nxt)], nullptr, &pb.counts[append_count(sp.set, kShadowCount)],
+                                    &pb.counts[append_count(sp.set, kRayCount)], cont, false, shadow, ray1, ray2);
     if (cont) pb.queue[nxt][a.next] = slot;
     if (shadow) pb.shadow_queue[a.shadow] = slot;
-    // one entry per shadow ray (slot * 2 + which), so k_shadow traces one ray per lane
+    // one entry per shadow ray (slot * 2 + which), which: 0 light sample, 1 BSDF sample
     if (ray1) pb.shadow_rays[a.ray1] = 2 * slot;
     if (ray2) pb.shadow_rays[a.ray2] = 2 * slot + 1;
   }
@@ -538,8 +525,7 @@ __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade(SceneView sc,
 template <bool kMsnn>
 __device__ __forceinline__ void shade_dense(const SceneView& sc, const PathBuffers& pb, const PathBuffers& nb,
                                             const ShadeParams& sp, const GBufferOut& gb) {
-  const int nxt = sp.cur ^ 1;
-  const int n = pb.counts[kCountStride * (sp.cur)];
+  const int n = pb.counts[wave_count(sp.cur)];
   const int stride = gridDim.x * blockDim.x;
   const int nloop = (n + stride - 1) / stride * stride;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nloop; i += stride) {
@@ -619,9 +605,10 @@ __device__ __forceinline__ void shade_dense(const SceneView& sc, const PathBuffe
       }
     }
     const bool done = live && !cont;
-    const Appended a = block_append(&pb.counts[kCountStride * nxt], &pb.counts[kCountStride * kDoneCount],
-                                    &pb.counts[kCountStride * 2], &pb.counts[kCountStride * 3], cont, done, shadow,
-                                    ray1, ray2);
+    const Appended a = block_append(
+        &pb.counts[append_count(sp.set, kNextCount)], &pb.counts[append_count(sp.set, kDoneCount)],
+        &pb.counts[append_count(sp.set, kShadowCount)], &pb.counts[append_count(sp.set, kRayCount)], cont, done, shadow,
+        ray1, ray2);
     const int p = a.next, dp = a.done;
     if (cont) {
       nb.ray_o[p] = no4;
@@ -666,8 +653,8 @@ __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade_dense_msnn(Sc
 // contributions go to the path where k_shade_dense moved it (kMsnn: the
 // short radiance too).
 template <bool kMsnn>
-__device__ __forceinline__ void shadow_resolve_dense(const PathBuffers& pb, const PathBuffers& nb) {
-  const int n = pb.counts[kCountStride * 2];
+__device__ __forceinline__ void shadow_resolve_dense(const PathBuffers& pb, const PathBuffers& nb, int set) {
+  const int n = pb.counts[append_count(set, kShadowCount)];
   const int stride = gridDim.x * blockDim.x;
   for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
     const int slot = pb.shadow_queue[j];
@@ -701,37 +688,18 @@ __device__ __forceinline__ void shadow_resolve_dense(const PathBuffers& pb, cons
   }
 }
 
-__global__ void k_shadow_resolve_dense(PathBuffers pb, PathBuffers nb) { shadow_resolve_dense<false>(pb, nb); }
+__global__ void k_shadow_resolve_dense(PathBuffers pb, PathBuffers nb, int set) {
+  shadow_resolve_dense<false>(pb, nb, set);
+}
 
-__global__ void k_shadow_resolve_dense_msnn(PathBuffers pb, PathBuffers nb) { shadow_resolve_dense<true>(pb, nb); }
-
-// Any-hit test of each pending shadow ray, one ray per lane; writes the
-// visibility byte of (slot, which).
-template <bool kCount, bool kCurves = false>
-__global__ void HM_TRACE_BOUNDS_T(kCurves) k_shadow(SceneView sc, PathBuffers pb, unsigned long long* stats) {
-  __shared__ int lds_stack[kStackLds * kTraceBlock];
-  TraceStack st = make_stack(lds_stack, pb);
-  TraceCounters cnt{0, 0, 0};
-  const int n = pb.counts[kCountStride * 3];
-  auto load = [&](int i, float4& o, float4& d) {
-    const int e = pb.shadow_rays[i];
-    const int slot = e >> 1;
-    o = (e & 1) ? pb.sh_o2[slot] : pb.sh_o1[slot];
-    d = (e & 1) ? pb.sh_d2[slot] : pb.sh_d1[slot];
-    return e;
-  };
-  auto store = [&](int e, bool hit) { pb.sh_vis[e] = hit ? 0 : 1; };
-  if constexpr (kCurves)
-    any_stream<kCount>(sc, st, n, CurveLeaf{sc.curves, sc.curve_caps}, cnt, load, store);
-  else
-    any_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store);
-  if (kCount) flush_counters(cnt, &stats[2], &stats[3], &stats[5]);
+__global__ void k_shadow_resolve_dense_msnn(PathBuffers pb, PathBuffers nb, int set) {
+  shadow_resolve_dense<true>(pb, nb, set);
 }
 
 // NRC training pixels also record the vertex's direct light (vertRadiance,
 // cuda/nrc.cu:200).
-__global__ void k_shadow_resolve(PathBuffers pb, int msnn, int depth, NrcPassArgs nr) {
-  const int n = pb.counts[kCountStride * 2];
+__global__ void k_shadow_resolve(PathBuffers pb, int msnn, int depth, int set, NrcPassArgs nr) {
+  const int n = pb.counts[append_count(set, kShadowCount)];
   const int stride = gridDim.x * blockDim.x;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     const int slot = pb.shadow_queue[i];
@@ -791,31 +759,55 @@ __global__ void HM_TRACE_BOUNDS_T(kCurves) k_trace_rays(SceneView sc, const floa
   __shared__ int lds_stack[kStackLds * kTraceBlock];
   TraceStack st;
   st.init(lds_stack, spill + blockIdx.x * blockDim.x + threadIdx.x, spill_stride, spill_levels);
-  TraceCounters cnt{0, 0, 0};
+  TraceCounters cnt[2] = {{0, 0, 0}, {0, 0, 0}};
   auto load = [&](int i, float4& o, float4& d) {
     o = rays[2 * (size_t)i];
     d = rays[2 * (size_t)i + 1];
-    return i;
   };
-  auto store = [&](int i, float t, int prim, float u) {
+  auto store_hit = [&](int i, float t, int prim, float u) {
     prim_out[i] = prim;
     if (t_out) t_out[i] = t;
     if (u_out) u_out[i] = u;
   };
   auto store_any = [&](int i, bool hit) { prim_out[i] = hit ? 1 : 0; };
-  if constexpr (kCurves) {
-    const CurveLeaf leaf{sc.curves, sc.curve_caps};
-    if (any_hit) any_stream<kCount>(sc, st, n, leaf, cnt, load, store_any);
-    else closest_stream<kCount>(sc, st, n, leaf, cnt, load, store);
-  } else {
-    if (any_hit) any_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store_any);
-    else closest_stream<kCount>(sc, st, n, SegLeaf{}, cnt, load, store);
-  }
-  if (kCount) flush_counters(cnt, &stats[0], &stats[1], &stats[4]);
+  const int n_closest = any_hit ? 0 : n, n_any = any_hit ? n : 0;
+  if constexpr (kCurves)
+    trace_stream<kCount>(sc, st, n_closest, n_any, CurveLeaf{sc.curves, sc.curve_caps}, cnt, load, store_hit,
+                         store_any);
+  else
+    trace_stream<kCount>(sc, st, n_closest, n_any, SegLeaf{}, cnt, load, store_hit, store_any);
+  if (kCount) flush_counters(cnt[any_hit ? 1 : 0], &stats[0], &stats[1], &stats[4]);
 }
 
 // ---------------------------------------------------------------------------
 // Host launchers
+
+// Blocks of a trace launch of at most n rays.
+static int trace_grid(int cap, long long n) {
+  return (int)std::min<long long>(cap, std::max<long long>(1, (n + kTraceBlock - 1) / kTraceBlock));
+}
+
+// One trace launch; with a timer, its closest hits (record kind 0) and its
+// shadow rays (kind 2) as launches of their own.
+static void launch_trace(bool count, bool dense, const SceneView& sc, const PathBuffers& pb, const PathBuffers& nb,
+                         TraceArgs a, int blocks, PassTimer* tm, unsigned long long* stats, hipStream_t st) {
+  auto go = [&](int kind, TraceArgs x) {
+    const dim3 g(blocks), b(kTraceBlock);
+    const bool curves = sc.curves != nullptr;
+    if (dense && curves) launch_timed(tm, kind, k_trace<false, true, true>, g, b, st, sc, pb, nb, x, stats);
+    else if (dense) launch_timed(tm, kind, k_trace<false, true, false>, g, b, st, sc, pb, nb, x, stats);
+    else if (count && curves) launch_timed(tm, kind, k_trace<true, false, true>, g, b, st, sc, pb, nb, x, stats);
+    else if (count) launch_timed(tm, kind, k_trace<true, false, false>, g, b, st, sc, pb, nb, x, stats);
+    else if (curves) launch_timed(tm, kind, k_trace<false, false, true>, g, b, st, sc, pb, nb, x, stats);
+    else launch_timed(tm, kind, k_trace<false, false, false>, g, b, st, sc, pb, nb, x, stats);
+  };
+  if (!tm || a.what != 3) {
+    go(a.what == 2 ? 2 : 0, a);
+    return;
+  }
+  go(0, TraceArgs{a.wave, a.set, 1, a.clear});
+  go(2, TraceArgs{a.wave, a.set, 2, 0});
+}
 
 int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hipStream_t stream,
                 std::string& err) {
@@ -836,30 +828,21 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
   }
   HM_TRY(check_launch("camera", err));
   const bool count = cfg.stats != nullptr;
-  const bool curves = sc.curves != nullptr;
   PassTimer* tm = cfg.timer;
 
   // Grids sized to the pass's paths (queues only shrink with depth), so a
   // small training-data pass does not dispatch the full-frame grid per depth.
   const int n0 = cfg.camera_mode != 0 ? cfg.n_slots : sc.width * sc.height;
-  const int ext_blocks = std::min(cfg.trace_blocks, std::max(1, (n0 + kTraceBlock - 1) / kTraceBlock));
-  const int sh_blocks = std::min(cfg.trace_blocks, std::max(1, (2 * n0 + kTraceBlock - 1) / kTraceBlock));
+  const int ext_blocks = trace_grid(cfg.trace_blocks, n0);
+  const int tr_blocks = trace_grid(cfg.trace_blocks, 3ll * n0);
   const int shade_blocks = std::min(cfg.shade_blocks, std::max(1, (n0 + 255) / 256));
   int cur = 0;
+  launch_trace(count, false, sc, pb, pb, TraceArgs{0, 1, 1, 1}, ext_blocks, tm, cfg.stats, stream);
   // depth 0 always runs: a camera miss shows the environment even when
   // pathTrace itself returns black (path_tracing.cu:50-57)
-  for (int depth = 0; depth <= std::max(0, cfg.max_vertex); ++depth) {
+  const int last = std::max(0, cfg.max_vertex);
+  for (int depth = 0; depth <= last; ++depth) {
     const int nxt = cur ^ 1;
-    hipLaunchKernelGGL(k_reset_counts, dim3(1), dim3(64), 0, stream, pb.counts, nxt, 2, 3);
-    const dim3 eg(ext_blocks), tb(kTraceBlock);
-    if (curves && count)
-      launch_timed(tm, 0, k_extend<true, false, true>, eg, tb, stream, sc, pb, cur, cfg.stats);
-    else if (curves)
-      launch_timed(tm, 0, k_extend<false, false, true>, eg, tb, stream, sc, pb, cur, cfg.stats);
-    else if (count)
-      launch_timed(tm, 0, k_extend<true>, eg, tb, stream, sc, pb, cur, cfg.stats);
-    else
-      launch_timed(tm, 0, k_extend<false>, eg, tb, stream, sc, pb, cur, cfg.stats);
     ShadeParams sp;
     sp.depth = depth;
     sp.dl_zero = cfg.dl_zero;
@@ -868,20 +851,14 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
     sp.trunc_beta = cfg.trunc_beta;
     sp.msnn = cfg.msnn;
     sp.cur = cur;
+    sp.set = depth & 1;
     if (cfg.nrc.enabled)
-      launch_timed(tm, 1, k_shade_nrc, dim3(shade_blocks), dim3(256), stream, sc, pb, depth, cur, cfg.nrc);
+      launch_timed(tm, 1, k_shade_nrc, dim3(shade_blocks), dim3(256), stream, sc, pb, sp, cfg.nrc);
     else
       launch_timed(tm, 1, k_shade, dim3(shade_blocks), dim3(256), stream, sc, pb, sp, cfg.gb);
-    const dim3 sg(sh_blocks);
-    if (curves && count)
-      launch_timed(tm, 2, k_shadow<true, true>, sg, tb, stream, sc, pb, cfg.stats);
-    else if (curves)
-      launch_timed(tm, 2, k_shadow<false, true>, sg, tb, stream, sc, pb, cfg.stats);
-    else if (count)
-      launch_timed(tm, 2, k_shadow<true>, sg, tb, stream, sc, pb, cfg.stats);
-    else
-      launch_timed(tm, 2, k_shadow<false>, sg, tb, stream, sc, pb, cfg.stats);
-    launch_timed(tm, 3, k_shadow_resolve, dim3(shade_blocks), dim3(256), stream, pb, cfg.msnn, depth, cfg.nrc);
+    launch_trace(count, false, sc, pb, pb, TraceArgs{nxt, sp.set, depth < last ? 3 : 2, 1}, tr_blocks, tm, cfg.stats,
+                 stream);
+    launch_timed(tm, 3, k_shadow_resolve, dim3(shade_blocks), dim3(256), stream, pb, cfg.msnn, depth, sp.set, cfg.nrc);
     HM_TRY(check_launch("wavefront vertex", err));
     cur = nxt;
   }
@@ -908,10 +885,10 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
 // ctl (64-bit, per group): two copies of the scheduler state, each [0] next
 // job, [1] passes accumulated, [2] free path capacity (set by the finishing
 // kernel), [8 + r] finished jobs of ring entry r.
-__global__ void k_stream_init(long long* ctl, int* counts, int slots) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < kStreamCtl) ctl[i] = i == 2 ? slots : 0;
-  if (i <= kDoneCount) counts[kCountStride * i] = 0;
+__global__ void k_stream_init(long long* ctl, int* counts) {
+  const int i = threadIdx.x;
+  if (i < kStreamCtl) ctl[i] = 0;
+  if (i < kCountInts / kCountStride) counts[kCountStride * i] = 0;
 }
 
 // Pixel px's planned passes p0 .. p0 + k - 1 from the ring into the running
@@ -937,18 +914,16 @@ __device__ __forceinline__ void accumulate_planned(const float4* ring, float4* a
   average[px] = make_float4(c.x * inv, c.y * inv, c.z * inv, 1.f);
 }
 
-// Finished paths from the finished list into the ring, counted per ring
-// entry; the free capacity for the plan; the new jobs' camera rays appended
-// to wavefront nb after the continuing paths.
-__global__ void k_stream_finish_dense(PathBuffers pb, long long* ctl, float4* ring, int npx, int nxt, int slots) {
+// Finished paths from the finished list into the ring, counted per ring entry
+// in the scheduler state T.
+__global__ void k_stream_finish_dense(PathBuffers pb, long long* T, float4* ring, int npx, int set) {
   // finished jobs per ring entry, counted in LDS; one global atomic per
   // block and entry (every block's waves adding to the same few counters
   // serialised on them)
   __shared__ int per_entry[kStreamRing];
   if (threadIdx.x < kStreamRing) per_entry[threadIdx.x] = 0;
   __syncthreads();
-  const int n = pb.counts[kCountStride * kDoneCount];
-  if (blockIdx.x == 0 && threadIdx.x == 0) ctl[2] = slots - pb.counts[kCountStride * nxt];  // free path capacity
+  const int n = pb.counts[append_count(set, kDoneCount)];
   const int stride = gridDim.x * blockDim.x;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     const int r = pb.done_pass[i] % kStreamRing;
@@ -957,24 +932,26 @@ __global__ void k_stream_finish_dense(PathBuffers pb, long long* ctl, float4* ri
   }
   __syncthreads();
   if (threadIdx.x < kStreamRing && per_entry[threadIdx.x] > 0)
-    atomicAdd((unsigned long long*)&ctl[8 + threadIdx.x], (unsigned long long)per_entry[threadIdx.x]);
+    atomicAdd((unsigned long long*)&T[8 + threadIdx.x], (unsigned long long)per_entry[threadIdx.x]);
 }
 
-// Plans and runs the next step of a group from scheduler state S (written
-// by the previous call and updated by the finishing kernel in between): every
-// thread derives the same plan from S (passes whose jobs are all done, at
-// most a ring's worth, are accumulated; free capacity x jobs inside the
-// window are issued), one thread writes the state after it to T and clears
-// the iteration's counters. Then the completed passes are added to the image
-// and the new jobs' camera rays appended to wavefront nb.
+// Plans and runs the next step of a group from scheduler state S (written by
+// the previous call and updated by the finishing kernel in between): every
+// thread derives the same plan from S and the number of continuing paths
+// (passes whose jobs are all done, at most a ring's worth, are accumulated;
+// free capacity x jobs inside the window are issued), one thread writes the
+// state after it to T and the new wavefront's length and clears the other
+// append set. Then the completed passes are added to the image and the new
+// jobs' camera rays appended to wavefront nb after the continuing paths.
 __global__ void k_stream_next_dense(SceneView sc, PathBuffers nb, const long long* S, long long* T, const float4* ring,
-                                    float4* accum, float4* average, int cur, int nxt, int first_pass, int seed_offset,
-                                    int npx, int g, int K, int cnt, int passes) {
+                                    float4* accum, float4* average, int nxt, int set, int slots, int first_pass,
+                                    int seed_offset, int npx, int g, int K, int cnt, int passes) {
   const long long acc = S[1], job0 = S[0];
   int k = 0;
   while (acc + k < passes && k < kStreamRing && S[8 + (int)((acc + k) % kStreamRing)] == cnt) ++k;
   const long long limit = (long long)min((long long)passes, acc + k + kStreamRing) * cnt;
-  const int n = (int)max(0ll, min(S[2], limit - job0));
+  const int cont = nb.counts[append_count(set, kNextCount)];
+  const int n = (int)max(0ll, min((long long)(slots - cont), limit - job0));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     T[0] = job0 + n;
     T[1] = acc + k;
@@ -982,21 +959,16 @@ __global__ void k_stream_next_dense(SceneView sc, PathBuffers nb, const long lon
       const long long d = (r - acc % kStreamRing + kStreamRing) % kStreamRing;  // ring entry r holds pass acc + d
       T[8 + r] = d < k ? 0 : S[8 + r];
     }
-    nb.counts[kCountStride * cur] = 0;
-    nb.counts[kCountStride * 2] = 0;
-    nb.counts[kCountStride * 3] = 0;
-    nb.counts[kCountStride * kDoneCount] = 0;
+    nb.counts[wave_count(nxt)] = cont + n;
+    for (int q = 0; q < 4; ++q) nb.counts[append_count(set ^ 1, q)] = 0;
   }
   const int work = max(k > 0 ? cnt : 0, n);
   const int stride = gridDim.x * blockDim.x;
-  const int nloop = (work + stride - 1) / stride * stride;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nloop; i += stride) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < work; i += stride) {
     if (k > 0 && i < cnt) accumulate_planned(ring, accum, average, acc, k, first_pass, npx, stream_group_pixel(i, g, K));
-    const bool go = i < n;
-    const int q = block_append1(&nb.counts[kCountStride * nxt], go);
-    if (go) {
+    if (i < n) {
       const long long job = job0 + i;
-      const int pass = (int)(job / cnt);
+      const int pass = (int)(job / cnt), q = cont + i;
       const int px = stream_group_pixel((int)(job % cnt), g, K);
       camera_path(sc, nb, q, px, first_pass + pass + seed_offset);
       nb.slot_pass[q] = pass;
@@ -1062,9 +1034,11 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
     long long* c = ctl + (size_t)g * kStreamCtl;
     const int slots = group_slots(cnt);
     const int blocks = (std::max(cnt, slots) + 255) / 256;
-    hipLaunchKernelGGL(k_stream_init, dim3(1), dim3(kStreamCtl), 0, streams[g], c, pbs[g]->counts, slots);
+    hipLaunchKernelGGL(k_stream_init, dim3(1), dim3(kStreamCtl), 0, streams[g], c, pbs[g]->counts);
     hipLaunchKernelGGL(k_stream_next_dense, dim3(blocks), dim3(256), 0, streams[g], sc, *pbs[g], c, c + kStreamHalf,
-                       ring, accum, average, 1, 0, cfg.accum_id, cfg.seed_offset, npx, g, K, cnt, passes);
+                       ring, accum, average, 0, 1, slots, cfg.accum_id, cfg.seed_offset, npx, g, K, cnt, passes);
+    launch_trace(false, true, sc, *pbs[g], *pbs[g], TraceArgs{0, 1, 1, 0}, trace_grid(cfg.trace_blocks, slots),
+                 g == 0 ? tm : nullptr, nullptr, streams[g]);
     calls[g] = 1;
   }
   HM_TRY(check_launch("stream start", err));
@@ -1091,21 +1065,13 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
       hipStream_t st = streams[g];
       const int cnt = stream_group_slots(npx, g, K);
       const int slots = group_slots(cnt);
-      const int ext_blocks = std::min(cfg.trace_blocks, std::max(1, (slots + kTraceBlock - 1) / kTraceBlock));
-      const int sh_blocks = std::min(cfg.trace_blocks, std::max(1, (2 * slots + kTraceBlock - 1) / kTraceBlock));
+      const int tr_blocks = trace_grid(cfg.trace_blocks, 3ll * slots);
       const int shade_blocks = std::min(cfg.shade_blocks, std::max(1, (std::max(cnt, slots) + 255) / 256));
-      const bool timed = g == 0 && tm;
+      PassTimer* t = g == 0 ? tm : nullptr;
       for (int k = 0; k < kBatch; ++k) {
         const int nxt = cur[g] ^ 1;
         const PathBuffers& A = views[cur[g]];
         const PathBuffers& B = views[nxt];
-        PassTimer* t = timed ? tm : nullptr;
-        if (sc.curves)
-          launch_timed(t, 0, k_extend<false, true, true>, dim3(ext_blocks), dim3(kTraceBlock), st, sc, A, cur[g],
-                       (unsigned long long*)nullptr);
-        else
-          launch_timed(t, 0, k_extend<false, true>, dim3(ext_blocks), dim3(kTraceBlock), st, sc, A, cur[g],
-                       (unsigned long long*)nullptr);
         ShadeParams sp;
         sp.depth = 0;
         sp.dl_zero = cfg.dl_zero;
@@ -1114,28 +1080,24 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
         sp.trunc_beta = cfg.trunc_beta;
         sp.msnn = 0;
         sp.cur = cur[g];
+        sp.set = cur[g];  // the state copies and the append sets alternate together
         launch_timed(t, 1, k_shade_dense, dim3(shade_blocks), dim3(256), st, sc, A, B, sp);
-        if (sc.curves)
-          launch_timed(t, 2, k_shadow<false, true>, dim3(sh_blocks), dim3(kTraceBlock), st, sc, A,
-                       (unsigned long long*)nullptr);
-        else
-          launch_timed(t, 2, k_shadow<false>, dim3(sh_blocks), dim3(kTraceBlock), st, sc, A,
-                       (unsigned long long*)nullptr);
-        launch_timed(t, 3, k_shadow_resolve_dense, dim3(shade_blocks), dim3(256), st, A, B);
-        // scheduler state: next call m reads half m % 2 and writes the other
+        // scheduler state: call m reads half m % 2 and writes the other
         long long* c = ctl + (size_t)g * kStreamCtl;
         long long* S = c + kStreamHalf * (calls[g] & 1);
         long long* T = c + kStreamHalf * ((calls[g] + 1) & 1);
-        launch_timed(t, 3, k_stream_finish_dense, dim3(shade_blocks), dim3(256), st, A, S, ring, npx, nxt, slots);
-        launch_timed(t, 3, k_stream_next_dense, dim3(shade_blocks), dim3(256), st, sc, B, S, T, ring, accum,
-                     average, cur[g], nxt, cfg.accum_id, cfg.seed_offset, npx, g, K, cnt, passes);
+        launch_timed(t, 3, k_stream_next_dense, dim3(shade_blocks), dim3(256), st, sc, B, S, T, ring, accum, average,
+                     nxt, sp.set, slots, cfg.accum_id, cfg.seed_offset, npx, g, K, cnt, passes);
+        launch_trace(false, true, sc, A, B, TraceArgs{nxt, sp.set, 3, 0}, tr_blocks, t, nullptr, st);
+        launch_timed(t, 3, k_shadow_resolve_dense, dim3(shade_blocks), dim3(256), st, A, B, sp.set);
+        launch_timed(t, 3, k_stream_finish_dense, dim3(shade_blocks), dim3(256), st, A, T, ring, npx, sp.set);
         ++calls[g];
         cur[g] = nxt;
       }
       iters[g] += kBatch;
       HM_TRY(check_launch("stream iteration", err));
       const int s = 2 * g + (batch & 1);
-      HM_HIP(hipMemcpyAsync(&live_host[s], pb.counts + kCountStride * cur[g], sizeof(int), hipMemcpyDeviceToHost, st),
+      HM_HIP(hipMemcpyAsync(&live_host[s], pb.counts + wave_count(cur[g]), sizeof(int), hipMemcpyDeviceToHost, st),
              err);
       HM_HIP(hipEventRecord(live_ev[s], st), err);
     }
@@ -1177,22 +1139,15 @@ struct JobCamera {
   int* pix;
 };
 
-__global__ void k_jobs_init(long long* ctl, int* counts, int capacity) {
+__global__ void k_jobs_init(long long* ctl, int* counts) {
   const int i = threadIdx.x;
-  if (i < kJobCtl) ctl[i] = i == 2 ? capacity : 0;
-  if (i <= kDoneCount) counts[kCountStride * i] = 0;
+  if (i < kJobCtl) ctl[i] = 0;
+  if (i < kCountInts / kCountStride) counts[kCountStride * i] = 0;
 }
 
-// Finished paths' radiance to their records; the free capacity for the
-// next issue; one more live iteration if the wavefront just shaded (cur)
-// held paths.
-__global__ void k_jobs_finish(PathBuffers pb, long long* S, long long* ctl, int cur, int nxt, int capacity,
-                              float4* out_L, float4* out_Ls) {
-  const int n = pb.counts[kCountStride * kDoneCount];
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    S[2] = capacity - pb.counts[kCountStride * nxt];
-    if (pb.counts[kCountStride * cur] > 0) ctl[kJobCtlLive] += 1;
-  }
+// Finished paths' radiance to their records.
+__global__ void k_jobs_finish(PathBuffers pb, int set, float4* out_L, float4* out_Ls) {
+  const int n = pb.counts[append_count(set, kDoneCount)];
   const int stride = gridDim.x * blockDim.x;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
     const int job = pb.done_px[i];
@@ -1202,34 +1157,30 @@ __global__ void k_jobs_finish(PathBuffers pb, long long* S, long long* ctl, int 
 }
 
 // Issues min(free capacity, records left) new records into wavefront nb
-// after its continuing paths, and clears the counters the next iteration
-// appends to. Every thread derives the same count from S.
-__global__ void k_jobs_next(SceneView sc, PathBuffers nb, const long long* S, long long* T, int cur, int nxt,
-                            JobCamera jc) {
+// after its continuing paths, sets the wavefront's length and clears the
+// other append set; one more live iteration if the wavefront holds paths.
+// Every thread derives the same count from S.
+__global__ void k_jobs_next(SceneView sc, PathBuffers nb, const long long* S, long long* T, long long* ctl, int nxt,
+                            int set, int capacity, JobCamera jc) {
   const long long job0 = S[0];
-  const int n = (int)max(0ll, min(S[2], (long long)jc.n_jobs - job0));
+  const int cont = nb.counts[append_count(set, kNextCount)];
+  const int n = (int)max(0ll, min((long long)(capacity - cont), (long long)jc.n_jobs - job0));
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     T[0] = job0 + n;
-    nb.counts[kCountStride * cur] = 0;
-    nb.counts[kCountStride * 2] = 0;
-    nb.counts[kCountStride * 3] = 0;
-    nb.counts[kCountStride * kDoneCount] = 0;
+    if (cont + n > 0) ctl[kJobCtlLive] += 1;
+    nb.counts[wave_count(nxt)] = cont + n;
+    for (int q = 0; q < 4; ++q) nb.counts[append_count(set ^ 1, q)] = 0;
   }
   const int stride = gridDim.x * blockDim.x;
-  const int nloop = (n + stride - 1) / stride * stride;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nloop; i += stride) {
-    const bool go = i < n;
-    const int q = block_append1(&nb.counts[kCountStride * nxt], go);
-    if (go) {
-      const int job = (int)(job0 + i);
-      if (jc.mode == 1)
-        camera_train_point(sc, nb, q, job, jc.accum_id, jc.chunk, jc.grid_w, jc.points);
-      else
-        camera_train_pixel(sc, nb, q, job, jc.accum_id, jc.chunk, jc.every_nth, jc.train_idx, jc.pix);
-      nb.slot_pass[q] = 0;
-      nb.slot_px[q] = job;
-      nb.slot_depth[q] = 0;
-    }
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const int job = (int)(job0 + i), q = cont + i;
+    if (jc.mode == 1)
+      camera_train_point(sc, nb, q, job, jc.accum_id, jc.chunk, jc.grid_w, jc.points);
+    else
+      camera_train_pixel(sc, nb, q, job, jc.accum_id, jc.chunk, jc.every_nth, jc.train_idx, jc.pix);
+    nb.slot_pass[q] = 0;
+    nb.slot_px[q] = job;
+    nb.slot_depth[q] = 0;
   }
 }
 
@@ -1259,10 +1210,12 @@ int pt_jobs_start(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, i
   }
   run = JobRun{};
   run.capacity = capacity;
-  hipLaunchKernelGGL(k_jobs_init, dim3(1), dim3(64), 0, stream, pb.job_ctl, pb.counts, capacity);
+  hipLaunchKernelGGL(k_jobs_init, dim3(1), dim3(64), 0, stream, pb.job_ctl, pb.counts);
   // first issue into wavefront 0 (state copy 0)
   hipLaunchKernelGGL(k_jobs_next, dim3(job_blocks(capacity, cfg.shade_blocks, 256)), dim3(256), 0, stream, sc, pb,
-                     pb.job_ctl, pb.job_ctl + kJobCtlHalf, 1, 0, job_camera(cfg));
+                     pb.job_ctl, pb.job_ctl + kJobCtlHalf, pb.job_ctl, 0, 1, capacity, job_camera(cfg));
+  launch_trace(false, true, sc, pb, pb, TraceArgs{0, 1, 1, 0}, trace_grid(cfg.trace_blocks, capacity), nullptr,
+               nullptr, stream);
   run.calls = 1;
   run.cur = 0;
   return check_launch("job schedule start", err);
@@ -1272,8 +1225,7 @@ int pt_jobs_iterate(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg,
                     float4* out_L, float4* out_Ls, hipStream_t stream, std::string& err) {
   const PathBuffers views[2] = {pb, other_state(pb)};
   const int C = run.capacity;
-  const int ext_blocks = job_blocks(C, cfg.trace_blocks, kTraceBlock);
-  const int sh_blocks = job_blocks(2 * C, cfg.trace_blocks, kTraceBlock);
+  const int tr_blocks = trace_grid(cfg.trace_blocks, 3ll * C);
   const int shade_blocks = job_blocks(C, cfg.shade_blocks, 256);
   const JobCamera jc = job_camera(cfg);
   ShadeParams sp;
@@ -1289,24 +1241,14 @@ int pt_jobs_iterate(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg,
     const PathBuffers& A = views[cur];
     const PathBuffers& B = views[nxt];
     sp.cur = cur;
-    if (sc.curves)
-      hipLaunchKernelGGL((k_extend<false, true, true>), dim3(ext_blocks), dim3(kTraceBlock), 0, stream, sc, A, cur,
-                         (unsigned long long*)nullptr);
-    else
-      hipLaunchKernelGGL((k_extend<false, true>), dim3(ext_blocks), dim3(kTraceBlock), 0, stream, sc, A, cur,
-                         (unsigned long long*)nullptr);
+    sp.set = cur;
     hipLaunchKernelGGL(k_shade_dense_msnn, dim3(shade_blocks), dim3(256), 0, stream, sc, A, B, sp, cfg.gb);
-    if (sc.curves)
-      hipLaunchKernelGGL((k_shadow<false, true>), dim3(sh_blocks), dim3(kTraceBlock), 0, stream, sc, A,
-                         (unsigned long long*)nullptr);
-    else
-      hipLaunchKernelGGL((k_shadow<false>), dim3(sh_blocks), dim3(kTraceBlock), 0, stream, sc, A,
-                         (unsigned long long*)nullptr);
-    hipLaunchKernelGGL(k_shadow_resolve_dense_msnn, dim3(shade_blocks), dim3(256), 0, stream, A, B);
     long long* S = c + kJobCtlHalf * (run.calls & 1);
     long long* T = c + kJobCtlHalf * ((run.calls + 1) & 1);
-    hipLaunchKernelGGL(k_jobs_finish, dim3(shade_blocks), dim3(256), 0, stream, A, S, c, cur, nxt, C, out_L, out_Ls);
-    hipLaunchKernelGGL(k_jobs_next, dim3(shade_blocks), dim3(256), 0, stream, sc, B, S, T, cur, nxt, jc);
+    hipLaunchKernelGGL(k_jobs_next, dim3(shade_blocks), dim3(256), 0, stream, sc, B, S, T, c, nxt, sp.set, C, jc);
+    launch_trace(false, true, sc, A, B, TraceArgs{nxt, sp.set, 3, 0}, tr_blocks, nullptr, nullptr, stream);
+    hipLaunchKernelGGL(k_shadow_resolve_dense_msnn, dim3(shade_blocks), dim3(256), 0, stream, A, B, sp.set);
+    hipLaunchKernelGGL(k_jobs_finish, dim3(shade_blocks), dim3(256), 0, stream, A, sp.set, out_L, out_Ls);
     ++run.calls;
     ++run.iters;
     run.cur = nxt;
@@ -1319,7 +1261,7 @@ int pt_jobs_status(const PathBuffers& pb, const JobRun& run, long long* host, hi
   // the wavefront count is an int: it lands in the low half of host[0]
   // (little-endian), whose high half is cleared here
   host[0] = 0;
-  HM_HIP(hipMemcpyAsync(host, pb.counts + kCountStride * run.cur, sizeof(int), hipMemcpyDeviceToHost, stream), err);
+  HM_HIP(hipMemcpyAsync(host, pb.counts + wave_count(run.cur), sizeof(int), hipMemcpyDeviceToHost, stream), err);
   HM_HIP(hipMemcpyAsync(host + 1, pb.job_ctl + kJobCtlLive, sizeof(long long), hipMemcpyDeviceToHost, stream), err);
   HM_HIP(hipEventRecord(ev, stream), err);
   return kOk;
