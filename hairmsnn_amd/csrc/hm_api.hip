@@ -216,7 +216,7 @@ int alloc_path_buffers(PathBuffers& pb, std::vector<void*>& allocs, size_t n, bo
 }
 
 int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots) {
-  const int want = std::max(scene.width * scene.height, min_slots);
+  const int want = std::max(stream_slots(scene.width * scene.height), min_slots);
   if (pb.ray_o && (!msnn_mode || pb_msnn) && pb_slots >= want) return kOk;
   free_path_buffers();
   const size_t n = (size_t)want;
@@ -233,11 +233,11 @@ int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots
   return kOk;
 }
 
-// Path-tracing buffers for flights 1.. (flight 0 is pb).
-int Context::ensure_flights(std::string& err) {
+// Path-tracing buffers for flights 1 .. count - 1 (flight 0 is pb).
+int Context::ensure_flights(int count, std::string& err) {
   if (!acc_event) HM_HIP(hipEventCreateWithFlags(&acc_event, hipEventDisableTiming), err);
-  const int want = scene.width * scene.height;
-  for (int f = 1; f < num_flights; ++f) {
+  const int want = stream_slots(scene.width * scene.height);
+  for (int f = 1; f < count; ++f) {
     Flight& fl = extra[f - 1];
     if (!fl.stream) HM_HIP(hipStreamCreateWithFlags(&fl.stream, hipStreamNonBlocking), err);
     if (fl.slots >= want) continue;
@@ -791,10 +791,10 @@ namespace hm {
 int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* avg, PassTimer* timer,
                   std::string& err) {
   HM_TRY(c.ensure_path_buffers(false, err));
-  HM_TRY(c.ensure_flights(err));
   const int n = c.scene.width * c.scene.height;
-  const int K = std::max(1, std::min(c.num_flights, Context::kMaxFlights));
   if (passes <= 0) return kOk;
+  const int K = (long long)n * passes < kTwoGroupJobs ? 1 : std::max(1, std::min(c.num_flights, kStreamGroups));
+  HM_TRY(c.ensure_flights(K, err));
   if (!c.live_host) {
     HM_HIP(hipHostMalloc((void**)&c.live_host, 2 * Context::kMaxFlights * sizeof(int)), err);
     for (hipEvent_t& e : c.live_ev) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
@@ -818,8 +818,8 @@ int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* a
   PassConfig cfg = c.pt_pass_config();
   cfg.accum_id = first_pass;
   cfg.timer = timer;
-  HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, acc, avg, c.stream_ring, c.stream_ctl, c.live_host,
-                       c.live_ev, err));
+  HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, stream_slots(n), acc, avg, c.stream_ring, c.stream_ctl,
+                       c.live_host, c.live_ev, err));
   // the context stream waits for every group
   for (int g = 1; g < K; ++g) {
     HM_HIP(hipEventRecord(c.acc_event, sts[g]), err);
@@ -841,18 +841,17 @@ static int run_pt_passes(Context& c, int passes, std::string& err, PassTimer* ti
   SceneView v = c.view;
   v.bvh.nodes = c.bvh.nodes_w;
   const int n = c.scene.width * c.scene.height;
-  HM_TRY(c.ensure_flights(err));
-  const int K = std::max(1, std::min(c.num_flights, Context::kMaxFlights));
   if (c.pt_schedule == 0) {
     if (passes <= 0) return kOk;
     HM_TRY(stream_passes(c, c.accum_id, passes, c.accum, c.average, timer, err));
     c.last_ring_entry = (passes - 1) % kStreamRing;
     c.accum_id += passes;
     c.last_streamed = true;
-    c.stream_groups = K;
     return kOk;
   }
   c.last_streamed = false;
+  const int K = std::max(1, std::min(c.num_flights, Context::kMaxFlights));
+  HM_TRY(c.ensure_flights(K, err));
   hipEvent_t start = nullptr;
   HM_HIP(hipEventCreateWithFlags(&start, hipEventDisableTiming), err);
   HM_HIP(hipEventRecord(start, c.stream), err);

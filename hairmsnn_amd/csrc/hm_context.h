@@ -96,13 +96,12 @@ struct Context {
   // path buffers), 1 one wavefront per pass with passes in flight
   int pt_schedule = 0;
   bool last_streamed = false;   // the last pt call used the streaming schedule
-  int stream_groups = 1;        // groups of that call
   int* live_host = nullptr;     // pinned, 2 per group: live-path count polls
   float4* stream_ring = nullptr;  // streaming schedule: kStreamRing passes of radiance per pixel
   long long* stream_ctl = nullptr;  // streaming schedule: scheduler counters per group
   int last_ring_entry = 0;          // ring entry of the last streamed pass
   hipEvent_t live_ev[2 * kMaxFlights] = {};
-  int ensure_flights(std::string& err);
+  int ensure_flights(int count, std::string& err);
   PathBuffers& flight_pb(int f) { return f == 0 ? pb : extra[f - 1].pb; }
   hipStream_t flight_stream(int f) { return f == 0 ? stream : extra[f - 1].stream; }
   // HairMSNN scene samples on the hair (3 floats each), made once per scene

@@ -869,22 +869,23 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
 // A job queue over a compacted wavefront. A job is (pass, pixel): job j of a
 // call is pass j / cnt of the group's pixel j % cnt, so jobs are handed out in
 // pass order, and a pixel's passes can run at the same time on different
-// paths. Each iteration: extend the current wavefront (path i at index i),
-// shade it (continuing paths written densely into the other copy of the
-// per-path state, finished ones into a finished list), trace and resolve the
-// shadow rays, move the finished radiance into a ring of kStreamRing passes
-// (indexed by the global pixel), plan, then add the passes whose jobs are all
-// done to the image (in pass order, so the accumulation and the image are the
-// per-pass schedule's) and append new jobs' camera rays after the continuing
-// paths, up to the group's path capacity. Jobs of pass p start only while
-// p < (accumulated passes) + kStreamRing, so the ring never overwrites a pass
-// that is not accumulated yet. The pixels are split into K groups, each with
-// its own path buffers and stream, so that one group's shading overlaps
-// another's traversal: group g owns the 64-pixel chunks g, g + K, g + 2K, ...
-// (balanced work, coherent camera rays within a wave).
+// paths. Each iteration: shade the current wavefront (path i at index i;
+// continuing paths written densely into the other copy of the per-path state,
+// finished ones into a finished list); plan: the passes whose jobs were all
+// done by the previous iteration are added to the image (in pass order, so
+// the accumulation and the image are the per-pass schedule's), and new jobs'
+// camera rays are appended after the continuing paths, up to the group's path
+// capacity; trace the new wavefront's closest hits together with the shaded
+// vertices' shadow rays; resolve the shadow rays; move the finished radiance
+// into a ring of kStreamRing passes (indexed by the global pixel). Jobs of
+// pass p start only while p < (accumulated passes) + kStreamRing, so the ring
+// never overwrites a pass that is not accumulated yet. The pixels are split
+// into K groups, each with its own path buffers and stream, so that one
+// group's shading overlaps another's traversal: group g owns the 64-pixel
+// chunks g, g + K, g + 2K, ... (balanced work, coherent camera rays within a
+// wave).
 // ctl (64-bit, per group): two copies of the scheduler state, each [0] next
-// job, [1] passes accumulated, [2] free path capacity (set by the finishing
-// kernel), [8 + r] finished jobs of ring entry r.
+// job, [1] passes accumulated, [8 + r] finished jobs of ring entry r.
 __global__ void k_stream_init(long long* ctl, int* counts) {
   const int i = threadIdx.x;
   if (i < kStreamCtl) ctl[i] = 0;
@@ -1008,24 +1009,18 @@ int stream_group_slots(int npx, int g, int K) {
 }
 
 int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_t* streams, int K,
-                  const PassConfig& cfg, int passes, float4* accum, float4* average, float4* ring, long long* ctl,
-                  int* live_host, hipEvent_t* live_ev, std::string& err) {
+                  const PassConfig& cfg, int passes, int slots_cap, float4* accum, float4* average, float4* ring,
+                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err) {
   const int npx = sc.width * sc.height;
   if (passes <= 0 || npx <= 0 || K < 1) return passes <= 0 ? kOk : (err = "bad stream groups", kEInval);
   PassTimer* tm = cfg.timer;
 
-// Two paths in flight per pixel of a group (four groups: 2M paths at 1024²)
-// measured 3% faster than one; four were 4% slower (a longer final drain).
-#ifndef HM_STREAM_SLOT_FACTOR
-#define HM_STREAM_SLOT_FACTOR 2
-#endif
   constexpr int kBatch = 8;  // even: each group's live queue is back at index 0 after a batch
   std::vector<int> cur(K, 0), live(K, 0), calls(K, 0);
   std::vector<long long> iters(K, 0);
-  // paths in flight per group: HM_STREAM_SLOT_FACTOR per pixel of the group,
-  // at most the npx slots its path buffers hold (jobs are still the group's
-  // pixels x passes)
-  auto group_slots = [&](int cnt) { return std::min(npx, HM_STREAM_SLOT_FACTOR * cnt); };
+  // paths in flight per group: what its buffers hold, but no more than the
+  // jobs the ring lets start
+  auto group_slots = [&](int cnt) { return (int)std::min<long long>(slots_cap, (long long)kStreamRing * cnt); };
   // first jobs: every slot free, then one issue round into queue 0
   for (int g = 0; g < K; ++g) {
     const int cnt = stream_group_slots(npx, g, K);
@@ -1125,10 +1120,10 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
 // ---- job schedule -----------------------------------------------------------
 // Records of a camera_mode 1 / 2 pass on a compacted wavefront (the path
 // kernels are those of the streaming schedule with HairMSNN training state):
-// each iteration extends, shades, traces and resolves the current
-// wavefront, moves the finished paths' radiance to their records' outputs
-// (k_jobs_finish) and appends new records' camera rays after the continuing
-// paths, up to the capacity (k_jobs_next). ctl holds two copies of the
+// each iteration shades the current wavefront, appends new records' camera
+// rays after the continuing paths, up to the capacity (k_jobs_next), traces
+// and resolves, and moves the finished paths' radiance to their records'
+// outputs (k_jobs_finish). ctl holds two copies of the
 // scheduler words; step m reads copy m % 2 and writes the other.
 
 struct JobCamera {

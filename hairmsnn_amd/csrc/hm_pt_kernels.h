@@ -162,6 +162,27 @@ inline int pt_jobs_bound(const PassConfig& cfg, int capacity) {
 
 // Passes the streaming schedule keeps in flight at most (its radiance ring).
 constexpr int kStreamRing = 16;
+// Stream groups at most, whatever hmsnn_set_pass_concurrency allows: two
+// groups' launches fill each other's tails, more only share the GPU's hardware
+// queues with whatever else the process runs (16 passes of the headline frame
+// took 62 to 75 ms with four, depending on which queues the streams got, 63
+// with two, 67 with one; a 640 x 363 frame of round curves 18.5 with three,
+// 17.1 with two). Calls of fewer jobs than kTwoGroupJobs run as one group: two
+// shorter wavefronts drain in as many launches each (128 x 128, 4 passes: 1.28
+// against 1.48 ms; 256 x 256, 16 passes: level).
+constexpr int kStreamGroups = 2;
+constexpr long long kTwoGroupJobs = 1 << 20;
+// Paths in flight over all groups. A launch ends with its longest rays, so
+// fewer and longer launches are better while there are jobs to fill them
+// (1, 2, 4 and 8 M paths: 64.9, 65.0, 62.9 and 62.2 ms on the headline frame),
+// and a small image keeps all its passes in flight (256 x 256, 16 passes: two
+// paths per pixel 4.0 ms, all 16 passes 2.6 ms). About 340 bytes per path.
+constexpr int kStreamPaths = 4 << 20;
+// Paths that a stream group's buffers hold for an image of npx pixels.
+inline int stream_slots(int npx) {
+  const long long share = kStreamPaths / kStreamGroups;
+  return (int)std::max<long long>(npx, std::min<long long>(share, (long long)kStreamRing * npx));
+}
 // Scheduler counters per stream group (64-bit).
 constexpr int kStreamCtl = 64;
 constexpr int kStreamHalf = 32;  // two copies of the scheduler state per group
@@ -175,11 +196,12 @@ static_assert(8 + kStreamRing <= kStreamHalf && 2 * kStreamHalf <= kStreamCtl, "
 // chunks dealt round-robin, the last one possibly partial), group g on pbs[g]
 // and streams[g] with ctl +
 // g * kStreamCtl; live_host (pinned, 2K ints) and live_ev (2K events) poll the
-// live-path counts. A timer records group 0's launches. The last pass's
+// live-path counts. slots_cap: paths that each group's buffers hold (at least
+// the image's pixels). A timer records group 0's launches. The last pass's
 // radiance is left in ring entry (passes - 1) % kStreamRing.
 int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_t* streams, int K,
-                  const PassConfig& cfg, int passes, float4* accum, float4* average, float4* ring, long long* ctl,
-                  int* live_host, hipEvent_t* live_ev, std::string& err);
+                  const PassConfig& cfg, int passes, int slots_cap, float4* accum, float4* average, float4* ring,
+                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err);
 // Pixels of stream group g of K over npx pixels, and the pixel of a group's
 // i-th pixel.
 int stream_group_slots(int npx, int g, int K);

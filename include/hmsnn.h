@@ -174,19 +174,20 @@ int hmsnn_set_strand_sigma_a(hmsnn_ctx* ctx, const float* sigma_host, int num_st
  * it lets a reference image and a test render use independent samples. */
 int hmsnn_set_seed_offset(hmsnn_ctx* ctx, int offset);
 /* Concurrency of path tracing (1..4, default 4): with the per-pass schedule
- * the passes kept in flight at once, with the streaming schedule the stream
- * groups the pixels are dealt to; each has its own path buffers and stream.
+ * the passes kept in flight at once, with the streaming schedule a limit on
+ * the stream groups the pixels are dealt to (at most two are used); each has
+ * its own path buffers and stream.
  * Accumulation stays in pass order, so the image does not depend on it. 1
  * runs everything on one stream (per-kernel timings of hmsnn_pt_time_passes
  * are then those of kernels running alone). No reference counterpart: the
  * reference renders one launch per frame. */
 int hmsnn_set_pass_concurrency(hmsnn_ctx* ctx, int passes_in_flight);
 /* Schedule of hmsnn_pt_passes. HMSNN_PT_STREAM (default): (pass, pixel)
- * jobs are handed out in pass order to a compacted wavefront of two paths per
- * pixel; a finished path's radiance waits in a 16-pass ring until its pass is
+ * jobs are handed out in pass order to a compacted wavefront of millions of
+ * paths; a finished path's radiance waits in a 16-pass ring until its pass is
  * complete, so each wavefront launch stays full until the call's last jobs
- * drain. hmsnn_set_pass_concurrency sets the number of stream groups the
- * pixels are dealt to. HMSNN_PT_PASSES: one wavefront per pass, passes in
+ * drain. hmsnn_set_pass_concurrency limits the stream groups the pixels are
+ * dealt to. HMSNN_PT_PASSES: one wavefront per pass, passes in
  * flight per hmsnn_set_pass_concurrency. Both accumulate each pixel's passes
  * in pass order: the images are equal. The setting also selects how
  * hmsnn_msnn_begin traces the warm-up's training records: HMSNN_PT_STREAM

@@ -164,6 +164,25 @@ def test_streaming_schedule_equals_pass_schedule(gpu, name, groups, calls, size)
     assert np.isfinite(imgs["stream"]).all() and imgs["stream"][..., :3].mean() > 0
 
 
+@pytest.mark.parametrize("calls", [(15,), (16,), (3, 33)])
+def test_streaming_schedule_two_groups(gpu, calls):
+    """Calls on both sides of the 2^20 jobs from which the streaming schedule
+    deals its pixels to two groups (128 x 513 has 1026 chunks of 64 pixels,
+    16 passes are the first call above), with the buffers of a small image
+    holding every pass the ring allows: the per-pass schedule's image, bit for
+    bit."""
+    cfg = scene_cfg("c0_hairball.json", 128, 513)
+    imgs = {}
+    for sched in ("passes", "stream"):
+        with gpu.Scene(json_text=cfg) as sc:
+            sc.set_pt_schedule(sched)
+            sc.pt_reset()
+            for n in calls:
+                sc.pt_passes(n)
+            imgs[sched] = sc.image(0).copy()
+    np.testing.assert_array_equal(imgs["stream"], imgs["passes"])
+
+
 def test_exr_environment_equals_procedural(gpu, tmp_path):
     """lights.environment.exr (loadEnvTexture, model.cpp:158-180): the
     procedural C0 environment written to a ZIP-compressed FLOAT EXR renders
