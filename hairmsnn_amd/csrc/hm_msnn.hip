@@ -87,8 +87,52 @@ struct TrainBatch {
   }
 };
 
+// Records of one warm-up job run; double-buffered, a run traces while the
+// previous one's steps train.
+struct WarmBuf {
+  std::vector<void*> allocs;
+  float* pts = nullptr;
+  float* input = nullptr;
+  float* target = nullptr;
+  uint8_t* hit = nullptr;
+  float4* L = nullptr;
+  float4* Ls = nullptr;
+  hipEvent_t ev_free = nullptr;
+  size_t rec = 0;  // records it holds
+  bool used = false;
+  void release() {
+    for (void* p : allocs) dev_free(p);
+    allocs.clear();
+    if (ev_free) (void)hipEventDestroy(ev_free), ev_free = nullptr;
+    rec = 0;
+  }
+  int ensure(size_t n, std::string& err) {
+    if (rec >= n) return kOk;
+    release();
+    auto A = [&](void** p, size_t bytes) -> int {
+      HM_TRY(dev_alloc(p, bytes, err));
+      allocs.push_back(*p);
+      return kOk;
+    };
+    HM_TRY(A((void**)&pts, sizeof(float) * 3 * n));
+    HM_TRY(A((void**)&input, sizeof(float) * 12 * n));
+    HM_TRY(A((void**)&target, sizeof(float) * 3 * n));
+    HM_TRY(A((void**)&hit, n));
+    HM_TRY(A((void**)&L, sizeof(float4) * n));
+    HM_TRY(A((void**)&Ls, sizeof(float4) * n));
+    HM_HIP(hipEventCreateWithFlags(&ev_free, hipEventDisableTiming), err);
+    rec = n;
+    return kOk;
+  }
+};
+
+// The buffers and streams stay with the context from one hmsnn_msnn_begin to
+// the next (about 3 GB at 1024 x 1024: allocating and freeing them took 75 ms
+// of a begin's 115); everything a run computes starts over.
 struct MsnnState {
   MlpState* mlp = nullptr;
+  bool ready = false;  // fully built (a failed setup is not reused)
+  int npx = 0;
   int BETA = 1;
   int kbeta = 0;       // kernel beta = BETA - 1
   int n_train = 0;     // training records per frame
@@ -113,6 +157,7 @@ struct MsnnState {
   int warm_batch = 1;
   MsnnSlot slots[kSlots];
   TrainBatch tb[2];
+  WarmBuf warm[2];
   float* nn_output = nullptr;    // W*H*3 (used in frame order on the context stream)
   float4* acc[3] = {nullptr, nullptr, nullptr};  // short, network, final
   float4* avg[3] = {nullptr, nullptr, nullptr};
@@ -130,6 +175,7 @@ struct MsnnState {
     if (batch_stream) (void)hipStreamDestroy(batch_stream);
     for (MsnnSlot& sl : slots) sl.release();
     for (TrainBatch& b : tb) b.release();
+    for (WarmBuf& b : warm) b.release();
     if (job_status) (void)hipHostFree(job_status);
     for (hipEvent_t& e : job_ev)
       if (e) (void)hipEventDestroy(e);
@@ -139,6 +185,22 @@ struct MsnnState {
       dev_free(acc[k]);
       dev_free(avg[k]);
     }
+  }
+  // Waits for the last run's work and forgets its results; the buffers stay.
+  int restart(std::string& err) {
+    HM_HIP(hipStreamSynchronize(ctx_stream), err);
+    if (batch_stream) HM_HIP(hipStreamSynchronize(batch_stream), err);
+    for (MsnnSlot& sl : slots) {
+      HM_HIP(hipStreamSynchronize(sl.st), err);
+      sl.used = false;
+    }
+    for (TrainBatch& b : tb) b.used = false;
+    for (WarmBuf& b : warm) b.used = false;
+    mlp_destroy(mlp);
+    mlp = nullptr;
+    train_steps = frame = gen_id = next_slot = batches_made = call_end = 0;
+    loss_last = 0.0;
+    return kOk;
   }
   uint64_t next_u64() {
     uint64_t z = (rng_state += 0x9E3779B97F4A7C15ull);
@@ -303,42 +365,18 @@ int ensure_scene_points(Context& c, uint64_t seed, std::string& err) {
   return kOk;
 }
 
-int msnn_setup(Context& c, int BETA, std::string& err) {
-  if (!c.scene.has_hair) {
-    err = "HairMSNN needs hair geometry";
-    return kEInval;
-  }
-  msnn_release(c.msnn);
-  c.msnn = nullptr;
-  MsnnState* m = new MsnnState();
-  c.msnn = m;
-  const Scene& s = c.scene;
-  m->BETA = BETA;
-  m->kbeta = BETA - 1;  // render_hair_msnn.cu:1170
-  m->n_train = std::max(128, s.msnn_train_records / 128 * 128);
-  const int npx = s.width * s.height;
-  m->every_nth = std::max(1, npx / m->n_train);  // render_hair_msnn.cu:106 (integer division)
-  m->grid_w = 1;
-  while (m->grid_w * m->grid_w < m->n_train) m->grid_w <<= 1;
-  m->lr = s.msnn_lr;
-  m->loss = s.msnn_loss == "RelativeL2" ? HMSNN_LOSS_RELATIVE_L2
-            : s.msnn_loss == "L2"        ? HMSNN_LOSS_L2
-                                         : HMSNN_LOSS_RELATIVE_L2_LUMINANCE;
-  m->rng_state = s.msnn_seed * 0x2545F4914F6CDD1Dull + 1;
-  const int prec = s.msnn_precision == "bf16" ? HMSNN_BF16 : s.msnn_precision == "fp8" ? HMSNN_FP8 : HMSNN_FP16;
-  HM_TRY(mlp_create(prec, s.msnn_seed, &m->mlp, err));
-  // tcnn.init_weights (scene.cpp:330-331 -> render_hair_msnn.cu:109-110)
-  if (!s.nrc_weights.empty()) HM_TRY(mlp_load(*m->mlp, scene_path(s, s.nrc_weights), err));
-  m->ctx_stream = c.stream;
+// The run's buffers, streams and events (m.n_train and m.npx are set).
+int msnn_alloc(Context& c, MsnnState& m, std::string& err) {
+  const int npx = m.npx;
   const int spill_levels = c.stack_levels();
   // a warm-up pass holds warm_batch training batches; the slots' path buffers
   // hold a frame or one such pass
-  m->warm_batch = std::max(1, std::min(MsnnState::kWarmBatch, std::max(npx, m->n_train) / m->n_train));
-  const size_t rec = (size_t)m->warm_batch * m->n_train;
-  m->slot_paths = (int)std::max((size_t)npx, rec);
-  HM_HIP(hipHostMalloc((void**)&m->job_status, sizeof(long long) * 4), err);
-  for (hipEvent_t& e : m->job_ev) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
-  for (MsnnSlot& sl : m->slots) {
+  m.warm_batch = std::max(1, std::min(MsnnState::kWarmBatch, std::max(npx, m.n_train) / m.n_train));
+  const size_t rec = (size_t)m.warm_batch * m.n_train;
+  m.slot_paths = (int)std::max((size_t)npx, rec);
+  HM_HIP(hipHostMalloc((void**)&m.job_status, sizeof(long long) * 4), err);
+  for (hipEvent_t& e : m.job_ev) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
+  for (MsnnSlot& sl : m.slots) {
     HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
     for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
       HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
@@ -355,11 +393,11 @@ int msnn_setup(Context& c, int BETA, std::string& err) {
     HM_TRY(A((void**)&sl.train_input, sizeof(float) * 12 * rec));
     HM_TRY(A((void**)&sl.train_target, sizeof(float) * 3 * rec));
     HM_TRY(A((void**)&sl.train_hit, rec));
-    HM_TRY(A((void**)&sl.train_idx, sizeof(int) * (size_t)m->n_train));
+    HM_TRY(A((void**)&sl.train_idx, sizeof(int) * (size_t)m.n_train));
     HM_TRY(A((void**)&sl.gen_points, sizeof(float) * 3 * rec));
-    HM_HIP(hipHostMalloc((void**)&sl.idx_host, sizeof(int) * (size_t)m->n_train), err);
+    HM_HIP(hipHostMalloc((void**)&sl.idx_host, sizeof(int) * (size_t)m.n_train), err);
   }
-  for (TrainBatch& b : m->tb) {
+  for (TrainBatch& b : m.tb) {
     for (hipEvent_t* e : {&b.ev_ready, &b.ev_free, &b.ev_copy})
       HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
     HM_TRY(alloc_path_buffers(b.pb, b.allocs, rec, true, spill_levels, c.trace_blocks * kTraceBlock, c.stream, err));
@@ -377,16 +415,56 @@ int msnn_setup(Context& c, int BETA, std::string& err) {
     HM_TRY(A((void**)&b.full, sizeof(float4) * rec));
     HM_HIP(hipHostMalloc((void**)&b.idx_host, sizeof(int) * rec), err);
   }
-  HM_TRY(dev_alloc((void**)&m->nn_output, sizeof(float) * 3 * (size_t)npx, err));
+  HM_TRY(dev_alloc((void**)&m.nn_output, sizeof(float) * 3 * (size_t)npx, err));
   for (int k = 0; k < 3; ++k) {
-    HM_TRY(dev_alloc((void**)&m->acc[k], sizeof(float4) * (size_t)npx, err));
-    HM_TRY(dev_alloc((void**)&m->avg[k], sizeof(float4) * (size_t)npx, err));
-    HM_HIP(hipMemsetAsync(m->avg[k], 0, sizeof(float4) * (size_t)npx, c.stream), err);
+    HM_TRY(dev_alloc((void**)&m.acc[k], sizeof(float4) * (size_t)npx, err));
+    HM_TRY(dev_alloc((void**)&m.avg[k], sizeof(float4) * (size_t)npx, err));
   }
+  return kOk;
+}
+
+int msnn_setup(Context& c, int BETA, std::string& err) {
+  if (!c.scene.has_hair) {
+    err = "HairMSNN needs hair geometry";
+    return kEInval;
+  }
+  const Scene& s = c.scene;
+  const int npx = s.width * s.height;
+  const int n_train = std::max(128, s.msnn_train_records / 128 * 128);
+  MsnnState* m = c.msnn;
+  const bool fresh = !m || !m->ready || m->n_train != n_train || m->npx != npx;
+  if (fresh) {
+    msnn_release(m);
+    c.msnn = nullptr;
+    m = c.msnn = new MsnnState();
+  } else {
+    HM_TRY(m->restart(err));
+  }
+  m->ready = false;
+  m->BETA = BETA;
+  m->kbeta = BETA - 1;  // render_hair_msnn.cu:1170
+  m->n_train = n_train;
+  m->npx = npx;
+  m->every_nth = std::max(1, npx / m->n_train);  // render_hair_msnn.cu:106 (integer division)
+  m->grid_w = 1;
+  while (m->grid_w * m->grid_w < m->n_train) m->grid_w <<= 1;
+  m->lr = s.msnn_lr;
+  m->loss = s.msnn_loss == "RelativeL2" ? HMSNN_LOSS_RELATIVE_L2
+            : s.msnn_loss == "L2"        ? HMSNN_LOSS_L2
+                                         : HMSNN_LOSS_RELATIVE_L2_LUMINANCE;
+  m->rng_state = s.msnn_seed * 0x2545F4914F6CDD1Dull + 1;
+  const int prec = s.msnn_precision == "bf16" ? HMSNN_BF16 : s.msnn_precision == "fp8" ? HMSNN_FP8 : HMSNN_FP16;
+  HM_TRY(mlp_create(prec, s.msnn_seed, &m->mlp, err));
+  // tcnn.init_weights (scene.cpp:330-331 -> render_hair_msnn.cu:109-110)
+  if (!s.nrc_weights.empty()) HM_TRY(mlp_load(*m->mlp, scene_path(s, s.nrc_weights), err));
+  m->ctx_stream = c.stream;
+  if (fresh) HM_TRY(msnn_alloc(c, *m, err));
+  for (int k = 0; k < 3; ++k) HM_HIP(hipMemsetAsync(m->avg[k], 0, sizeof(float4) * (size_t)npx, c.stream), err);
   // the slots' first passes start after the set-up work on the context stream
   HM_HIP(hipStreamSynchronize(c.stream), err);
   for (MsnnSlot& sl : m->slots) HM_HIP(hipStreamSynchronize(sl.st), err);
   HM_TRY(ensure_scene_points(c, s.msnn_seed, err));
+  m->ready = true;
   return kOk;
 }
 
@@ -496,82 +574,46 @@ int msnn_warmup_jobs(Context& c, MsnnState& m, int steps, std::string& err) {
   if (steps <= 0) return kOk;
   const int per = std::min(steps, kWarmJobSteps);
   const size_t rec = (size_t)per * m.n_train;
-  struct Buf {
-    float* pts = nullptr;
-    float* input = nullptr;
-    float* target = nullptr;
-    uint8_t* hit = nullptr;
-    float4* L = nullptr;
-    float4* Ls = nullptr;
-    hipEvent_t ev_free = nullptr;
-    bool used = false;
-  } buf[2];
-  std::vector<void*> allocs;
-  auto release = [&]() {
-    (void)hipStreamSynchronize(c.stream);
-    for (void* p : allocs) dev_free(p);
-    for (Buf& b : buf)
-      if (b.ev_free) (void)hipEventDestroy(b.ev_free);
-  };
-  auto body = [&]() -> int {
-    const int nbuf = steps > per ? 2 : 1;
-    for (int k = 0; k < nbuf; ++k) {
-      Buf& b = buf[k];
-      auto A = [&](void** p, size_t bytes) -> int {
-        HM_TRY(dev_alloc(p, bytes, err));
-        allocs.push_back(*p);
-        return kOk;
-      };
-      HM_TRY(A((void**)&b.pts, sizeof(float) * 3 * rec));
-      HM_TRY(A((void**)&b.input, sizeof(float) * 12 * rec));
-      HM_TRY(A((void**)&b.target, sizeof(float) * 3 * rec));
-      HM_TRY(A((void**)&b.hit, rec));
-      HM_TRY(A((void**)&b.L, sizeof(float4) * rec));
-      HM_TRY(A((void**)&b.Ls, sizeof(float4) * rec));
-      HM_HIP(hipEventCreateWithFlags(&b.ev_free, hipEventDisableTiming), err);
-    }
-    const SceneView sc = c.view_no_caps();
-    for (int k = 0, r = 0; k < steps; ++r) {
-      const int nb = std::min(per, steps - k);
-      const int n = nb * m.n_train;
-      Buf& b = buf[r % 2];
-      MsnnSlot& sl = m.take_slot();
-      HM_TRY(acquire_slot(sl, err));
-      if (b.used) HM_HIP(hipStreamWaitEvent(sl.st, b.ev_free, 0), err);
-      b.used = true;
-      HM_TRY(sample_gen_points(c, m, sl.st, b.pts, nb, err));
-      PassConfig cfg = msnn_pass_config(c, m);
-      cfg.camera_mode = 1;
-      cfg.n_slots = n;
-      cfg.chunk = m.n_train;
-      cfg.grid_w = m.grid_w;
-      cfg.points = b.pts;
-      cfg.accum_id = m.gen_id;
-      m.gen_id += nb;
-      cfg.gb.enabled = 1;
-      cfg.gb.nn_input = b.input;
-      cfg.gb.hit_flags = b.hit;
-      cfg.gb.scene_scale = c.scene_scale;
-      JobRun run;
-      HM_TRY(pt_jobs_start(sc, sl.pb, cfg, std::min(n, m.slot_paths), run, sl.st, err));
-      HM_TRY(pt_jobs_drain(sc, sl.pb, cfg, run, b.L, b.Ls, m.job_status, m.job_ev, sl.st, err));
-      hipLaunchKernelGGL(k_msnn_finalize, dim3((n + 255) / 256), dim3(256), 0, sl.st, b.L, b.Ls,
-                         (const uint32_t*)nullptr, n, 1, 1, n, b.input, b.hit, b.input, b.target, (float4*)nullptr);
-      HM_TRY(check_launch("msnn finalize (warm-up)", err));
-      HM_HIP(hipEventRecord(sl.ev_gb, sl.st), err);
-      HM_HIP(hipStreamWaitEvent(c.stream, sl.ev_gb, 0), err);
-      for (int j = 0; j < nb; ++j)
-        HM_TRY(train_step(c, m, b.input + 12 * (size_t)j * m.n_train, b.target + 3 * (size_t)j * m.n_train, err,
-                          nullptr));
-      HM_HIP(hipEventRecord(b.ev_free, c.stream), err);
-      HM_HIP(hipEventRecord(sl.ev_done, c.stream), err);
-      k += nb;
-    }
-    return kOk;
-  };
-  const int rc = body();
-  release();
-  return rc;
+  const int nbuf = steps > per ? 2 : 1;
+  for (int k = 0; k < nbuf; ++k) HM_TRY(m.warm[k].ensure(rec, err));
+  const SceneView sc = c.view_no_caps();
+  for (int k = 0, r = 0; k < steps; ++r) {
+    const int nb = std::min(per, steps - k);
+    const int n = nb * m.n_train;
+    WarmBuf& b = m.warm[r % 2];
+    MsnnSlot& sl = m.take_slot();
+    HM_TRY(acquire_slot(sl, err));
+    if (b.used) HM_HIP(hipStreamWaitEvent(sl.st, b.ev_free, 0), err);
+    b.used = true;
+    HM_TRY(sample_gen_points(c, m, sl.st, b.pts, nb, err));
+    PassConfig cfg = msnn_pass_config(c, m);
+    cfg.camera_mode = 1;
+    cfg.n_slots = n;
+    cfg.chunk = m.n_train;
+    cfg.grid_w = m.grid_w;
+    cfg.points = b.pts;
+    cfg.accum_id = m.gen_id;
+    m.gen_id += nb;
+    cfg.gb.enabled = 1;
+    cfg.gb.nn_input = b.input;
+    cfg.gb.hit_flags = b.hit;
+    cfg.gb.scene_scale = c.scene_scale;
+    JobRun run;
+    HM_TRY(pt_jobs_start(sc, sl.pb, cfg, std::min(n, m.slot_paths), run, sl.st, err));
+    HM_TRY(pt_jobs_drain(sc, sl.pb, cfg, run, b.L, b.Ls, m.job_status, m.job_ev, sl.st, err));
+    hipLaunchKernelGGL(k_msnn_finalize, dim3((n + 255) / 256), dim3(256), 0, sl.st, b.L, b.Ls,
+                       (const uint32_t*)nullptr, n, 1, 1, n, b.input, b.hit, b.input, b.target, (float4*)nullptr);
+    HM_TRY(check_launch("msnn finalize (warm-up)", err));
+    HM_HIP(hipEventRecord(sl.ev_gb, sl.st), err);
+    HM_HIP(hipStreamWaitEvent(c.stream, sl.ev_gb, 0), err);
+    for (int j = 0; j < nb; ++j)
+      HM_TRY(train_step(c, m, b.input + 12 * (size_t)j * m.n_train, b.target + 3 * (size_t)j * m.n_train, err,
+                        nullptr));
+    HM_HIP(hipEventRecord(b.ev_free, c.stream), err);
+    HM_HIP(hipEventRecord(sl.ev_done, c.stream), err);
+    k += nb;
+  }
+  return kOk;
 }
 
 int msnn_warmup(Context& c, MsnnState& m, int steps, std::string& err) {
@@ -748,7 +790,7 @@ int hmsnn_msnn_begin(hmsnn_ctx* ctx, int BETA) {
 int hmsnn_msnn_frames(hmsnn_ctx* ctx, int frames, hmsnn_msnn_stats* stats) {
   if (!ctx || frames < 0) return fail(HMSNN_EINVAL, "hmsnn_msnn_frames: bad arguments");
   Context& c = ctx->c;
-  if (!c.msnn) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
+  if (!c.msnn || !c.msnn->ready) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
   std::string err;
   std::vector<EventTimer> timers(stats ? (size_t)frames : 0);
   c.msnn->call_end = c.msnn->frame + frames;
@@ -784,7 +826,7 @@ int hmsnn_msnn_frames(hmsnn_ctx* ctx, int frames, hmsnn_msnn_stats* stats) {
 int hmsnn_msnn_save_weights(hmsnn_ctx* ctx, const char* path) {
   if (!ctx || !path) return fail(HMSNN_EINVAL, "hmsnn_msnn_save_weights: bad arguments");
   Context& c = ctx->c;
-  if (!c.msnn) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
+  if (!c.msnn || !c.msnn->ready) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
   std::string err;
   int rc = hipStreamSynchronize(c.stream) == hipSuccess ? kOk : kEDevice;
   if (rc) err = "hmsnn_msnn_save_weights: device error";

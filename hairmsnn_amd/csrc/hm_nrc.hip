@@ -61,8 +61,12 @@ struct NrcSlot {
   }
 };
 
+// The buffers and streams stay with the context from one hmsnn_nrc_begin to
+// the next (allocating and freeing them took 47 ms of a begin at 512 x 512,
+// twice the 8 frames that followed); everything a run computes starts over.
 struct NrcState {
   MlpState* mlp = nullptr;
+  bool ready = false;  // fully built (a failed setup is not reused)
   int n_rec = 0;       // training records per step (numTrainingRecords)
   int n_tpx = 0;       // training pixels (numTrainingPixels)
   int every_nth = 1;
@@ -96,6 +100,19 @@ struct NrcState {
     for (NrcSlot& sl : slots) sl.release();
     for (void* p : allocs) dev_free(p);
     if (mlp) mlp_destroy(mlp);
+  }
+  // Waits for the last run's work and forgets its results; the buffers stay.
+  int restart(std::string& err) {
+    HM_HIP(hipStreamSynchronize(ctx_stream), err);
+    for (NrcSlot& sl : slots) {
+      HM_HIP(hipStreamSynchronize(sl.st), err);
+      sl.used = false;
+    }
+    mlp_destroy(mlp);
+    mlp = nullptr;
+    train_steps = frame = next_slot = 0;
+    last_slot = -1;
+    return kOk;
   }
   uint64_t next_u64() {
     uint64_t z = (rng_state += 0x9E3779B97F4A7C15ull);
@@ -222,15 +239,63 @@ float nrc_lr_at(float base, int step) {
   return base * std::pow(0.33f, (float)((step - 4000) / 4000 + 1));
 }
 
+// The run's buffers, streams and events (the sizes in m are set).
+int nrc_alloc(Context& c, NrcState& m, std::string& err) {
+  const int npx = m.frame_size;
+  auto A = [&](void** p, size_t bytes) -> int {
+    HM_TRY(dev_alloc(p, bytes, err));
+    m.allocs.push_back(*p);
+    return kOk;
+  };
+  const size_t nv = (size_t)m.n_tpx * kNrcMaxBounces;
+  for (NrcSlot& sl : m.slots) {
+    HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
+    for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
+      HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
+    HM_TRY(alloc_path_buffers(sl.pb, sl.allocs, (size_t)npx, true, c.stack_levels(), c.trace_blocks * kTraceBlock,
+                              sl.st, err));
+    auto S = [&](void** p, size_t bytes) -> int {
+      HM_TRY(dev_alloc(p, bytes, err));
+      sl.allocs.push_back(*p);
+      return kOk;
+    };
+    HM_TRY(S((void**)&sl.train_idx, sizeof(int) * (size_t)m.n_tpx));
+    HM_TRY(S((void**)&sl.query, sizeof(float) * kNnInputCh * (size_t)m.n_query));
+    HM_TRY(S((void**)&sl.gb_beta, sizeof(float4) * (size_t)npx));
+    HM_TRY(S((void**)&sl.gb_hit, (size_t)npx));
+    HM_TRY(S((void**)&sl.state, sizeof(float4) * (size_t)npx));
+    HM_TRY(S((void**)&sl.prev, sizeof(float4) * (size_t)npx));
+    for (float4*& t : sl.tb) HM_TRY(S((void**)&t, sizeof(float4) * nv));
+    HM_TRY(S((void**)&sl.tb_bounces, sizeof(int) * (size_t)m.n_tpx));
+    HM_TRY(S((void**)&sl.tb_hit, (size_t)m.n_tpx));
+    HM_HIP(hipHostMalloc((void**)&sl.idx_host, sizeof(int) * (size_t)m.n_tpx), err);
+  }
+  HM_TRY(A((void**)&m.cache, sizeof(float) * 3 * (size_t)m.n_query));
+  HM_TRY(A((void**)&m.gb_rad, sizeof(float4) * (size_t)npx));
+  HM_TRY(A((void**)&m.train_in, sizeof(float) * kNnInputCh * (size_t)m.n_rec));
+  HM_TRY(A((void**)&m.train_tgt, sizeof(float) * 3 * (size_t)m.n_rec));
+  HM_TRY(A((void**)&m.acc, sizeof(float4) * (size_t)npx));
+  HM_TRY(A((void**)&m.avg, sizeof(float4) * (size_t)npx));
+  HM_TRY(A((void**)&m.counts_dev, sizeof(int) * 4));
+  return kOk;
+}
+
 int nrc_setup(Context& c, std::string& err) {
-  nrc_release(c.nrc);
-  c.nrc = nullptr;
-  NrcState* m = new NrcState();
-  c.nrc = m;
   const Scene& s = c.scene;
   const int npx = s.width * s.height;
+  const int n_rec = std::max(128, s.nrc_train_records / 128 * 128);
+  NrcState* m = c.nrc;
+  const bool fresh = !m || !m->ready || m->frame_size != npx || m->n_rec != n_rec;
+  if (fresh) {
+    nrc_release(m);
+    c.nrc = nullptr;
+    m = c.nrc = new NrcState();
+  } else {
+    HM_TRY(m->restart(err));
+  }
+  m->ready = false;
   m->frame_size = npx;
-  m->n_rec = std::max(128, s.nrc_train_records / 128 * 128);
+  m->n_rec = n_rec;
   // render_nrc.cu:130-146, integer divisions as in the reference
   m->n_tpx = std::max(1, m->n_rec / kNrcMaxBounces);
   m->every_nth = std::max(1, npx / m->n_tpx);
@@ -247,47 +312,14 @@ int nrc_setup(Context& c, std::string& err) {
   // tcnn.init_weights (scene.cpp:330-331 -> render_nrc.cu:149-150)
   if (!s.nrc_weights.empty()) HM_TRY(mlp_load(*m->mlp, scene_path(s, s.nrc_weights), err));
   m->ctx_stream = c.stream;
-  auto A = [&](void** p, size_t bytes) -> int {
-    HM_TRY(dev_alloc(p, bytes, err));
-    m->allocs.push_back(*p);
-    return kOk;
-  };
-  const size_t nv = (size_t)m->n_tpx * kNrcMaxBounces;
-  for (NrcSlot& sl : m->slots) {
-    HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
-    for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
-      HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
-    HM_TRY(alloc_path_buffers(sl.pb, sl.allocs, (size_t)npx, true, c.stack_levels(), c.trace_blocks * kTraceBlock,
-                              sl.st, err));
-    auto S = [&](void** p, size_t bytes) -> int {
-      HM_TRY(dev_alloc(p, bytes, err));
-      sl.allocs.push_back(*p);
-      return kOk;
-    };
-    HM_TRY(S((void**)&sl.train_idx, sizeof(int) * (size_t)m->n_tpx));
-    HM_TRY(S((void**)&sl.query, sizeof(float) * kNnInputCh * (size_t)m->n_query));
-    HM_TRY(S((void**)&sl.gb_beta, sizeof(float4) * (size_t)npx));
-    HM_TRY(S((void**)&sl.gb_hit, (size_t)npx));
-    HM_TRY(S((void**)&sl.state, sizeof(float4) * (size_t)npx));
-    HM_TRY(S((void**)&sl.prev, sizeof(float4) * (size_t)npx));
-    for (float4*& t : sl.tb) HM_TRY(S((void**)&t, sizeof(float4) * nv));
-    HM_TRY(S((void**)&sl.tb_bounces, sizeof(int) * (size_t)m->n_tpx));
-    HM_TRY(S((void**)&sl.tb_hit, (size_t)m->n_tpx));
-    HM_HIP(hipHostMalloc((void**)&sl.idx_host, sizeof(int) * (size_t)m->n_tpx), err);
-  }
-  HM_TRY(A((void**)&m->cache, sizeof(float) * 3 * (size_t)m->n_query));
-  HM_TRY(A((void**)&m->gb_rad, sizeof(float4) * (size_t)npx));
-  HM_TRY(A((void**)&m->train_in, sizeof(float) * kNnInputCh * (size_t)m->n_rec));
-  HM_TRY(A((void**)&m->train_tgt, sizeof(float) * 3 * (size_t)m->n_rec));
-  HM_TRY(A((void**)&m->acc, sizeof(float4) * (size_t)npx));
-  HM_TRY(A((void**)&m->avg, sizeof(float4) * (size_t)npx));
-  HM_TRY(A((void**)&m->counts_dev, sizeof(int) * 4));
+  if (fresh) HM_TRY(nrc_alloc(c, *m, err));
   HM_HIP(hipMemsetAsync(m->avg, 0, sizeof(float4) * (size_t)npx, c.stream), err);
   m->idx.resize(m->n_tpx);
   for (int i = 0; i < m->n_tpx; ++i) m->idx[i] = i;  // thrust::sequence (render_nrc.cu:170-173)
   // the slots' first passes start after the set-up work
   HM_HIP(hipStreamSynchronize(c.stream), err);
   for (NrcSlot& sl : m->slots) HM_HIP(hipStreamSynchronize(sl.st), err);
+  m->ready = true;
   return kOk;
 }
 
@@ -415,7 +447,7 @@ int hmsnn_nrc_set_params(hmsnn_ctx* ctx, float c_spread, int all_unbiased) {
 int hmsnn_nrc_frames(hmsnn_ctx* ctx, int frames, hmsnn_nrc_stats* stats) {
   if (!ctx || frames < 0) return fail(HMSNN_EINVAL, "hmsnn_nrc_frames: bad arguments");
   Context& c = ctx->c;
-  if (!c.nrc) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
+  if (!c.nrc || !c.nrc->ready) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
   std::string err;
   std::vector<NrcTimer> timers(stats ? (size_t)frames : 0);
   const auto t0 = std::chrono::steady_clock::now();
@@ -498,7 +530,7 @@ int hmsnn_nrc_get_buffer(hmsnn_ctx* ctx, int which, void* host, size_t bytes) {
 
 int hmsnn_nrc_get_mlp_weights(hmsnn_ctx* ctx, float* w_host, int n) {
   if (!ctx || !w_host || n != kMlpWeightCount) return fail(HMSNN_EINVAL, "hmsnn_nrc_get_mlp_weights: bad arguments");
-  if (!ctx->c.nrc) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
+  if (!ctx->c.nrc || !ctx->c.nrc->ready) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
   std::string err;
   if (hipStreamSynchronize(ctx->c.stream) != hipSuccess) return fail(HMSNN_EDEVICE, "stream failed");
   int rc = mlp_get_weights(*ctx->c.nrc->mlp, w_host, err);
@@ -507,7 +539,7 @@ int hmsnn_nrc_get_mlp_weights(hmsnn_ctx* ctx, float* w_host, int n) {
 
 int hmsnn_nrc_save_weights(hmsnn_ctx* ctx, const char* path) {
   if (!ctx || !path) return fail(HMSNN_EINVAL, "hmsnn_nrc_save_weights: bad arguments");
-  if (!ctx->c.nrc) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
+  if (!ctx->c.nrc || !ctx->c.nrc->ready) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
   std::string err;
   if (hipStreamSynchronize(ctx->c.stream) != hipSuccess) return fail(HMSNN_EDEVICE, "stream failed");
   int rc = mlp_save(*ctx->c.nrc->mlp, path, err);
@@ -516,7 +548,7 @@ int hmsnn_nrc_save_weights(hmsnn_ctx* ctx, const char* path) {
 
 int hmsnn_nrc_set_mlp_weights(hmsnn_ctx* ctx, const float* w_host, int n) {
   if (!ctx || !w_host || n != kMlpWeightCount) return fail(HMSNN_EINVAL, "hmsnn_nrc_set_mlp_weights: bad arguments");
-  if (!ctx->c.nrc) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
+  if (!ctx->c.nrc || !ctx->c.nrc->ready) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
   std::string err;
   if (hipStreamSynchronize(ctx->c.stream) != hipSuccess) return fail(HMSNN_EDEVICE, "stream failed");
   int rc = mlp_set_weights(*ctx->c.nrc->mlp, w_host, err);

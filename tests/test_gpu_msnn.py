@@ -327,3 +327,15 @@ def test_training_pixel_shuffles(gpu):
     b, _, _ = residues(4)
     for x, y in zip(a, b):
         np.testing.assert_array_equal(x, y)
+
+
+def test_second_run_on_a_scene_equals_the_first(gpu):
+    """hmsnn_msnn_begin keeps the buffers of an earlier run on the same scene:
+    a second render, after one with another BETA and more frames than a
+    training batch holds, is the first one bit for bit."""
+    cfg = cfg_small(records=1024, warmup=40)
+    with gpu.Scene(json_text=cfg) as sc:
+        a = sc.render_hair_msnn(1, 11)
+        sc.render_hair_msnn(3, 5)
+        b = sc.render_hair_msnn(1, 11)
+    np.testing.assert_array_equal(a, b)

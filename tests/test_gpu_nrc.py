@@ -147,3 +147,19 @@ def test_render_composite_and_frame_stats(gpu):
     assert st["frames"] == 1 and st["train_steps"] == 1 and st8["train_steps"] == 9
     assert st["cache_queries"] > 0 and st["train_records_used"] > 0
     assert np.isfinite(img9).all()
+
+
+def test_second_run_on_a_scene_equals_the_first(gpu):
+    """hmsnn_nrc_begin keeps the buffers of an earlier run on the same scene:
+    image and trained weights of a second run, after one with other
+    parameters, are the first one's bit for bit."""
+    out = []
+    with gpu.Scene(json_text=cfg_small()) as sc:
+        for c in (None, 0.5, None):
+            sc.nrc_begin()
+            if c is not None:
+                sc.nrc_set_params(c, True)
+            sc.nrc_frames(7)
+            out.append((sc.nrc_image(), sc.nrc_weights()))
+    np.testing.assert_array_equal(out[0][0], out[2][0])
+    np.testing.assert_array_equal(out[0][1], out[2][1])
