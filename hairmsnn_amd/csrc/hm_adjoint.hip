@@ -1,11 +1,14 @@
-// Path-replay adjoint of the path tracer for differentiable hair appearance:
-// gradients of L(mean image) w.r.t. per-strand sigma_a and global beta_m,
-// beta_n, alpha, given dL/d(image).
+// Adjoint of the path tracer for differentiable hair appearance: gradients of
+// L(mean image) w.r.t. per-strand sigma_a and global beta_m, beta_n, alpha,
+// given dL/d(image).
 //
-// Each (pixel, pass) path is traced twice from the same seed (the reference's
-// per-pixel streams, cuda/path_tracing.cu:29): a primal pass that sums the
-// path's radiance, then a replay that differentiates every factor that
-// depends on the parameters at each hair vertex, with adj = dL/dI / spp:
+// The wavefront tracer renders the paths of up to 16 passes (the reference's
+// per-pixel streams, cuda/path_tracing.cu:29) into its radiance ring and
+// records every hair vertex on a tape: ray, hit, throughput, random state,
+// radiance gathered before it and the visibility of its two light samples, 81
+// bytes. The vertices are then independent: one thread per record evaluates
+// the vertex again from its random state and differentiates every factor that
+// depends on the parameters, with adj = dL/dI / spp:
 //   direct-lighting sample k:  c_k = f_k * w_k * (parameter-free factor), so
 //     dc_k = (c_k / f_k) * df_k + c_k * dw_k / w_k, where w_k is the
 //     power-heuristic MIS weight through the BSDF pdf (1 for delta lights);
@@ -13,8 +16,12 @@
 //     proportional to f, so it contributes rem * df / f.
 // Sampled directions, the sampling pdfs in the estimators' denominators and
 // Russian roulette are held fixed (detached): the estimator stays unbiased
-// for the derivative of the expected image without storing a tape.
+// for the derivative of the expected image.
 // Per-strand gradients are reduced with FP64 atomics.
+//
+// Tracing the paths once more instead of taping them (one lane per path, all
+// its rays included) took 39 ms of a 73 ms step at 512 x 512, 16 passes, 3.2 M
+// segments. The tape is sequential memory, 2 GB there, on a GPU of 288 GB.
 #include <hip/hip_runtime.h>
 
 #include "../../include/hmsnn.h"
@@ -30,14 +37,11 @@ struct AdjArgs {
   HairConstsAD hcd;
   const float4* dl_dimg;  // w*h
   float inv_spp;
-  int pass0, npass;
   int dl_zero, dl_from, max_vertex;
-  const float4* ring;  // primal radiance of pass pass0 + p at ring[p * npx + pixel]
+  const float4* ring;  // primal radiance of pass p of the run at ring[p * npx + pixel]
   double* g_sigma;  // num_strands * 3
   double* g_glob;   // 3
   float* g_px;      // optional: w*h*3 per-pixel d/d(beta_m, beta_n, alpha)
-  int* spill;
-  int spill_stride, spill_levels;
 };
 
 HM_D int strand_of(const SceneView& sc, int prim) { return (int)sc.seg_by_id[8 * (size_t)prim + 7]; }
@@ -73,176 +77,97 @@ HM_D V3 safe_ratio(V3 c, V3 f) {
   return v3(f.x != 0.f ? c.x / f.x : 0.f, f.y != 0.f ? c.y / f.y : 0.f, f.z != 0.f ? c.z / f.z : 0.f);
 }
 
-// A replayed path between vertices: the ray to trace next and what the
-// vertices so far left (the operations and random draws are those of
-// k_camera / k_shade / k_shadow for the path's seed).
-struct AdjPath {
-  uint32_t rng;
-  V3 o, d;      // the ray to trace next
-  V3 beta, L;   // throughput and radiance gathered so far
-  V3 Lt, adj;   // the path's primal radiance and dLoss/dI / spp
-  int depth;    // the vertex the next hit is
-  int pix;
-  float gp[3];  // the path's global gradient
-};
-
-// The camera ray of pixel (x, y) in pass `pass` (path_tracing.cu:29-48).
-HM_D void adj_start(const SceneView& sc, int x, int y, int pass, AdjPath& q) {
-  q.rng = path_seed((uint32_t)(pass + 10007), (uint32_t)x, (uint32_t)y, (uint32_t)sc.width);
-  const float jx = draw(q.rng), jy = draw(q.rng);
-  const float sx = ((float)x + jx) / (float)sc.width, sy = ((float)y + jy) / (float)sc.height;
-  q.d = normalize(sc.cam_d00 + sx * sc.cam_du + sy * sc.cam_dv);
-  q.o = sc.cam_pos;
-  q.beta = v3(1.f);
-  q.L = v3(0.f);
-  q.depth = 0;
-  q.gp[0] = q.gp[1] = q.gp[2] = 0.f;
-}
-
-// The vertex the path's ray hit (t, prim, u): its direct lighting with its
-// two shadow rays, the gradient of every factor there that depends on the
-// parameters, Russian roulette and the continuation. Returns whether the
-// path goes on (q then holds the next ray). Given the path's primal
-// radiance Lt, the continuation's gradient uses the radiance still to come,
-// Lt - L.
-HM_D bool adj_vertex(const SceneView& sc, const AdjArgs& a, TraceStack& st, float t, int prim, float u,
-                     AdjPath& q) {
-  TraceCounters cnt{0, 0, 0};
-  const int depth = q.depth;
+// One taped vertex: the gradient of its direct lighting (shadow rays visible
+// per vis) and of its continuation, which the radiance still to come, Lt - L,
+// is proportional to. The operations and random draws are those the tracer's
+// shading makes from the same random state. gg receives the global part.
+HM_D void adj_vertex(const SceneView& sc, const AdjArgs& a, V3 o, V3 d, float t, int prim, float u, V3 beta,
+                     uint32_t rng, V3 L, V3 Lt, V3 adj, int depth, int vis, float gg[3]) {
   Hit h;
-  setup_hit(sc, q.o, q.d, t, prim, u, h);
-  const bool hair = !h.surface;
+  setup_hit(sc, o, d, t, prim, u, h);
+  const V3 sigma = strand_sigma_of(sc, prim);
   if (depth == 0 ? a.dl_zero != 0 : depth >= a.dl_from) {
     DirectOut dl;
-    direct_lighting(sc, h, q.rng, dl);
-    const bool v1 = dl.has1 && !(sc.curves ? occluded<false, true>(sc, dl.o1, dl.d1, st, cnt)
-                                           : occluded<false>(sc, dl.o1, dl.d1, st, cnt));
-    const bool v2 = dl.has2 && !(sc.curves ? occluded<false, true>(sc, dl.o2, dl.d2, st, cnt)
-                                           : occluded<false>(sc, dl.o2, dl.d2, st, cnt));
+    direct_lighting(sc, h, rng, dl);
+    const bool v1 = dl.has1 && (vis & 1), v2 = dl.has2 && (vis & 2);
     V3 sum = v3(0.f);
     if (v1) sum = sum + dl.c1;
     if (v2) sum = sum + dl.c2;
-    const bool bad = any_nan(sum);
-    if (bad) sum = v3(0.f);
-    if (hair && !bad) {
-      const V3 sigma = strand_sigma_of(sc, prim);
-      const V3 W = q.adj * q.beta;  // dLoss / dc per channel
-      float r[kAdParams];
-      if (v1) {
+    if (any_nan(sum)) {
+      sum = v3(0.f);
+    } else {
+      const V3 W = adj * beta;  // dLoss / dc per channel
+      // one copy of the derivative code for both light samples
+#pragma unroll 1
+      for (int k = 0; k < 2; ++k) {
+        if (!(k ? v2 : v1)) continue;
         Dual f[3], pd;
-        hair_eval_dual(a.hcd, h.wo_local, dl.wl1, h.hw.h, sigma, f, &pd);
-        const float pb = dl.bp1, pl = dl.lp1;
+        hair_eval_dual(a.hcd, h.wo_local, k ? dl.wl2 : dl.wl1, h.hw.h, sigma, f, &pd);
+        const float pb = k ? dl.bp2 : dl.bp1, pl = k ? dl.lp2 : dl.lp1;
+        // d(weight) / weight through the BSDF pdf: of the light sample's weight
+        // pl^2 / (pl^2 + pb^2), of the BSDF sample's pb^2 / (pb^2 + pl^2)
+        float c = 0.f;
+        if (k == 0) c = dl.mis1 ? -2.f * pb / (pl * pl + pb * pb) : 0.f;
+        else c = pb > 0.f ? 2.f * pl * pl / (pb * (pb * pb + pl * pl)) : 0.f;
+        float r[kAdParams];
 #pragma unroll
-        for (int k = 0; k < kAdParams; ++k) r[k] = dl.mis1 ? -2.f * pb * pd.d[k] / (pl * pl + pb * pb) : 0.f;
-        add_grad(sc, a, prim, f, W * safe_ratio(dl.c1, dl.f1), dot(W, dl.c1), r, q.gp);
-      }
-      if (v2) {
-        Dual f[3], pd;
-        hair_eval_dual(a.hcd, h.wo_local, dl.wl2, h.hw.h, sigma, f, &pd);
-        const float pb = dl.bp2, pl = dl.lp2;
-#pragma unroll
-        for (int k = 0; k < kAdParams; ++k) r[k] = pb > 0.f ? 2.f * pl * pl * pd.d[k] / (pb * (pb * pb + pl * pl)) : 0.f;
-        add_grad(sc, a, prim, f, W * safe_ratio(dl.c2, dl.f2), dot(W, dl.c2), r, q.gp);
+        for (int q = 0; q < kAdParams; ++q) r[q] = c * pd.d[q];
+        const V3 cc = k ? dl.c2 : dl.c1;
+        add_grad(sc, a, prim, f, W * safe_ratio(cc, k ? dl.f2 : dl.f1), dot(W, cc), r, gg);
       }
     }
-    q.L = q.L + q.beta * sum;
+    L = L + beta * sum;
   }
   if (depth >= 1) {
-    const float rr = fmaxf(0.05f, 1.f - luminance(q.beta));
-    if (draw(q.rng) < rr) return false;
-    q.beta = q.beta / (1.f - rr);
+    const float rr = fmaxf(0.05f, 1.f - luminance(beta));
+    if (draw(rng) < rr) return;
   }
-  if (depth + 1 > a.max_vertex) return false;
-  const BsdfSample bs = sample_bsdf(sc, h, q.rng);
-  const V3 wl = bs.wl, wi = bs.wi, f = bs.f;
-  const float pdf = bs.pdf;
-  V3 mul = (pdf == 0.f) ? f : f / pdf;
-  const bool mul_bad = any_nan(mul);
-  if (mul_bad) mul = v3(1.f);
-  if (hair && !mul_bad) {
-    const V3 rem = q.Lt - q.L;  // radiance gathered after this vertex
-    Dual fd[3], pd;
-    hair_eval_dual(a.hcd, h.wo_local, wl, h.hw.h, strand_sigma_of(sc, prim), fd, &pd);
-    float r[kAdParams];
+  if (depth + 1 > a.max_vertex) return;
+  const BsdfSample bs = sample_bsdf(sc, h, rng);
+  if (any_nan((bs.pdf == 0.f) ? bs.f : bs.f / bs.pdf)) return;
+  const V3 rem = Lt - L;  // radiance gathered after this vertex
+  Dual fd[3], pd;
+  hair_eval_dual(a.hcd, h.wo_local, bs.wl, h.hw.h, sigma, fd, &pd);
+  float r[kAdParams];
 #pragma unroll
-    for (int k = 0; k < kAdParams; ++k) r[k] = 0.f;
-    add_grad(sc, a, prim, fd, q.adj * safe_ratio(rem, f), 0.f, r, q.gp);
-  }
-  q.beta = q.beta * mul;
-  V3 p = h.p, nd = h.n;
-  if (dot(wi, h.n) < 0.f && hair) {
-    nd = -1.f * h.n;
-    p = p + (2.f * h.radius) * nd;
-  }
-  q.o = p + 1e-3f * nd;
-  q.d = wi;
-  q.depth = depth + 1;
-  return true;
+  for (int k = 0; k < kAdParams; ++k) r[k] = 0.f;
+  add_grad(sc, a, prim, fd, adj * safe_ratio(rem, bs.f), 0.f, r, gg);
 }
 
-// Waves per SIMD the replay kernel is compiled for. At 512x512 C1, 16 spp,
-// with path regeneration the replay ran at 55.4 M paths/s with 2 waves, 59.3
-// with 3, 62-63 with 4, 54.0 with 5 and 49.8 with 6 (the registers beyond
-// the budget spill to scratch: 784 bytes per lane at 4). Without
-// regeneration (each lane's path run to its end while the wave waited for
-// its longest path) the best was 48.3 with 3 waves.
-#ifndef HM_ADJ_MIN_WAVES
-#define HM_ADJ_MIN_WAVES 4
-#endif
-__global__ void __launch_bounds__(kTraceBlock, HM_ADJ_MIN_WAVES) k_adjoint(SceneView sc, AdjArgs a) {
-  __shared__ int lds_stack[kStackLds * kTraceBlock];
-  TraceStack st;
-  st.init(lds_stack, a.spill + blockIdx.x * blockDim.x + threadIdx.x, a.spill_stride, a.spill_levels);
+// Bound by its vector arithmetic (the dual-number evaluations carry six
+// tangents): 3.4 ms for the 13 M records of one of two groups. Two waves per
+// SIMD keep its registers (1, 2, 3 and 4 waves: 42.7, 40.9, 42.4 and 42.2 ms
+// for the whole 512 x 512, 16-pass step).
+__global__ void __launch_bounds__(256, 2) k_adjoint(SceneView sc, AdjArgs a, VertexTape tape,
+                                                                   const long long* count) {
   const int npx = sc.width * sc.height;
-  const long long total = (long long)npx * a.npass;
-  float gg[3] = {0.f, 0.f, 0.f};
+  const long long n = min(*count, tape.cap);
   const long long stride = (long long)gridDim.x * blockDim.x;
-  // Path regeneration: each lane replays its paths i, i + stride, ... one
-  // vertex per iteration, and a lane whose path has ended starts its next
-  // one in the same iteration, so the wave's lanes stay busy instead of
-  // waiting for the longest path of the wave.
-  long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x - stride;
-  bool live = false;
-  AdjPath q;
-  for (;;) {
-    if (!live) {
-      for (i += stride; i < total; i += stride) {
-        const int pix = (int)(i % npx), pass = a.pass0 + (int)(i / npx);
-        const float4 g4 = a.dl_dimg[pix];
-        const V3 adj = a.inv_spp * v3(g4.x, g4.y, g4.z);
-        if (adj.x == 0.f && adj.y == 0.f && adj.z == 0.f) continue;
-        const float4 l = a.ring[i];  // i = (pass - pass0) * npx + pix
-        const V3 Lt = v3(l.x, l.y, l.z);
-        if (any_nan(Lt)) continue;  // writePixel drops NaN samples (utils.cuh:20-21)
-        adj_start(sc, pix % sc.width, pix / sc.width, pass, q);
-        q.adj = adj;
-        q.Lt = Lt;
-        q.pix = pix;
-        live = true;
-        break;
-      }
-    }
-    if (!__any(live)) break;
-    if (!live) continue;
-    float t, u;
-    int prim;
-    TraceCounters cnt{0, 0, 0};
-    if (sc.curves)
-      closest_hit<false, true>(sc, q.o, q.d, st, t, prim, u, cnt);
-    else
-      closest_hit<false>(sc, q.o, q.d, st, t, prim, u, cnt);
-    live = prim != kPrimMiss && adj_vertex(sc, a, st, t, prim, u, q);
-    if (!live) {
+  float gg[3] = {0.f, 0.f, 0.f};
+  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) {
+    const float4 l = tape.L[i];
+    const int prim = __float_as_int(l.w);
+    if (prim < 0) continue;
+    const int4 m = tape.meta[i];
+    const float4 g4 = a.dl_dimg[m.x];
+    const V3 adj = a.inv_spp * v3(g4.x, g4.y, g4.z);
+    if (adj.x == 0.f && adj.y == 0.f && adj.z == 0.f) continue;
+    const float4 lt = a.ring[(size_t)m.y * npx + m.x];
+    const V3 Lt = v3(lt.x, lt.y, lt.z);
+    if (any_nan(Lt)) continue;  // writePixel drops NaN samples (utils.cuh:20-21)
+    const float4 o = tape.o[i], d = tape.d[i], b = tape.beta[i];
+    float gv[3] = {0.f, 0.f, 0.f};
+    adj_vertex(sc, a, v3(o.x, o.y, o.z), v3(d.x, d.y, d.z), o.w, prim, d.w, v3(b.x, b.y, b.z), __float_as_uint(b.w),
+               v3(l.x, l.y, l.z), Lt, adj, m.z, tape.vis[i], gv);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        gg[k] += q.gp[k];
-        if (a.g_px && q.gp[k] != 0.f) atomicAdd(&a.g_px[3 * (size_t)q.pix + k], q.gp[k]);
-      }
+    for (int k = 0; k < 3; ++k) {
+      gg[k] += gv[k];
+      if (a.g_px && gv[k] != 0.f) atomicAdd(&a.g_px[3 * (size_t)m.x + k], gv[k]);
     }
   }
   // the global gradients: wave sums, block sums in LDS, one FP64 atomic per
   // block and parameter
-  __shared__ float part[kTraceBlock / 64][3];
+  __shared__ float part[4][3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     float v = gg[k];
@@ -252,8 +177,85 @@ __global__ void __launch_bounds__(kTraceBlock, HM_ADJ_MIN_WAVES) k_adjoint(Scene
   __syncthreads();
   if (threadIdx.x < 3) {
     double v = 0.0;
-    for (int w = 0; w < kTraceBlock / 64; ++w) v += (double)part[w][threadIdx.x];
+    for (int w = 0; w < 4; ++w) v += (double)part[w][threadIdx.x];
     if (v != 0.0) atomicAdd(&a.g_glob[threadIdx.x], v);
+  }
+}
+
+// Records a path is expected to leave (its hair vertices and its last, missed
+// ray); a run that leaves more is repeated with a larger tape. Passes per run:
+// as many as a tape of kTapeBytes is expected to hold.
+constexpr int kTapePerPath = 10;
+constexpr size_t kTapeBytes = (size_t)8 << 30;
+
+// Makes the context's tape hold at least `records`.
+int tape_ensure(Context& c, long long records, std::string& err) {
+  if (c.tape.cap >= records) return kOk;
+  for (void* p : c.tape_allocs) dev_free(p);
+  c.tape_allocs.clear();
+  c.tape = VertexTape{};
+  const size_t n = (size_t)records;
+  auto A = [&](void** p, size_t bytes) -> int {
+    HM_TRY(dev_alloc(p, bytes, err));
+    c.tape_allocs.push_back(*p);
+    return kOk;
+  };
+  for (float4** p : {&c.tape.o, &c.tape.d, &c.tape.beta, &c.tape.L}) HM_TRY(A((void**)p, sizeof(float4) * n));
+  HM_TRY(A((void**)&c.tape.meta, sizeof(int4) * n));
+  HM_TRY(A((void**)&c.tape.vis, n));
+  c.tape.cap = records;
+  return kOk;
+}
+
+// Group g of K's share of the tape.
+VertexTape tape_share(const VertexTape& t, int g, int K) {
+  VertexTape v = t;
+  v.cap = t.cap / K;
+  const size_t off = (size_t)v.cap * g;
+  v.o += off;
+  v.d += off;
+  v.beta += off;
+  v.L += off;
+  v.meta += off;
+  v.vis += off;
+  return v;
+}
+
+// Passes p0 .. p0 + np - 1 (at most kStreamRing): traced with the tape, then
+// differentiated.
+int adjoint_passes(Context& c, const AdjArgs& a, int p0, int np, float4* tmp_acc, std::string& err) {
+  const size_t npx = (size_t)c.scene.width * c.scene.height;
+  const int K = stream_groups(c, np);
+  long long want = kTapePerPath * (long long)npx * np + 64;
+  for (;;) {
+    const int rc = tape_ensure(c, want, err);
+    if (rc && np > 1) {  // no room: half the passes at a time
+      err.clear();
+      (void)hipGetLastError();
+      HM_TRY(adjoint_passes(c, a, p0, np / 2, tmp_acc, err));
+      return adjoint_passes(c, a, p0 + np / 2, np - np / 2, tmp_acc, err);
+    }
+    HM_TRY(rc);
+    StreamTape st{};
+    for (int g = 0; g < K; ++g) st.tape[g] = tape_share(c.tape, g, K);
+    HM_TRY(stream_passes(c, p0, np, tmp_acc, tmp_acc + npx, nullptr, err, &st));
+    long long count[kStreamGroups] = {};
+    for (int g = 0; g < K; ++g)
+      HM_HIP(hipMemcpyAsync(&count[g], st.count[g], sizeof(long long), hipMemcpyDeviceToHost, c.stream), err);
+    HM_HIP(hipStreamSynchronize(c.stream), err);
+    long long most = 0;
+    for (int g = 0; g < K; ++g) most = std::max(most, count[g]);
+    if (most > st.tape[0].cap) {
+      want = K * (most + most / 8);
+      continue;
+    }
+    AdjArgs x = a;
+    x.ring = c.stream_ring;
+    for (int g = 0; g < K; ++g) {
+      const int blocks = (int)std::min<long long>(c.num_cus * 8ll, std::max<long long>(1, (count[g] + 255) / 256));
+      hipLaunchKernelGGL(k_adjoint, dim3(blocks), dim3(256), 0, c.stream, c.view, x, st.tape[g], st.count[g]);
+    }
+    return check_launch("adjoint", err);
   }
 }
 
@@ -329,25 +331,12 @@ int hmsnn_adjoint_render(hmsnn_ctx* ctx, int spp, const float* dl_dimg, double* 
   a.g_sigma = d_gs;
   a.g_glob = d_gg;
   a.g_px = d_px;
-  a.spill = c.pb.spill;
-  a.spill_stride = c.pb.spill_stride;
-  a.spill_levels = c.pb.spill_levels;
-  // The primal radiance of every path comes from the wavefront path tracer
-  // (the same paths: same seeds, same operations), kStreamRing passes at a
-  // time into the context's radiance ring; the replay kernel then only runs
-  // the adjoint pass over them.
   float4* tmp_acc = nullptr;
   rc = dev_alloc((void**)&tmp_acc, 2 * sizeof(float4) * (size_t)npx, err);
-  for (int p0 = 0; !rc && p0 < spp; p0 += kStreamRing) {
-    const int np = std::min(kStreamRing, spp - p0);
-    rc = stream_passes(c, p0, np, tmp_acc, tmp_acc + npx, nullptr, err);
-    if (rc) break;
-    a.ring = c.stream_ring;
-    a.pass0 = c.seed_offset + p0;
-    a.npass = np;
-    hipLaunchKernelGGL(k_adjoint, dim3(c.trace_blocks), dim3(kTraceBlock), 0, c.stream, c.view, a);
-    rc = check_launch("adjoint", err);
-  }
+  const size_t pass_bytes = (size_t)kTapePerPath * kTapeRecordBytes * npx;
+  const int chunk = (int)std::max<size_t>(1, std::min<size_t>(kStreamRing, kTapeBytes / pass_bytes));
+  for (int p0 = 0; !rc && p0 < spp; p0 += chunk)
+    rc = adjoint_passes(c, a, p0, std::min(chunk, spp - p0), tmp_acc, err);
   (void)hipStreamSynchronize(c.stream);
   dev_free(tmp_acc);
   if (!rc) {

@@ -122,6 +122,7 @@ Context::~Context() {
   if (live_host) (void)hipHostFree(live_host);
   dev_free(stream_ring);
   dev_free(stream_ctl);
+  for (void* p : tape_allocs) dev_free(p);
   msnn_release(msnn);
   msnn = nullptr;
   nrc_release(nrc);
@@ -788,12 +789,17 @@ namespace hm {
 // pixel accumulated into acc / avg (the context's image, or scratch buffers of
 // a caller that only wants the radiance ring); the context stream waits for
 // every group. The ring then holds the last (up to) 16 passes' radiance.
+int stream_groups(const Context& c, int passes) {
+  const long long jobs = (long long)c.scene.width * c.scene.height * passes;
+  return jobs < kTwoGroupJobs ? 1 : std::max(1, std::min(c.num_flights, kStreamGroups));
+}
+
 int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* avg, PassTimer* timer,
-                  std::string& err) {
+                  std::string& err, StreamTape* tape) {
   HM_TRY(c.ensure_path_buffers(false, err));
   const int n = c.scene.width * c.scene.height;
   if (passes <= 0) return kOk;
-  const int K = (long long)n * passes < kTwoGroupJobs ? 1 : std::max(1, std::min(c.num_flights, kStreamGroups));
+  const int K = stream_groups(c, passes);
   HM_TRY(c.ensure_flights(K, err));
   if (!c.live_host) {
     HM_HIP(hipHostMalloc((void**)&c.live_host, 2 * Context::kMaxFlights * sizeof(int)), err);
@@ -819,7 +825,7 @@ int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* a
   cfg.accum_id = first_pass;
   cfg.timer = timer;
   HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, stream_slots(n), acc, avg, c.stream_ring, c.stream_ctl,
-                       c.live_host, c.live_ev, err));
+                       c.live_host, c.live_ev, err, tape));
   // the context stream waits for every group
   for (int g = 1; g < K; ++g) {
     HM_HIP(hipEventRecord(c.acc_event, sts[g]), err);

@@ -101,6 +101,9 @@ struct Context {
   long long* stream_ctl = nullptr;  // streaming schedule: scheduler counters per group
   int last_ring_entry = 0;          // ring entry of the last streamed pass
   hipEvent_t live_ev[2 * kMaxFlights] = {};
+  // vertex tape of the adjoint, grown on demand
+  std::vector<void*> tape_allocs;
+  VertexTape tape{};
   int ensure_flights(int count, std::string& err);
   PathBuffers& flight_pb(int f) { return f == 0 ? pb : extra[f - 1].pb; }
   hipStream_t flight_stream(int f) { return f == 0 ? stream : extra[f - 1].stream; }
@@ -123,7 +126,10 @@ struct Context {
 // Streaming-schedule passes first_pass .. first_pass + passes - 1 into acc /
 // avg; afterwards the context stream is ordered after them and c.stream_ring
 // holds the radiance of the last (up to) kStreamRing passes by pass - first_pass.
+// With a tape, every path vertex is recorded on it.
 int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* avg, PassTimer* timer,
-                  std::string& err);
+                  std::string& err, StreamTape* tape = nullptr);
+// Stream groups of a call of `passes` passes.
+int stream_groups(const Context& c, int passes);
 
 }  // namespace hm

@@ -522,9 +522,11 @@ __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade(SceneView sc,
 // is a HairMSNN training path (full and short throughput, the short one cut
 // after vertex trunc_beta); the primary hit's network input goes to gb at
 // the path's job (slot_px), and the short radiance travels with the path.
-template <bool kMsnn>
+// kTape: hair vertices are also recorded on the tape from record tape_base on.
+template <bool kMsnn, bool kTape = false>
 __device__ __forceinline__ void shade_dense(const SceneView& sc, const PathBuffers& pb, const PathBuffers& nb,
-                                            const ShadeParams& sp, const GBufferOut& gb) {
+                                            const ShadeParams& sp, const GBufferOut& gb,
+                                            const VertexTape& tape = VertexTape{}, long long tape_base = 0) {
   const int n = pb.counts[wave_count(sp.cur)];
   const int stride = gridDim.x * blockDim.x;
   const int nloop = (n + stride - 1) / stride * stride;
@@ -542,6 +544,20 @@ __device__ __forceinline__ void shade_dense(const SceneView& sc, const PathBuffe
       const V3 o = v3(o4.x, o4.y, o4.z), d = v3(d4.x, d4.y, d4.z);
       L = pb.L[i];
       if constexpr (kMsnn) Ls = pb.L_short[i];
+      if constexpr (kTape) {
+        const long long r = tape_base + i;
+        if (r < tape.cap) {
+          tape.L[r] = make_float4(L.x, L.y, L.z, __int_as_float(prim));
+          if (prim >= 0) {
+            const float4 b4 = pb.beta[i];
+            tape.o[r] = make_float4(o4.x, o4.y, o4.z, pb.hit_t[i]);
+            tape.d[r] = make_float4(d4.x, d4.y, d4.z, pb.hit_u[i]);
+            tape.beta[r] = make_float4(b4.x, b4.y, b4.z, __uint_as_float(pb.rng[i]));
+            tape.meta[r] = make_int4(pb.slot_px[i], pb.slot_pass[i], depth, 0);
+            tape.vis[r] = 0;
+          }
+        }
+      }
       if (prim == kPrimMiss) {
         if (depth == 0) {
           // camera ray escaped: the miss program's radiance (optix_common.cuh:604-616)
@@ -643,6 +659,13 @@ __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade_dense(SceneVi
   shade_dense<false>(sc, pb, nb, sp, GBufferOut{});
 }
 
+__global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade_dense_tape(SceneView sc, PathBuffers pb,
+                                                                               PathBuffers nb, ShadeParams sp,
+                                                                               VertexTape tape,
+                                                                               const long long* base) {
+  shade_dense<false, true>(sc, pb, nb, sp, GBufferOut{}, tape, *base);
+}
+
 __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade_dense_msnn(SceneView sc, PathBuffers pb,
                                                                                PathBuffers nb, ShadeParams sp,
                                                                                GBufferOut gb) {
@@ -652,13 +675,21 @@ __global__ void __launch_bounds__(256, HM_SHADE_MIN_WAVES) k_shade_dense_msnn(Sc
 // The resolve of k_shadow_resolve for a compacted wavefront: the visible
 // contributions go to the path where k_shade_dense moved it (kMsnn: the
 // short radiance too).
-template <bool kMsnn>
-__device__ __forceinline__ void shadow_resolve_dense(const PathBuffers& pb, const PathBuffers& nb, int set) {
+// kTape: the visibilities go to the tape.
+template <bool kMsnn, bool kTape = false>
+__device__ __forceinline__ void shadow_resolve_dense(const PathBuffers& pb, const PathBuffers& nb, int set,
+                                                     const VertexTape& tape = VertexTape{}, long long tape_base = 0) {
   const int n = pb.counts[append_count(set, kShadowCount)];
   const int stride = gridDim.x * blockDim.x;
   for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < n; j += stride) {
     const int slot = pb.shadow_queue[j];
     V3 sum = v3(0.f);
+    if constexpr (kTape) {
+      const long long r = tape_base + slot;
+      if (r < tape.cap)
+        tape.vis[r] = (uint8_t)((pb.sh_o1[slot].w != 0.f && pb.sh_vis[2 * slot] ? 1 : 0) |
+                                (pb.sh_o2[slot].w != 0.f && pb.sh_vis[2 * slot + 1] ? 2 : 0));
+    }
     if (pb.sh_o1[slot].w != 0.f && pb.sh_vis[2 * slot]) {
       const float4 c = pb.sh_c1[slot];
       sum = sum + v3(c.x, c.y, c.z);
@@ -690,6 +721,11 @@ __device__ __forceinline__ void shadow_resolve_dense(const PathBuffers& pb, cons
 
 __global__ void k_shadow_resolve_dense(PathBuffers pb, PathBuffers nb, int set) {
   shadow_resolve_dense<false>(pb, nb, set);
+}
+
+__global__ void k_shadow_resolve_dense_tape(PathBuffers pb, PathBuffers nb, int set, VertexTape tape,
+                                            const long long* base) {
+  shadow_resolve_dense<false, true>(pb, nb, set, tape, *base);
 }
 
 __global__ void k_shadow_resolve_dense_msnn(PathBuffers pb, PathBuffers nb, int set) {
@@ -885,7 +921,8 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
 // chunks g, g + K, g + 2K, ... (balanced work, coherent camera rays within a
 // wave).
 // ctl (64-bit, per group): two copies of the scheduler state, each [0] next
-// job, [1] passes accumulated, [8 + r] finished jobs of ring entry r.
+// job, [1] passes accumulated, [3] vertex tape records of the wavefronts shaded
+// so far, [8 + r] finished jobs of ring entry r.
 __global__ void k_stream_init(long long* ctl, int* counts) {
   const int i = threadIdx.x;
   if (i < kStreamCtl) ctl[i] = 0;
@@ -956,6 +993,7 @@ __global__ void k_stream_next_dense(SceneView sc, PathBuffers nb, const long lon
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     T[0] = job0 + n;
     T[1] = acc + k;
+    T[3] = S[3] + nb.counts[wave_count(nxt ^ 1)];
     for (int r = 0; r < kStreamRing; ++r) {
       const long long d = (r - acc % kStreamRing + kStreamRing) % kStreamRing;  // ring entry r holds pass acc + d
       T[8 + r] = d < k ? 0 : S[8 + r];
@@ -1010,7 +1048,7 @@ int stream_group_slots(int npx, int g, int K) {
 
 int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_t* streams, int K,
                   const PassConfig& cfg, int passes, int slots_cap, float4* accum, float4* average, float4* ring,
-                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err) {
+                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err, StreamTape* tape) {
   const int npx = sc.width * sc.height;
   if (passes <= 0 || npx <= 0 || K < 1) return passes <= 0 ? kOk : (err = "bad stream groups", kEInval);
   PassTimer* tm = cfg.timer;
@@ -1076,15 +1114,23 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
         sp.msnn = 0;
         sp.cur = cur[g];
         sp.set = cur[g];  // the state copies and the append sets alternate together
-        launch_timed(t, 1, k_shade_dense, dim3(shade_blocks), dim3(256), st, sc, A, B, sp);
         // scheduler state: call m reads half m % 2 and writes the other
         long long* c = ctl + (size_t)g * kStreamCtl;
         long long* S = c + kStreamHalf * (calls[g] & 1);
         long long* T = c + kStreamHalf * ((calls[g] + 1) & 1);
+        if (tape)
+          launch_timed(t, 1, k_shade_dense_tape, dim3(shade_blocks), dim3(256), st, sc, A, B, sp, tape->tape[g],
+                       (const long long*)(S + 3));
+        else
+          launch_timed(t, 1, k_shade_dense, dim3(shade_blocks), dim3(256), st, sc, A, B, sp);
         launch_timed(t, 3, k_stream_next_dense, dim3(shade_blocks), dim3(256), st, sc, B, S, T, ring, accum, average,
                      nxt, sp.set, slots, cfg.accum_id, cfg.seed_offset, npx, g, K, cnt, passes);
         launch_trace(false, true, sc, A, B, TraceArgs{nxt, sp.set, 3, 0}, tr_blocks, t, nullptr, st);
-        launch_timed(t, 3, k_shadow_resolve_dense, dim3(shade_blocks), dim3(256), st, A, B, sp.set);
+        if (tape)
+          launch_timed(t, 3, k_shadow_resolve_dense_tape, dim3(shade_blocks), dim3(256), st, A, B, sp.set,
+                       tape->tape[g], (const long long*)(S + 3));
+        else
+          launch_timed(t, 3, k_shadow_resolve_dense, dim3(shade_blocks), dim3(256), st, A, B, sp.set);
         launch_timed(t, 3, k_stream_finish_dense, dim3(shade_blocks), dim3(256), st, A, T, ring, npx, sp.set);
         ++calls[g];
         cur[g] = nxt;
@@ -1114,6 +1160,8 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
       }
     }
   }
+  if (tape)
+    for (int g = 0; g < K; ++g) tape->count[g] = ctl + (size_t)g * kStreamCtl + kStreamHalf * (calls[g] & 1) + 3;
   return kOk;
 }
 

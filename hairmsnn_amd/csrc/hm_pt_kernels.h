@@ -178,6 +178,25 @@ constexpr long long kTwoGroupJobs = 1 << 20;
 // and a small image keeps all its passes in flight (256 x 256, 16 passes: two
 // paths per pixel 4.0 ms, all 16 passes 2.6 ms). About 340 bytes per path.
 constexpr int kStreamPaths = 4 << 20;
+// Vertex tape of the streaming schedule, for the adjoint: one record per path
+// and iteration, in wavefront order (record base + i is path i of the
+// iteration's wavefront; the base is the sum of the wavefronts before).
+struct VertexTape {
+  float4* o;      // ray origin, hit distance
+  float4* d;      // ray direction, hit coordinate u
+  float4* beta;   // throughput, random state (bits)
+  float4* L;      // radiance gathered before the vertex, prim (bits; < 0: no hair vertex, the other arrays are not written)
+  int4* meta;     // pixel, pass (relative to the call's first), vertex depth, unused
+  uint8_t* vis;   // bit 0 / 1: the light / BSDF sample's shadow ray was visible
+  long long cap;  // records it holds; later ones are counted but not written
+};
+constexpr size_t kTapeRecordBytes = 4 * sizeof(float4) + sizeof(int4) + 1;
+// Tapes of the stream groups and, after the run, where each group's record
+// count is.
+struct StreamTape {
+  VertexTape tape[kStreamGroups];
+  const long long* count[kStreamGroups];
+};
 // Paths that a stream group's buffers hold for an image of npx pixels.
 inline int stream_slots(int npx) {
   const long long share = kStreamPaths / kStreamGroups;
@@ -201,7 +220,7 @@ static_assert(8 + kStreamRing <= kStreamHalf && 2 * kStreamHalf <= kStreamCtl, "
 // radiance is left in ring entry (passes - 1) % kStreamRing.
 int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_t* streams, int K,
                   const PassConfig& cfg, int passes, int slots_cap, float4* accum, float4* average, float4* ring,
-                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err);
+                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err, StreamTape* tape = nullptr);
 // Pixels of stream group g of K over npx pixels, and the pixel of a group's
 // i-th pixel.
 int stream_group_slots(int npx, int g, int K);

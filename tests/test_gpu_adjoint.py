@@ -257,3 +257,29 @@ def test_c3_on_c1_geometry_central_differences(gpu):
         sc.set_strand_sigma_a(sig)
     print(f"64 central differences: {64 - bad} agree")
     assert bad <= 2
+
+
+def test_long_paths_outgrow_the_first_tape(gpu):
+    """Lossless hair seen from inside: the paths leave more vertices than the
+    vertex tape is first sized for (10 per path), so the first call repeats its
+    trace with a larger tape. Its gradients are the sums of the passes' own
+    (seed offsets 0..5, on the grown tape). Bound: the same FP32 terms summed in
+    another order, about 3e5 of them with 2^-24 each, random signs."""
+    cfg = json.loads((SCENES / "c0_hairball.json").read_text())
+    cfg["integrator"].update({"width": 64, "height": 64})
+    cfg["hair"]["sigma_a"] = [0.0, 0.0, 0.0]
+    cfg["hair"]["procedural"].update({"strands": 40_000, "radius": 0.02})
+    cfg["camera"].update({"from": [0.0, -1.2, 0.0], "to": [0.0, -3.0, 0.0]})
+    rng = np.random.default_rng(3)
+    d = rng.normal(size=(64, 64, 3)).astype(np.float32)
+    with gpu.Scene(json_text=cfg) as sc:
+        rays = sc.trace_stats(2)["closest_rays"] / (2 * 64 * 64)
+        assert rays > 15, rays
+        gs, gg, gp = sc.adjoint(d, 6, per_pixel=True)
+        one = []
+        for k in range(6):
+            sc.set_seed_offset(k)
+            one.append(sc.adjoint(d / 6, 1, per_pixel=True))
+    for whole, parts in ((gs, [x[0] for x in one]), (gg, [x[1] for x in one]), (gp, [x[2] for x in one])):
+        tot = np.sum([p.astype(np.float64) for p in parts], axis=0)
+        assert np.linalg.norm(whole - tot) <= 3e-5 * np.linalg.norm(tot)
