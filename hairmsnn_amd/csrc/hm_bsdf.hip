@@ -2,7 +2,7 @@
 // hmsnn_hair_bsdf_sample_dev: one query per lane, 40-byte query records.
 #include <hip/hip_runtime.h>
 
-#include "hm_hair_bsdf.h"
+#include "hm_hair_stream.h"
 #include "hm_internal.h"
 
 namespace hm {
@@ -20,13 +20,14 @@ __global__ void k_bsdf_eval(HairConsts hc, const BsdfQuery* q, int n, float* f_r
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const BsdfQuery x = q[i];
-  const HairWo w = hair_prepare(hc, v3(x.wo[0], x.wo[1], x.wo[2]), x.h, v3(x.sigma_a[0], x.sigma_a[1], x.sigma_a[2]));
-  float p;
-  const V3 f = hair_eval(hc, w, v3(x.wi[0], x.wi[1], x.wi[2]), &p);
-  f_rgb[3 * (size_t)i] = f.x;
-  f_rgb[3 * (size_t)i + 1] = f.y;
-  f_rgb[3 * (size_t)i + 2] = f.z;
-  pdf[i] = p;
+  const V3 wo = v3(x.wo[0], x.wo[1], x.wo[2]);
+  const HairWo w = stream_prepare(hc, wo, x.h, v3(x.sigma_a[0], x.sigma_a[1], x.sigma_a[2]));
+  const V3 wi = v3(x.wi[0], x.wi[1], x.wi[2]);
+  const FPdf e = stream_eval(hc, w, wo, wi);
+  f_rgb[3 * (size_t)i] = e.f.x;
+  f_rgb[3 * (size_t)i + 1] = e.f.y;
+  f_rgb[3 * (size_t)i + 2] = e.f.z;
+  pdf[i] = e.pdf;
 }
 
 __global__ void k_bsdf_sample(HairConsts hc, const BsdfQuery* q, const float4* u4, int n, float* wi_out,
@@ -34,19 +35,19 @@ __global__ void k_bsdf_sample(HairConsts hc, const BsdfQuery* q, const float4* u
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const BsdfQuery x = q[i];
-  const HairWo w = hair_prepare(hc, v3(x.wo[0], x.wo[1], x.wo[2]), x.h, v3(x.sigma_a[0], x.sigma_a[1], x.sigma_a[2]));
+  const V3 wo = v3(x.wo[0], x.wo[1], x.wo[2]), sigma_a = v3(x.sigma_a[0], x.sigma_a[1], x.sigma_a[2]);
+  const HairWo w = stream_prepare(hc, wo, x.h, sigma_a);
   const float4 u = u4[i];
   int p;
-  const V3 wi = hair_sample_dir(hc, w, u.x, u.y, u.z, u.w, &p);
-  float pd;
-  const V3 f = hair_eval(hc, w, wi, &pd);
+  const V3 wi = stream_sample_dir(hc, w, wo, sigma_a, u.x, u.y, u.z, u.w, &p);
+  const FPdf e = stream_eval(hc, w, wo, wi);
   wi_out[3 * (size_t)i] = wi.x;
   wi_out[3 * (size_t)i + 1] = wi.y;
   wi_out[3 * (size_t)i + 2] = wi.z;
-  f_rgb[3 * (size_t)i] = f.x;
-  f_rgb[3 * (size_t)i + 1] = f.y;
-  f_rgb[3 * (size_t)i + 2] = f.z;
-  pdf[i] = pd;
+  f_rgb[3 * (size_t)i] = e.f.x;
+  f_rgb[3 * (size_t)i + 1] = e.f.y;
+  f_rgb[3 * (size_t)i + 2] = e.f.z;
+  pdf[i] = e.pdf;
   if (lobe) lobe[i] = p;
 }
 

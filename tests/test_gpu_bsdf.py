@@ -74,3 +74,55 @@ def test_sample_matches_fp64(gpu):
     # and the sampled f, pdf match the FP64 oracle where the direction matched
     e = np.abs(p32[good].astype(np.float64) - p64[good]) / p64[good]
     assert np.quantile(e, 0.999) <= 1e-4
+
+
+def edge_queries(case, n=257):
+    """A ragged count of queries beside the places where the streams change
+    formula: the arc sine's halves (|h| = 1/2 and 1), the arc tangent's octants
+    (tan(pi / 8), the axes with either sign of zero), the longitudinal lobe's
+    Bessel argument of 12, directions along the fibre."""
+    q = bsdf_queries(n, seed=11)
+    if case == "h":
+        q[:, 6] = np.resize(np.float32([0.5, np.nextafter(np.float32(0.5), np.float32(1)), -0.5, 0.0, -0.0, 0.99, -0.99]), n)
+    elif case == "azimuth":
+        a = np.resize(np.arange(-16, 17) * (np.pi / 16), n) + np.resize([0.0, 1e-7, -1e-7, 1e-3], n)
+        r = np.sqrt(1.0 - q[:, 3].astype(np.float64) ** 2)
+        q[:, 4], q[:, 5] = r * np.cos(a), r * np.sin(a)
+        q[:, 1] = np.resize(np.float32([0.0, -0.0]), n)
+        q[:, 2] = np.sqrt(1.0 - q[:, 0].astype(np.float64) ** 2) * np.resize([1.0, 1.0, -1.0], n)
+    else:
+        assert case == "along"
+        q[:, 0] = np.resize(np.float32([1.0, -1.0]), n)
+        q[:, 1:3] = np.resize(np.float32([0.0, 0.0, -0.0, 0.0, -0.0, -0.0]), 2 * n).reshape(n, 2)
+    return q
+
+
+@pytest.mark.parametrize("beta", [0.12, 0.3, 0.6])
+@pytest.mark.parametrize("case", ["h", "azimuth", "along"])
+def test_streams_at_the_edges_of_their_formulas(gpu, case, beta):
+    """Against FP64: an azimuth off by a rounding (pi 2^-23) moves N_p by that
+    over its scale s, a sine or cosine product off by two roundings moves M_p
+    by those over v; three of the first and four of the second may add up. The
+    lobe is the FP64 one wherever the draw is not beside an edge."""
+    q = edge_queries(case)
+    u = uniforms(q.shape[0], 4, 12)
+    prm = ol.hair_params(beta, beta, ALPHA_2DEG)
+    s = np.sqrt(np.pi / 8) * (0.265 * beta + 1.194 * beta**2 + 5.372 * beta**22)
+    v = 0.25 * (0.726 * beta + 0.812 * beta**2 + 3.7 * beta**20) ** 2  # the narrowest lobe's
+    tol = 2.0**-23 * (3 * np.pi / s + 4 / v) + 1e-6
+    f64, p64 = ol.hair_eval(q, prm, 0)
+    f32, p32 = gpu.hair_bsdf_eval(q, beta, beta, ALPHA_2DEG)
+    for g, o in ((f32, f64), (p32, p64)):
+        e = np.linalg.norm(g - o) / np.linalg.norm(o)
+        print(f"{case} {beta}: {e:.2e} of {tol:.2e}")
+        assert np.all(np.isfinite(g)) and e <= tol
+    wi64, sf64, sp64, l64 = ol.hair_sample(q, u, prm, 0)
+    wi32, sf32, sp32, l32 = gpu.hair_bsdf_sample(q, u, beta, beta, ALPHA_2DEG)
+    same = l32 == l64
+    assert same.sum() >= same.size - 1
+    assert np.all(np.isfinite(wi32)) and np.abs(np.linalg.norm(wi32, axis=1) - 1).max() <= 4e-7
+    # the direction's azimuth and inclination carry the rounding of a draw
+    # next to 0 or 1 (2^-24 of it over the logistic's or the lobe's slope)
+    assert np.quantile(np.linalg.norm(wi32 - wi64, axis=1)[same], 0.95) <= 2e-5
+    e = np.abs(sp32[same] - sp64[same]) / sp64[same]
+    assert np.median(e) <= tol
