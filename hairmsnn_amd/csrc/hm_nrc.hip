@@ -25,12 +25,14 @@
 
 namespace hm {
 
-// Per-frame state of one pipeline slot: path buffers, the G_BUFFER arrays
-// and training records of one frame, and the stream its G_BUFFER pass runs
-// on. The pass does not depend on the network, so consecutive frames' passes
-// run on consecutive slots and overlap; inference, RENDER and training run in
-// frame order on the context stream.
+// State of one pipeline slot: path buffers, the G_BUFFER arrays and training
+// records of up to `frames` consecutive frames, and the stream their G_BUFFER
+// pass runs on. The pass does not depend on the network, so consecutive
+// frames are traced as one pass and consecutive batches' passes run on
+// consecutive slots and overlap; inference, RENDER and training run in frame
+// order on the context stream.
 struct NrcSlot {
+  int frames = 0;  // capacity
   PathBuffers pb{};
   std::vector<void*> allocs;
   hipStream_t st = nullptr;
@@ -52,6 +54,8 @@ struct NrcSlot {
     if (st) (void)hipStreamSynchronize(st);
     for (void* p : allocs) dev_free(p);
     allocs.clear();
+    frames = 0;
+    used = false;
     if (idx_host) (void)hipHostFree(idx_host);
     idx_host = nullptr;
     for (hipEvent_t* e : {&ev_gb, &ev_done, &ev_copy})
@@ -63,7 +67,8 @@ struct NrcSlot {
 
 // The buffers and streams stay with the context from one hmsnn_nrc_begin to
 // the next (allocating and freeing them took 47 ms of a begin at 512 x 512,
-// twice the 8 frames that followed); everything a run computes starts over.
+// several times the 8 frames that followed); everything a run computes starts
+// over.
 struct NrcState {
   MlpState* mlp = nullptr;
   bool ready = false;  // fully built (a failed setup is not reused)
@@ -80,11 +85,17 @@ struct NrcState {
   int frame = 0;
   uint64_t rng_state = 0;
   std::vector<int> idx;  // current permutation of the training indices
-  // frames in flight: 4 took 10.3 ms per C1 frame against 12.3 ms with 3
-  // (0.54 s against 0.57 s for 64 frames in the benchmark process)
-  static constexpr int kSlots = 4;
+  // Frames of one pass: a pass's 40 depths are bound by their longest rays'
+  // chains, about 0.14 ms each at any path count past the tenth, so frames
+  // share them (20 frames of 256 x 256: 11.8 ms one by one on four slots, 4.4
+  // ms at 8 to a pass, 3.5 ms at 16, 4.0 ms at 32). Two slots overlap one
+  // pass's last depths with the next one's first; a call of at least
+  // kSplitPaths paths is two passes or more for that (8 frames of 512 x 512:
+  // 24.4 ms one by one, 11.4 ms in one pass, 10.8 ms in two).
+  static constexpr int kSlots = 2, kBatch = 16;
+  static constexpr int kBatchPaths = 4 << 20, kSplitPaths = 2 << 20;
   NrcSlot slots[kSlots];
-  int next_slot = 0, last_slot = -1;
+  int next_slot = 0, last_slot = -1, last_frame = 0;  // the last frame: its slot and place there
   // shared, used in frame order on the context stream
   std::vector<void*> allocs;
   float* cache = nullptr;    // n_query x 3
@@ -105,7 +116,7 @@ struct NrcState {
   int restart(std::string& err) {
     HM_HIP(hipStreamSynchronize(ctx_stream), err);
     for (NrcSlot& sl : slots) {
-      HM_HIP(hipStreamSynchronize(sl.st), err);
+      if (sl.st) HM_HIP(hipStreamSynchronize(sl.st), err);
       sl.used = false;
     }
     mlp_destroy(mlp);
@@ -144,13 +155,14 @@ __device__ __forceinline__ void block_count(int* counter, int v) {
 // plus throughput x max(cache, 0), a NaN cache counting as 0; accumulated
 // like writePixel (utils.cuh:13-35, NaN scrub). Also stores the G-buffer
 // radiance for inspection and counts the frame's cache queries.
-__global__ void k_nrc_render(PathBuffers pb, NrcPassArgs nr, const float* cache, float4* gb_rad, float4* acc,
+// first: the frame's first slot in pb; nr holds the frame's own arrays.
+__global__ void k_nrc_render(PathBuffers pb, int first, NrcPassArgs nr, const float* cache, float4* gb_rad, float4* acc,
                              float4* avg, int accum_id, int* counts) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   const bool in = i < nr.frame_size;
   bool queried = false;
   if (in) {
-    const float4 l4 = (pb.flags[i] & kNrcSuffix) ? pb.L_short[i] : pb.L[i];
+    const float4 l4 = (pb.flags[first + i] & kNrcSuffix) ? pb.L_short[first + i] : pb.L[first + i];
     const float4 b4 = nr.gb_beta[i];
     V3 cr = v3(cache[3 * (size_t)i], cache[3 * (size_t)i + 1], cache[3 * (size_t)i + 2]);
     if (any_nan(cr)) cr = v3(0.f);
@@ -239,7 +251,58 @@ float nrc_lr_at(float base, int step) {
   return base * std::pow(0.33f, (float)((step - 4000) / 4000 + 1));
 }
 
-// The run's buffers, streams and events (the sizes in m are set).
+// Buffers, stream and events of a slot for passes of `frames` frames.
+int nrc_alloc_slot(Context& c, const NrcState& m, NrcSlot& sl, int frames, std::string& err) {
+  const size_t npx = (size_t)m.frame_size * frames, tpx = (size_t)m.n_tpx * frames;
+  auto S = [&](void** p, size_t bytes) -> int {
+    HM_TRY(dev_alloc(p, bytes, err));
+    sl.allocs.push_back(*p);
+    return kOk;
+  };
+  HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
+  for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
+    HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
+  HM_TRY(alloc_path_buffers(sl.pb, sl.allocs, npx, true, c.stack_levels(), c.trace_blocks * kTraceBlock, sl.st, err));
+  HM_TRY(S((void**)&sl.train_idx, sizeof(int) * tpx));
+  HM_TRY(S((void**)&sl.query, sizeof(float) * kNnInputCh * (size_t)m.n_query * frames));
+  HM_TRY(S((void**)&sl.gb_beta, sizeof(float4) * npx));
+  HM_TRY(S((void**)&sl.gb_hit, npx));
+  HM_TRY(S((void**)&sl.state, sizeof(float4) * npx));
+  HM_TRY(S((void**)&sl.prev, sizeof(float4) * npx));
+  for (float4*& t : sl.tb) HM_TRY(S((void**)&t, sizeof(float4) * tpx * kNrcMaxBounces));
+  HM_TRY(S((void**)&sl.tb_bounces, sizeof(int) * tpx));
+  HM_TRY(S((void**)&sl.tb_hit, tpx));
+  HM_HIP(hipHostMalloc((void**)&sl.idx_host, sizeof(int) * tpx), err);
+  HM_HIP(hipStreamSynchronize(sl.st), err);  // the set-up work
+  sl.frames = frames;
+  return kOk;
+}
+
+// The frames of one pass in a call of `frames` frames, and the slots for it.
+// Without the memory for larger or more slots the ones that are there serve
+// (nrc_setup made one for single frames). No slot has work in flight.
+int nrc_batch(Context& c, NrcState& m, int frames) {
+  const int cap = std::clamp(NrcState::kBatchPaths / m.frame_size, 1, NrcState::kBatch);
+  const int least = frames > 1 && (long long)frames * m.frame_size >= NrcState::kSplitPaths ? 2 : 1;
+  const int batches = std::max(least, (frames - 1) / cap + 1), want = (frames - 1) / batches + 1;
+  for (int k = 0; k < std::min(NrcState::kSlots, batches); ++k) {
+    NrcSlot& sl = m.slots[k];
+    if (sl.frames >= want) continue;
+    NrcSlot grown;
+    std::string err;
+    if (nrc_alloc_slot(c, m, grown, want, err)) {
+      grown.release();
+      (void)hipGetLastError();
+      break;
+    }
+    sl.release();
+    sl = std::move(grown);
+    if (m.last_slot == k) m.last_slot = -1;
+  }
+  return std::min(want, m.slots[0].frames);
+}
+
+// The buffers that the frames share (the sizes in m are set), and a slot.
 int nrc_alloc(Context& c, NrcState& m, std::string& err) {
   const int npx = m.frame_size;
   auto A = [&](void** p, size_t bytes) -> int {
@@ -247,29 +310,7 @@ int nrc_alloc(Context& c, NrcState& m, std::string& err) {
     m.allocs.push_back(*p);
     return kOk;
   };
-  const size_t nv = (size_t)m.n_tpx * kNrcMaxBounces;
-  for (NrcSlot& sl : m.slots) {
-    HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
-    for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
-      HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
-    HM_TRY(alloc_path_buffers(sl.pb, sl.allocs, (size_t)npx, true, c.stack_levels(), c.trace_blocks * kTraceBlock,
-                              sl.st, err));
-    auto S = [&](void** p, size_t bytes) -> int {
-      HM_TRY(dev_alloc(p, bytes, err));
-      sl.allocs.push_back(*p);
-      return kOk;
-    };
-    HM_TRY(S((void**)&sl.train_idx, sizeof(int) * (size_t)m.n_tpx));
-    HM_TRY(S((void**)&sl.query, sizeof(float) * kNnInputCh * (size_t)m.n_query));
-    HM_TRY(S((void**)&sl.gb_beta, sizeof(float4) * (size_t)npx));
-    HM_TRY(S((void**)&sl.gb_hit, (size_t)npx));
-    HM_TRY(S((void**)&sl.state, sizeof(float4) * (size_t)npx));
-    HM_TRY(S((void**)&sl.prev, sizeof(float4) * (size_t)npx));
-    for (float4*& t : sl.tb) HM_TRY(S((void**)&t, sizeof(float4) * nv));
-    HM_TRY(S((void**)&sl.tb_bounces, sizeof(int) * (size_t)m.n_tpx));
-    HM_TRY(S((void**)&sl.tb_hit, (size_t)m.n_tpx));
-    HM_HIP(hipHostMalloc((void**)&sl.idx_host, sizeof(int) * (size_t)m.n_tpx), err);
-  }
+  HM_TRY(nrc_alloc_slot(c, m, m.slots[0], 1, err));
   HM_TRY(A((void**)&m.cache, sizeof(float) * 3 * (size_t)m.n_query));
   HM_TRY(A((void**)&m.gb_rad, sizeof(float4) * (size_t)npx));
   HM_TRY(A((void**)&m.train_in, sizeof(float) * kNnInputCh * (size_t)m.n_rec));
@@ -316,14 +357,14 @@ int nrc_setup(Context& c, std::string& err) {
   HM_HIP(hipMemsetAsync(m->avg, 0, sizeof(float4) * (size_t)npx, c.stream), err);
   m->idx.resize(m->n_tpx);
   for (int i = 0; i < m->n_tpx; ++i) m->idx[i] = i;  // thrust::sequence (render_nrc.cu:170-173)
-  // the slots' first passes start after the set-up work
-  HM_HIP(hipStreamSynchronize(c.stream), err);
-  for (NrcSlot& sl : m->slots) HM_HIP(hipStreamSynchronize(sl.st), err);
+  HM_HIP(hipStreamSynchronize(c.stream), err);  // the first passes start after the set-up work
   m->ready = true;
   return kOk;
 }
 
-NrcPassArgs nrc_args(const Context& c, const NrcState& m, const NrcSlot& sl) {
+// The pass's arguments, its arrays from frame f of the slot on.
+NrcPassArgs nrc_args(const Context& c, const NrcState& m, const NrcSlot& sl, int f) {
+  const size_t npx = (size_t)f * m.frame_size, tpx = (size_t)f * m.n_tpx, nv = tpx * kNrcMaxBounces;
   NrcPassArgs a{};
   a.enabled = 1;
   a.all_unbiased = m.all_unbiased;
@@ -332,86 +373,97 @@ NrcPassArgs nrc_args(const Context& c, const NrcState& m, const NrcSlot& sl) {
   a.frame_size = m.frame_size;
   a.n_tpx = m.n_tpx;
   a.every_nth = m.every_nth;
-  a.query = sl.query;
-  a.gb_beta = sl.gb_beta;
-  a.gb_hit = sl.gb_hit;
-  a.state = sl.state;
-  a.prev = sl.prev;
-  a.tb_pos = sl.tb[0];
-  a.tb_wo = sl.tb[1];
-  a.tb_n = sl.tb[2];
-  a.tb_rad = sl.tb[3];
-  a.tb_beta = sl.tb[4];
-  a.tb_bounces = sl.tb_bounces;
-  a.tb_hit = sl.tb_hit;
+  a.n_query = m.n_query;
+  a.query = sl.query + (size_t)f * m.n_query * kNnInputCh;
+  a.gb_beta = sl.gb_beta + npx;
+  a.gb_hit = sl.gb_hit + npx;
+  a.state = sl.state + npx;
+  a.prev = sl.prev + npx;
+  a.tb_pos = sl.tb[0] + nv;
+  a.tb_wo = sl.tb[1] + nv;
+  a.tb_n = sl.tb[2] + nv;
+  a.tb_rad = sl.tb[3] + nv;
+  a.tb_beta = sl.tb[4] + nv;
+  a.tb_bounces = sl.tb_bounces + tpx;
+  a.tb_hit = sl.tb_hit + tpx;
   return a;
 }
 
-// One frame (render_nrc.cu:640-701): the shuffle and G_BUFFER pass on the
-// frame's slot, then inference, RENDER and training in frame order on the
-// context stream. tm, when given, receives events: [0], [1] around the
+// `frames` consecutive frames (render_nrc.cu:640-701): their shuffles and
+// G_BUFFER passes, as one pass, on the next slot, then inference, RENDER and
+// training in frame order on the context stream. tm, when given, is the
+// frames' timers, whose events mark: [0], [1] (the first frame's only) the
 // G_BUFFER pass on the slot's stream; [2] inference start, [3] RENDER start,
 // [4] training start and [5] end on the context stream.
-int nrc_frame(Context& c, NrcState& m, NrcTimer* tm, std::string& err) {
+int nrc_frames(Context& c, NrcState& m, int frames, NrcTimer* tm, std::string& err) {
   const int npx = m.frame_size;
   NrcSlot& sl = m.slots[m.next_slot];
   m.last_slot = m.next_slot;
+  m.last_frame = frames - 1;
   m.next_slot = (m.next_slot + 1) % NrcState::kSlots;
+  if (m.slots[m.next_slot].frames < frames) m.next_slot = 0;
   hipStream_t st = sl.st, cs = c.stream;
   if (sl.used) HM_HIP(hipStreamWaitEvent(st, sl.ev_done, 0), err);
   sl.used = true;
-  if (tm) (void)hipEventRecord(tm->e[0], st);
-  // ---- shuffle (render_nrc.cu:652-655): seeded, applied to the previous order ----
+  if (tm) (void)hipEventRecord(tm[0].e[0], st);
+  // ---- shuffles (render_nrc.cu:652-655): seeded, applied to the previous order ----
   HM_HIP(hipEventSynchronize(sl.ev_copy), err);  // the slot's staging buffer is free again
-  for (int i = m.n_tpx - 1; i > 0; --i) std::swap(m.idx[i], m.idx[(int)(m.next_u64() % (uint64_t)(i + 1))]);
-  std::copy(m.idx.begin(), m.idx.end(), sl.idx_host);
-  HM_HIP(hipMemcpyAsync(sl.train_idx, sl.idx_host, sizeof(int) * (size_t)m.n_tpx, hipMemcpyHostToDevice, st), err);
+  const size_t tpx = (size_t)m.n_tpx * frames, nv = tpx * kNrcMaxBounces;
+  for (int f = 0; f < frames; ++f) {
+    for (int i = m.n_tpx - 1; i > 0; --i) std::swap(m.idx[i], m.idx[(int)(m.next_u64() % (uint64_t)(i + 1))]);
+    std::copy(m.idx.begin(), m.idx.end(), sl.idx_host + (size_t)f * m.n_tpx);
+  }
+  HM_HIP(hipMemcpyAsync(sl.train_idx, sl.idx_host, sizeof(int) * tpx, hipMemcpyHostToDevice, st), err);
   HM_HIP(hipEventRecord(sl.ev_copy, st), err);
-  // ---- clear the frame's buffers (owlBufferClear + RESET, render_nrc.cu:684-692) ----
-  const size_t nv = (size_t)m.n_tpx * kNrcMaxBounces;
-  HM_HIP(hipMemsetAsync(sl.query, 0, sizeof(float) * kNnInputCh * (size_t)m.n_query, st), err);
-  HM_HIP(hipMemsetAsync(sl.gb_beta, 0, sizeof(float4) * (size_t)npx, st), err);
-  HM_HIP(hipMemsetAsync(sl.gb_hit, 0, (size_t)npx, st), err);
+  // ---- clear the frames' buffers (owlBufferClear + RESET, render_nrc.cu:684-692) ----
+  HM_HIP(hipMemsetAsync(sl.query, 0, sizeof(float) * kNnInputCh * (size_t)m.n_query * frames, st), err);
+  HM_HIP(hipMemsetAsync(sl.gb_beta, 0, sizeof(float4) * (size_t)npx * frames, st), err);
+  HM_HIP(hipMemsetAsync(sl.gb_hit, 0, (size_t)npx * frames, st), err);
   for (float4* t : sl.tb) HM_HIP(hipMemsetAsync(t, 0, sizeof(float4) * nv, st), err);
-  HM_HIP(hipMemsetAsync(sl.tb_bounces, 0, sizeof(int) * (size_t)m.n_tpx, st), err);
-  HM_HIP(hipMemsetAsync(sl.tb_hit, 0, (size_t)m.n_tpx, st), err);
+  HM_HIP(hipMemsetAsync(sl.tb_bounces, 0, sizeof(int) * tpx, st), err);
+  HM_HIP(hipMemsetAsync(sl.tb_hit, 0, tpx, st), err);
   // ---- G_BUFFER ----
   PassConfig cfg = c.pt_pass_config();
   cfg.accum_id = m.frame;
+  cfg.frames = frames;
   cfg.dl_zero = 1;  // nrcTracePaths lights every vertex (nrc.cu:166-169)
   cfg.dl_from = 1;
   cfg.max_vertex = kNrcMaxBounces - 1;
   cfg.train_idx = sl.train_idx;
   cfg.every_nth = m.every_nth;
-  cfg.nrc = nrc_args(c, m, sl);
+  cfg.nrc = nrc_args(c, m, sl, 0);
   HM_TRY(pt_run_pass(c.view_no_caps(), sl.pb, cfg, st, err));
-  if (tm) (void)hipEventRecord(tm->e[1], st);
+  if (tm) (void)hipEventRecord(tm[0].e[1], st);
   HM_HIP(hipEventRecord(sl.ev_gb, st), err);
   HM_HIP(hipStreamWaitEvent(cs, sl.ev_gb, 0), err);
-  // ---- infer (context stream, frame order) ----
-  if (tm) (void)hipEventRecord(tm->e[2], cs);
-  HM_HIP(hipMemsetAsync(m.train_in, 0, sizeof(float) * kNnInputCh * (size_t)m.n_rec, cs), err);
-  HM_HIP(hipMemsetAsync(m.train_tgt, 0, sizeof(float) * 3 * (size_t)m.n_rec, cs), err);
-  HM_HIP(hipMemsetAsync(m.counts_dev, 0, sizeof(int) * 4, cs), err);
-  HM_TRY(mlp_forward(*m.mlp, sl.query, m.n_query, m.cache, cs, err));
-  if (tm) (void)hipEventRecord(tm->e[3], cs);
-  // ---- RENDER ----
-  hipLaunchKernelGGL(k_nrc_render, dim3((npx + 255) / 256), dim3(256), 0, cs, sl.pb, cfg.nrc, m.cache, m.gb_rad,
-                     m.acc, m.avg, m.frame, m.counts_dev);
-  hipLaunchKernelGGL(k_nrc_train_data, dim3((m.n_tpx + 255) / 256), dim3(256), 0, cs, cfg.nrc, sl.train_idx,
-                     m.cache, m.train_in, m.train_tgt, m.n_rec, m.counts_dev);
-  HM_TRY(check_launch("nrc render", err));
-  if (tm) (void)hipEventRecord(tm->e[4], cs);
-  // ---- train ----
-  if (c.scene.nrc_train) {
-    const float lr = nrc_lr_at(m.lr, m.train_steps);
-    HM_TRY(mlp_loss_grad_step(*m.mlp, m.train_in, m.train_tgt, m.n_rec, m.loss, nullptr, nullptr, true, lr, cs,
-                              err));
-    m.train_steps++;
+  for (int f = 0; f < frames; ++f) {
+    const NrcPassArgs nr = nrc_args(c, m, sl, f);
+    hipEvent_t* e = tm ? tm[f].e : nullptr;
+    // ---- infer (context stream, frame order) ----
+    if (e) (void)hipEventRecord(e[2], cs);
+    HM_HIP(hipMemsetAsync(m.train_in, 0, sizeof(float) * kNnInputCh * (size_t)m.n_rec, cs), err);
+    HM_HIP(hipMemsetAsync(m.train_tgt, 0, sizeof(float) * 3 * (size_t)m.n_rec, cs), err);
+    HM_HIP(hipMemsetAsync(m.counts_dev, 0, sizeof(int) * 4, cs), err);
+    HM_TRY(mlp_forward(*m.mlp, nr.query, m.n_query, m.cache, cs, err));
+    if (e) (void)hipEventRecord(e[3], cs);
+    // ---- RENDER ----
+    hipLaunchKernelGGL(k_nrc_render, dim3((npx + 255) / 256), dim3(256), 0, cs, sl.pb, f * npx, nr, m.cache, m.gb_rad,
+                       m.acc, m.avg, m.frame, m.counts_dev);
+    hipLaunchKernelGGL(k_nrc_train_data, dim3((m.n_tpx + 255) / 256), dim3(256), 0, cs, nr,
+                       sl.train_idx + (size_t)f * m.n_tpx, m.cache, m.train_in, m.train_tgt, m.n_rec, m.counts_dev);
+    HM_TRY(check_launch("nrc render", err));
+    if (e) (void)hipEventRecord(e[4], cs);
+    // ---- train ----
+    if (c.scene.nrc_train) {
+      const float lr = nrc_lr_at(m.lr, m.train_steps);
+      HM_TRY(mlp_loss_grad_step(*m.mlp, m.train_in, m.train_tgt, m.n_rec, m.loss, nullptr, nullptr, true, lr, cs,
+                                err));
+      m.train_steps++;
+    }
+    if (e) (void)hipEventRecord(e[5], cs);
+    m.frame++;
   }
-  if (tm) (void)hipEventRecord(tm->e[5], cs);
   HM_HIP(hipEventRecord(sl.ev_done, cs), err);
-  m.frame++;
   return kOk;
 }
 
@@ -451,8 +503,10 @@ int hmsnn_nrc_frames(hmsnn_ctx* ctx, int frames, hmsnn_nrc_stats* stats) {
   std::string err;
   std::vector<NrcTimer> timers(stats ? (size_t)frames : 0);
   const auto t0 = std::chrono::steady_clock::now();
-  for (int k = 0; k < frames; ++k) {
-    int rc = nrc_frame(c, *c.nrc, stats ? &timers[k] : nullptr, err);
+  const int batch = frames > 0 ? nrc_batch(c, *c.nrc, frames) : 1;
+  c.nrc->next_slot = 0;
+  for (int k = 0; k < frames; k += batch) {
+    int rc = nrc_frames(c, *c.nrc, std::min(batch, frames - k), stats ? &timers[k] : nullptr, err);
     if (rc) return fail(rc, err);
   }
   hipError_t e = hipStreamSynchronize(c.stream);
@@ -460,8 +514,8 @@ int hmsnn_nrc_frames(hmsnn_ctx* ctx, int frames, hmsnn_nrc_stats* stats) {
   const auto t1 = std::chrono::steady_clock::now();
   if (stats) {
     hmsnn_nrc_stats local{};
+    for (int k = 0; k < frames; k += batch) local.gbuffer_ms += NrcTimer::ms(timers[k].e[0], timers[k].e[1]);
     for (NrcTimer& tm : timers) {
-      local.gbuffer_ms += NrcTimer::ms(tm.e[0], tm.e[1]);
       local.infer_ms += NrcTimer::ms(tm.e[2], tm.e[3]);
       local.render_ms += NrcTimer::ms(tm.e[3], tm.e[4]);
       local.train_ms += NrcTimer::ms(tm.e[4], tm.e[5]);
@@ -507,19 +561,20 @@ int hmsnn_nrc_get_buffer(hmsnn_ctx* ctx, int which, void* host, size_t bytes) {
   const size_t npx = (size_t)m->frame_size;
   if (m->last_slot < 0) return fail(HMSNN_EINVAL, "hmsnn_nrc_get_buffer: no frame rendered yet");
   const NrcSlot& sl = m->slots[m->last_slot];
+  const NrcPassArgs nr = nrc_args(ctx->c, *m, sl, m->last_frame);
   const void* src = nullptr;
   size_t need = 0;
   switch (which) {
-    case HMSNN_NRC_QUERY: src = sl.query, need = sizeof(float) * kNnInputCh * (size_t)m->n_query; break;
+    case HMSNN_NRC_QUERY: src = nr.query, need = sizeof(float) * kNnInputCh * (size_t)m->n_query; break;
     case HMSNN_NRC_CACHE: src = m->cache, need = sizeof(float) * 3 * (size_t)m->n_query; break;
     case HMSNN_NRC_GB_RADIANCE: src = m->gb_rad, need = sizeof(float4) * npx; break;
-    case HMSNN_NRC_GB_BETA: src = sl.gb_beta, need = sizeof(float4) * npx; break;
-    case HMSNN_NRC_GB_HIT: src = sl.gb_hit, need = npx; break;
+    case HMSNN_NRC_GB_BETA: src = nr.gb_beta, need = sizeof(float4) * npx; break;
+    case HMSNN_NRC_GB_HIT: src = nr.gb_hit, need = npx; break;
     case HMSNN_NRC_TRAIN_INPUT: src = m->train_in, need = sizeof(float) * kNnInputCh * (size_t)m->n_rec; break;
     case HMSNN_NRC_TRAIN_TARGET: src = m->train_tgt, need = sizeof(float) * 3 * (size_t)m->n_rec; break;
-    case HMSNN_NRC_TRAIN_IDX: src = sl.train_idx, need = sizeof(int) * (size_t)m->n_tpx; break;
-    case HMSNN_NRC_TRAIN_BOUNCES: src = sl.tb_bounces, need = sizeof(int) * (size_t)m->n_tpx; break;
-    case HMSNN_NRC_TRAIN_HIT: src = sl.tb_hit, need = (size_t)m->n_tpx; break;
+    case HMSNN_NRC_TRAIN_IDX: src = sl.train_idx + (size_t)m->last_frame * m->n_tpx, need = sizeof(int) * (size_t)m->n_tpx; break;
+    case HMSNN_NRC_TRAIN_BOUNCES: src = nr.tb_bounces, need = sizeof(int) * (size_t)m->n_tpx; break;
+    case HMSNN_NRC_TRAIN_HIT: src = nr.tb_hit, need = (size_t)m->n_tpx; break;
     default: return fail(HMSNN_EINVAL, "hmsnn_nrc_get_buffer: unknown buffer");
   }
   if (bytes != need) return fail(HMSNN_EINVAL, "hmsnn_nrc_get_buffer: size mismatch");

@@ -126,14 +126,16 @@ __device__ __forceinline__ void camera_path(const SceneView& sc, const PathBuffe
 // Primary rays for every pixel of pass `accum_id` (path_tracing.cu:29-48).
 // HairMSNN training pixels (hair_msnn.cu:206-209) are flagged here.
 // NRC (nrc != 0): training pixels by the same rule (cuda/nrc.cu:371-377),
-// every 16th of them, or all with all_unbiased, tracing an unbiased suffix.
+// every 16th of them, or all with all_unbiased, tracing an unbiased suffix;
+// train_idx holds n_train entries for each of the `frames` frames.
 __global__ void k_camera(SceneView sc, PathBuffers pb, int accum_id, int msnn, const int* train_idx,
-                         int every_nth, int n_train, int nrc, int all_unbiased) {
-  const int n = sc.width * sc.height;
+                         int every_nth, int n_train, int nrc, int all_unbiased, int frames) {
+  const int npx = sc.width * sc.height, n = npx * frames;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i == 0) pb.counts[wave_count(0)] = n;
   if (i >= n) return;
-  camera_path(sc, pb, i, i, accum_id);
+  const int f = i / npx, px = i - f * npx;
+  camera_path(sc, pb, i, px, accum_id + f);
   pb.queue[0][i] = i;
   uint32_t flags = 0;
   if (msnn) {
@@ -143,8 +145,8 @@ __global__ void k_camera(SceneView sc, PathBuffers pb, int accum_id, int msnn, c
     pb.L_short[i] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
   if (nrc) {
-    const int tr = i / every_nth;
-    if (tr < n_train && i % every_nth == train_idx[tr] % every_nth) {
+    const int tr = px / every_nth;
+    if (tr < n_train && px % every_nth == train_idx[f * n_train + tr] % every_nth) {
       flags |= kNrcTrain;
       if (tr % 16 == 0 || all_unbiased) flags |= kNrcUnbiased;
     }
@@ -249,7 +251,9 @@ __global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb,
       const V3 o = v3(o4.x, o4.y, o4.z), d = v3(d4.x, d4.y, d4.z);
       uint32_t fl = pb.flags[slot];
       const bool training = fl & kNrcTrain;
-      const int tr = slot / nr.every_nth;
+      const int frame = slot / nr.frame_size;
+      const int tr_px = (slot - frame * nr.frame_size) / nr.every_nth;  // within the frame
+      const int tr = frame * nr.n_tpx + tr_px;
       const bool miss = prim == kPrimMiss;
       Hit h;
       if (!miss) setup_hit(sc, o, d, pb.hit_t[slot], prim, pb.hit_u[slot], h);
@@ -290,7 +294,7 @@ __global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb,
             // primary path ends in a cache query at this vertex (nrc.cu:222-271)
             const float4 b4 = pb.beta[slot];
             nr.gb_beta[slot] = b4;
-            float* r = nr.query + (size_t)slot * kNnInputCh;
+            float* r = nr.query + ((size_t)frame * (nr.n_query - nr.frame_size) + slot) * kNnInputCh;
             const V3 p = h.p / nr.scene_scale;
             r[0] = p.x; r[1] = p.y; r[2] = p.z;
             r[3] = h.wo.x; r[4] = h.wo.y; r[5] = h.wo.z;
@@ -305,7 +309,7 @@ __global__ void __launch_bounds__(256) k_shade_nrc(SceneView sc, PathBuffers pb,
             }
           } else if (spread_cond) {
             // training suffix ends in a cache query (nrc.cu:273-309)
-            float* r = nr.query + ((size_t)nr.frame_size + tr) * kNnInputCh;
+            float* r = nr.query + ((size_t)frame * nr.n_query + nr.frame_size + tr_px) * kNnInputCh;
             const V3 p = h.p / nr.scene_scale;
             r[0] = p.x; r[1] = p.y; r[2] = p.z;
             r[3] = h.wo.x; r[4] = h.wo.y; r[5] = h.wo.z;
@@ -764,7 +768,9 @@ __global__ void k_shadow_resolve(PathBuffers pb, int msnn, int depth, int set, N
       pb.L_short[slot] = Ls;
     }
     if (nr.enabled && (pb.flags[slot] & kNrcTrain)) {
-      const int rec = slot / nr.every_nth * kNrcMaxBounces + depth;
+      const int frame = slot / nr.frame_size;
+      const int tr = frame * nr.n_tpx + (slot - frame * nr.frame_size) / nr.every_nth;
+      const int rec = tr * kNrcMaxBounces + depth;
       nr.tb_rad[rec] = make_float4(sum.x, sum.y, sum.z, 0.f);
     }
   }
@@ -857,10 +863,10 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
     hipLaunchKernelGGL(k_camera_points, dim3((n + 255) / 256), dim3(256), 0, stream, sc, pb,
                        cfg.accum_id + cfg.seed_offset, n, cfg.chunk > 0 ? cfg.chunk : n, cfg.grid_w, cfg.points);
   } else {
-    const int n = sc.width * sc.height;
+    const int n = sc.width * sc.height * cfg.frames;
     hipLaunchKernelGGL(k_camera, dim3((n + 255) / 256), dim3(256), 0, stream, sc, pb, cfg.accum_id + cfg.seed_offset,
                        cfg.msnn, cfg.train_idx, cfg.every_nth, cfg.nrc.enabled ? cfg.nrc.n_tpx : cfg.n_slots,
-                       cfg.nrc.enabled, cfg.nrc.all_unbiased);
+                       cfg.nrc.enabled, cfg.nrc.all_unbiased, cfg.frames);
   }
   HM_TRY(check_launch("camera", err));
   const bool count = cfg.stats != nullptr;
@@ -868,7 +874,7 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
 
   // Grids sized to the pass's paths (queues only shrink with depth), so a
   // small training-data pass does not dispatch the full-frame grid per depth.
-  const int n0 = cfg.camera_mode != 0 ? cfg.n_slots : sc.width * sc.height;
+  const int n0 = cfg.camera_mode != 0 ? cfg.n_slots : sc.width * sc.height * cfg.frames;
   const int ext_blocks = trace_grid(cfg.trace_blocks, n0);
   const int tr_blocks = trace_grid(cfg.trace_blocks, 3ll * n0);
   const int shade_blocks = std::min(cfg.shade_blocks, std::max(1, (n0 + 255) / 256));

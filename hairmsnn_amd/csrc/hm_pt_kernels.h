@@ -52,7 +52,8 @@ HM_D void gbuffer_write_miss(const GBufferOut& gb, int slot, V3 dir) {
 // Neural radiance caching G_BUFFER pass (cuda/nrc.cu:135-398): paths end
 // where their spread reaches the camera footprint (NRC sect. 3.4) and query
 // the cache there; training pixels keep tracing a suffix whose vertices
-// become training records. Slots are pixels.
+// become training records. Slot f * frame_size + p is pixel p of the pass's
+// f-th frame; every array below holds the frames' parts one after the other.
 constexpr int kNrcMaxBounces = 40;  // MAX_BOUNCES (nrc.cuh:13)
 constexpr uint32_t kNrcTrain = 1u, kNrcUnbiased = 2u, kNrcSuffix = 4u, kNrcRecalcA0 = 8u;
 
@@ -62,6 +63,7 @@ struct NrcPassArgs {
   float c;             // spread threshold multiplier
   float scene_scale;
   int frame_size;      // pixels; suffix cache queries follow at frame_size + training index
+  int n_query;         // cache queries of a frame
   int n_tpx;           // training pixels
   int every_nth;       // training pixel of pixel p: index p / every_nth
   float* query;        // cache-query records, 12 floats each
@@ -117,6 +119,7 @@ struct PassConfig {
   // each, train_idx per record); their pixel indices are written to pix
   int* pix = nullptr;
   NrcPassArgs nrc{};
+  int frames = 1;  // camera_mode 0: frames accum_id .. traced as one pass (NRC)
 };
 
 // Runs one full sample pass (camera -> all vertices). Leaves per-pixel

@@ -163,3 +163,32 @@ def test_second_run_on_a_scene_equals_the_first(gpu):
             out.append((sc.nrc_image(), sc.nrc_weights()))
     np.testing.assert_array_equal(out[0][0], out[2][0])
     np.testing.assert_array_equal(out[0][1], out[2][1])
+
+
+@pytest.mark.parametrize("frames", [2, 16, 17, 35])
+def test_frames_of_one_call_equal_frames_of_many(gpu, frames):
+    """A call traces up to 16 frames as one pass, in batches of like sizes on
+    two sets of buffers; image, weights and the last frame's buffers are those
+    of single-frame calls bit for bit, also on buffers that grew meanwhile."""
+    names = ("train_idx", "query", "gb_radiance", "gb_beta", "gb_hit", "train_input", "train_target", "train_bounces")
+
+    def result(sc):
+        return [sc.nrc_image(), sc.nrc_weights()] + [sc.nrc_buffer(n) for n in names]
+
+    with gpu.Scene(json_text=cfg_small(w=40, h=32, records=1280)) as sc:
+        sc.nrc_begin()
+        for _ in range(frames):
+            one = sc.nrc_frames(1)
+        single = result(sc)
+        sc.nrc_begin()
+        all_ = sc.nrc_frames(frames)
+        whole = result(sc)
+        sc.nrc_begin()
+        sc.nrc_frames(frames // 2)
+        sc.nrc_frames(frames - frames // 2)
+        halves = result(sc)
+    assert one["train_steps"] == all_["train_steps"] == frames
+    assert one["cache_queries"] == all_["cache_queries"] and one["train_records_used"] == all_["train_records_used"]
+    for a, b, c in zip(single, whole, halves):
+        np.testing.assert_array_equal(a, b)
+        np.testing.assert_array_equal(a, c)
