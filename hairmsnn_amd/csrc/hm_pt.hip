@@ -824,9 +824,12 @@ __global__ void HM_TRACE_BOUNDS_T(kCurves) k_trace_rays(SceneView sc, const floa
 // ---------------------------------------------------------------------------
 // Host launchers
 
-// Blocks of a trace launch of at most n rays.
+// Blocks of a trace launch of at most n rays: four rays to a wave until the
+// grid is full (RayQueue spreads them; one ray to a wave or 64 measured the
+// same within 3% at 1,000 to 100,000 rays).
+constexpr int kRaysPerBlock = 4 * (kTraceBlock / 64);
 static int trace_grid(int cap, long long n) {
-  return (int)std::min<long long>(cap, std::max<long long>(1, (n + kTraceBlock - 1) / kTraceBlock));
+  return (int)std::min<long long>(cap, std::max<long long>(1, (n + kRaysPerBlock - 1) / kRaysPerBlock));
 }
 
 // One trace launch; with a timer, its closest hits (record kind 0) and its
