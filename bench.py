@@ -48,7 +48,10 @@ SHADE_VERTEX_BYTES, SHADE_HIT_BYTES, SHADE_MOVE_BYTES, SHADE_DONE_BYTES, SHADE_S
 # WRITE_SIZE runs (copy-calibrated); counters cannot be read from inside this
 # process
 TRAFFIC_JSON = ROOT / "profiles" / "pt_c1_1024_hbm_traffic.json"
-PASS_KERNELS = {"extend": "k_extend<false, true, false>", "shade": "k_shade_dense", "shadow": "k_shadow<false, false>"}
+# k_trace traces both kinds of rays in one launch; timed per kernel they are
+# launches of their own, whose traffic and operations are not counted apart
+PASS_KERNELS = {"extend": "k_trace<false, true, false> (closest hits)", "shade": "k_shade_dense",
+                "shadow": "k_trace<false, true, false> (shadow rays)"}
 # FP32 VALU operations per launch (rocprofv3 SQ_INSTS_VALU_FLOPS_FP32 x 64
 # lanes) of the pass kernels and of the BSDF streams, for the VALU FLOP rates
 FLOPS_JSON = ROOT / "profiles" / "pt_c1_1024_flops.json"
@@ -280,7 +283,7 @@ def adjoint_rate(hm, scene_path: Path, size: int = 512, spp: int = 16) -> dict:
     """The differentiable-appearance workload: c1 geometry at size^2, spp
     samples, per-strand sigma_a ~ U(0.01, 0.5) (seed 3) and the global
     roughness / tilt; gradient of an L2 loss against a target rendered with
-    the scene's own sigma_a. Times the forward render and the path-replay
+    the scene's own sigma_a. Times the forward render and the path-wise
     adjoint."""
     cfg = json.loads(scene_path.read_text())
     cfg["integrator"].update({"width": size, "height": size, "spp": spp})

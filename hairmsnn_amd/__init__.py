@@ -269,7 +269,7 @@ class Scene:
         return int(self.info["num_strands"])
 
     def adjoint(self, dl_dimage: np.ndarray, spp: int, per_pixel: bool = False):
-        """Path-replay gradient of a loss of the spp-pass mean image given
+        """Path-wise gradient of a loss of the spp-pass mean image given
         dL/d(image) (H x W x 3 or 4): returns (d/d sigma_a per strand
         (num_strands x 3), d/d (beta_m, beta_n, alpha), and optionally each
         pixel's share of the latter (H x W x 3))."""

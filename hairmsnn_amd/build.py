@@ -55,7 +55,7 @@ def _run(cmd: list[str]) -> None:
 
 # Sources whose floating-point code must not depend on how the compiler fuses
 # multiplies and adds across statements: every shading kernel (per-pass,
-# streaming, NRC) and the adjoint's replay share the same inlined routines,
+# streaming, NRC) and the adjoint share the same inlined routines,
 # and schedules that trace the same paths must produce the same bits whatever
 # the surrounding kernel looks like. (Explicit fmaf calls are kept.)
 NO_CONTRACT = {"hm_pt.hip", "hm_adjoint.hip"}

@@ -1,6 +1,6 @@
 // Forward-mode derivatives of the hair BSDF value f * |cos| with respect to
 // the appearance parameters (beta_m, beta_n, alpha, sigma_a r/g/b), for the
-// path-replay adjoint.
+// path-wise adjoint.
 //
 // Directions, h and every sampling decision are held fixed (detached), so
 // only f itself is differentiated: through the lobe variances v (beta_m), the

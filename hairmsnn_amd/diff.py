@@ -1,4 +1,4 @@
-"""torch.autograd harness over the path tracer and its path-replay adjoint.
+"""torch.autograd harness over the path tracer and its path-wise adjoint.
 
 `render_hair(scene, sigma_a, params, spp)` renders the spp-pass mean image
 with per-strand absorption `sigma_a` (num_strands x 3) and global

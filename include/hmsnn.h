@@ -169,7 +169,7 @@ int hmsnn_set_strand_sigma_a(hmsnn_ctx* ctx, const float* sigma_host, int num_st
 
 /* Adds offset to the pass index that seeds each pixel's random stream
  * (path_tracing.cu:29 seeds with accumId + 10007), for every later pass of
- * this context (path tracing, HairMSNN frames and the adjoint's replay).
+ * this context (path tracing, HairMSNN frames and the adjoint).
  * Default 0 reproduces the reference's streams. No reference counterpart:
  * it lets a reference image and a test render use independent samples. */
 int hmsnn_set_seed_offset(hmsnn_ctx* ctx, int offset);
@@ -394,7 +394,7 @@ int hmsnn_save_exr(const char* path, const float* rgba, int width, int height);
 int hmsnn_exr_size(const char* path, int* width, int* height);
 int hmsnn_load_exr(const char* path, float* rgba_host, int width, int height);
 
-/* ---- differentiable appearance (path-replay adjoint) --------------------- */
+/* ---- differentiable appearance (path-wise adjoint) --------------------- */
 
 /* Sets the global hair roughness and scale tilt (the values parseScene reads,
  * scene.cpp:201-208; alpha in radians). */
@@ -403,7 +403,7 @@ int hmsnn_set_hair_params(hmsnn_ctx* ctx, float beta_m, float beta_n, float alph
  * width x height x 4 floats (w ignored): per-strand d/d sigma_a
  * (num_strands x 3, FP64, NULL to skip), d/d (beta_m, beta_n, alpha), and
  * optionally each pixel's share of the latter (width x height x 3 floats,
- * NULL to skip). Paths are replayed from the passes 0..spp-1 of the path
+ * NULL to skip). Paths are those of the passes 0..spp-1 of the path
  * tracer's streams (the image hmsnn_render_path_tracing(ctx, spp) makes);
  * sampled directions, sampling pdfs and Russian roulette are held fixed,
  * while f and the MIS weights are differentiated. No reference counterpart:
