@@ -216,8 +216,9 @@ int alloc_path_buffers(PathBuffers& pb, std::vector<void*>& allocs, size_t n, bo
   return kOk;
 }
 
-int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots) {
-  const int want = std::max(stream_slots(scene.width * scene.height), min_slots);
+int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots, bool rays_only) {
+  const int npx = scene.width * scene.height;
+  const int want = std::max(rays_only ? npx : stream_slots(npx, 1), min_slots);
   if (pb.ray_o && (!msnn_mode || pb_msnn) && pb_slots >= want) return kOk;
   free_path_buffers();
   const size_t n = (size_t)want;
@@ -225,7 +226,7 @@ int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots
   spill_levels = stack_levels();
   HM_TRY(alloc_path_buffers(pb, pb_allocs, n, msnn_mode, spill_levels, trace_blocks * kTraceBlock, stream, err));
   pb_msnn = msnn_mode;
-  const size_t f4 = sizeof(float4) * n;
+  const size_t f4 = sizeof(float4) * (size_t)npx;
   HM_TRY(dev_alloc((void**)&accum, f4, err));
   HM_TRY(dev_alloc((void**)&average, f4, err));
   HM_HIP(hipMemsetAsync(accum, 0, f4, stream), err);
@@ -237,7 +238,7 @@ int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots
 // Path-tracing buffers for flights 1 .. count - 1 (flight 0 is pb).
 int Context::ensure_flights(int count, std::string& err) {
   if (!acc_event) HM_HIP(hipEventCreateWithFlags(&acc_event, hipEventDisableTiming), err);
-  const int want = stream_slots(scene.width * scene.height);
+  const int want = stream_slots(scene.width * scene.height, kStreamGroups);
   for (int f = 1; f < count; ++f) {
     Flight& fl = extra[f - 1];
     if (!fl.stream) HM_HIP(hipStreamCreateWithFlags(&fl.stream, hipStreamNonBlocking), err);
@@ -757,6 +758,7 @@ int hmsnn_set_pass_concurrency(hmsnn_ctx* ctx, int passes_in_flight) {
   Context& c = ctx->c;
   (void)hipStreamSynchronize(c.stream);  // every flight's work is behind the context stream
   c.num_flights = passes_in_flight;
+  c.max_groups = std::min(passes_in_flight, kStreamGroups);
   return HMSNN_OK;
 }
 
@@ -791,7 +793,7 @@ namespace hm {
 // every group. The ring then holds the last (up to) 16 passes' radiance.
 int stream_groups(const Context& c, int passes) {
   const long long jobs = (long long)c.scene.width * c.scene.height * passes;
-  return jobs < kTwoGroupJobs ? 1 : std::max(1, std::min(c.num_flights, kStreamGroups));
+  return jobs < kTwoGroupJobs ? 1 : c.max_groups;
 }
 
 int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* avg, PassTimer* timer,
@@ -824,7 +826,7 @@ int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* a
   PassConfig cfg = c.pt_pass_config();
   cfg.accum_id = first_pass;
   cfg.timer = timer;
-  HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, stream_slots(n), acc, avg, c.stream_ring, c.stream_ctl,
+  HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, stream_slots(n, K), acc, avg, c.stream_ring, c.stream_ctl,
                        c.live_host, c.live_ev, err, tape));
   // the context stream waits for every group
   for (int g = 1; g < K; ++g) {
@@ -1025,7 +1027,7 @@ int hmsnn_trace_rays_dev(hmsnn_ctx* ctx, const float* rays, int n, int any_hit, 
   if (!ctx || n < 0 || (n > 0 && (!rays || !prim))) return fail(HMSNN_EINVAL, "hmsnn_trace_rays_dev: bad arguments");
   Context& c = ctx->c;
   std::string err;
-  int rc = c.ensure_path_buffers(false, err);
+  int rc = c.ensure_path_buffers(false, err, 0, true);
   if (rc) return fail(rc, err);
   rc = trace_rays(c.view, rays, n, any_hit, prim, t, u, c.pb.spill, c.pb.spill_stride, c.pb.spill_levels,
                   c.ray_blocks, nullptr, c.stream, err);

@@ -89,6 +89,7 @@ struct Context {
   // path-tracing passes in flight at once: flight 0 is (pb, stream)
   static constexpr int kMaxFlights = 4;
   int num_flights = 4;
+  int max_groups = 1;  // stream groups at most
   Flight extra[kMaxFlights - 1];
   hipEvent_t acc_event = nullptr;  // last accumulate issued (any flight)
   bool acc_pending = false;
@@ -113,9 +114,10 @@ struct Context {
 
   ~Context();
   int init(std::string& err);
-  // Path state for max(width * height, min_slots) slots; msnn_mode adds the
-  // training-path arrays.
-  int ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots = 0);
+  // Path state for at least a frame's and min_slots paths, and for a stream
+  // group's unless only rays are traced; msnn_mode adds the training-path
+  // arrays.
+  int ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots = 0, bool rays_only = false);
   int pb_slots = 0;
   void free_path_buffers();
   PassConfig pt_pass_config() const;

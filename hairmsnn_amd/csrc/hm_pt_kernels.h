@@ -165,12 +165,14 @@ inline int pt_jobs_bound(const PassConfig& cfg, int capacity) {
 
 // Passes the streaming schedule keeps in flight at most (its radiance ring).
 constexpr int kStreamRing = 16;
-// Stream groups at most, whatever hmsnn_set_pass_concurrency allows: two
-// groups' launches fill each other's tails, more only share the GPU's hardware
-// queues with whatever else the process runs (16 passes of the headline frame
-// took 62 to 75 ms with four, depending on which queues the streams got, 63
-// with two, 67 with one; a 640 x 363 frame of round curves 18.5 with three,
-// 17.1 with two). Calls of fewer jobs than kTwoGroupJobs run as one group: two
+// Stream groups: one, and two where the caller asks for concurrency
+// (hmsnn_set_pass_concurrency) and there are kTwoGroupJobs jobs. Two groups'
+// launches fill each other's tails where their streams have a hardware queue
+// each (16 passes of the headline frame 63 ms against 67, a 640 x 363 frame of
+// round curves 15.6 against 16.2), which depends on every stream the process
+// has made: in one that had rendered other scenes before, the same two groups
+// took 70 to 74 and 21 to 23 ms, and 256 x 256 at 16 passes 3.4 to 3.8 ms
+// against 2.5. More than two only share the queues. Below kTwoGroupJobs two
 // shorter wavefronts drain in as many launches each (128 x 128, 4 passes: 1.28
 // against 1.48 ms; 256 x 256, 16 passes: level).
 constexpr int kStreamGroups = 2;
@@ -200,9 +202,10 @@ struct StreamTape {
   VertexTape tape[kStreamGroups];
   const long long* count[kStreamGroups];
 };
-// Paths that a stream group's buffers hold for an image of npx pixels.
-inline int stream_slots(int npx) {
-  const long long share = kStreamPaths / kStreamGroups;
+// Paths that the buffers of one of K stream groups hold for an image of npx
+// pixels.
+inline int stream_slots(int npx, int K) {
+  const long long share = kStreamPaths / K;
   return (int)std::max<long long>(npx, std::min<long long>(share, (long long)kStreamRing * npx));
 }
 // Scheduler counters per stream group (64-bit).

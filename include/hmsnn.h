@@ -173,10 +173,11 @@ int hmsnn_set_strand_sigma_a(hmsnn_ctx* ctx, const float* sigma_host, int num_st
  * Default 0 reproduces the reference's streams. No reference counterpart:
  * it lets a reference image and a test render use independent samples. */
 int hmsnn_set_seed_offset(hmsnn_ctx* ctx, int offset);
-/* Concurrency of path tracing (1..4, default 4): with the per-pass schedule
- * the passes kept in flight at once, with the streaming schedule a limit on
- * the stream groups the pixels are dealt to (at most two are used); each has
- * its own path buffers and stream.
+/* Concurrency of path tracing (1..4): with the per-pass schedule the passes
+ * kept in flight at once (default 4), with the streaming schedule a limit on
+ * the stream groups the pixels are dealt to (default 1, at most two are used:
+ * worth a few per cent in a process with few other streams); each has its own
+ * path buffers and stream.
  * Accumulation stays in pass order, so the image does not depend on it. 1
  * runs everything on one stream (per-kernel timings of hmsnn_pt_time_passes
  * are then those of kernels running alone). No reference counterpart: the

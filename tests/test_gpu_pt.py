@@ -164,10 +164,11 @@ def test_streaming_schedule_equals_pass_schedule(gpu, name, groups, calls, size)
     assert np.isfinite(imgs["stream"]).all() and imgs["stream"][..., :3].mean() > 0
 
 
+@pytest.mark.parametrize("groups", [1, 2])
 @pytest.mark.parametrize("calls", [(15,), (16,), (3, 33)])
-def test_streaming_schedule_two_groups(gpu, calls):
+def test_streaming_schedule_two_groups(gpu, calls, groups):
     """Calls on both sides of the 2^20 jobs from which the streaming schedule
-    deals its pixels to two groups (128 x 513 has 1026 chunks of 64 pixels,
+    deals its pixels to two groups where it may (128 x 513 has 1026 chunks of 64 pixels,
     16 passes are the first call above), with the buffers of a small image
     holding every pass the ring allows: the per-pass schedule's image, bit for
     bit."""
@@ -176,6 +177,8 @@ def test_streaming_schedule_two_groups(gpu, calls):
     for sched in ("passes", "stream"):
         with gpu.Scene(json_text=cfg) as sc:
             sc.set_pt_schedule(sched)
+            if groups > 1:
+                sc.set_pass_concurrency(groups)
             sc.pt_reset()
             for n in calls:
                 sc.pt_passes(n)
