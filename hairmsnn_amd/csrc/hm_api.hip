@@ -804,7 +804,7 @@ int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* a
   const int K = stream_groups(c, passes);
   HM_TRY(c.ensure_flights(K, err));
   if (!c.live_host) {
-    HM_HIP(hipHostMalloc((void**)&c.live_host, 2 * Context::kMaxFlights * sizeof(int)), err);
+    HM_HIP(hipHostMalloc((void**)&c.live_host, 4 * Context::kMaxFlights * sizeof(long long)), err);
     for (hipEvent_t& e : c.live_ev) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
   }
   if (!c.stream_ring) {

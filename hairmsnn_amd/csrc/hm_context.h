@@ -97,7 +97,7 @@ struct Context {
   // path buffers), 1 one wavefront per pass with passes in flight
   int pt_schedule = 0;
   bool last_streamed = false;   // the last pt call used the streaming schedule
-  int* live_host = nullptr;     // pinned, 2 per group: live-path count polls
+  long long* live_host = nullptr;  // pinned, 4 per group: polls of the streaming schedule's progress
   float4* stream_ring = nullptr;  // streaming schedule: kStreamRing passes of radiance per pixel
   long long* stream_ctl = nullptr;  // streaming schedule: scheduler counters per group
   int last_ring_entry = 0;          // ring entry of the last streamed pass

@@ -929,9 +929,17 @@ int pt_run_pass(const SceneView& sc, PathBuffers& pb, const PassConfig& cfg, hip
 // group's shading overlaps another's traversal: group g owns the 64-pixel
 // chunks g, g + K, g + 2K, ... (balanced work, coherent camera rays within a
 // wave).
+// The plan sees the jobs finished by the iteration before, so a wavefront can
+// be empty while jobs remain: when the last paths of a fully issued window end
+// in the same iteration (small images start all the window's passes together,
+// and their longest paths end at the vertex limit), the next plan accumulates
+// the window and issues again. What tells that a group has drained is
+// therefore the plan's count of paths and jobs left, not the wavefront's
+// length.
 // ctl (64-bit, per group): two copies of the scheduler state, each [0] next
-// job, [1] passes accumulated, [3] vertex tape records of the wavefronts shaded
-// so far, [8 + r] finished jobs of ring entry r.
+// job, [1] passes accumulated, [2] paths of the new wavefront and jobs not
+// issued yet, [3] vertex tape records of the wavefronts shaded so far, [8 + r]
+// finished jobs of ring entry r.
 __global__ void k_stream_init(long long* ctl, int* counts) {
   const int i = threadIdx.x;
   if (i < kStreamCtl) ctl[i] = 0;
@@ -1002,6 +1010,7 @@ __global__ void k_stream_next_dense(SceneView sc, PathBuffers nb, const long lon
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     T[0] = job0 + n;
     T[1] = acc + k;
+    T[2] = cont + (long long)passes * cnt - job0;
     T[3] = S[3] + nb.counts[wave_count(nxt ^ 1)];
     for (int r = 0; r < kStreamRing; ++r) {
       const long long d = (r - acc % kStreamRing + kStreamRing) % kStreamRing;  // ring entry r holds pass acc + d
@@ -1057,13 +1066,13 @@ int stream_group_slots(int npx, int g, int K) {
 
 int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_t* streams, int K,
                   const PassConfig& cfg, int passes, int slots_cap, float4* accum, float4* average, float4* ring,
-                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err, StreamTape* tape) {
+                  long long* ctl, long long* live_host, hipEvent_t* live_ev, std::string& err, StreamTape* tape) {
   const int npx = sc.width * sc.height;
   if (passes <= 0 || npx <= 0 || K < 1) return passes <= 0 ? kOk : (err = "bad stream groups", kEInval);
   PassTimer* tm = cfg.timer;
 
   constexpr int kBatch = 8;  // even: each group's live queue is back at index 0 after a batch
-  std::vector<int> cur(K, 0), live(K, 0), calls(K, 0);
+  std::vector<int> cur(K, 0), live(K, 0), calls(K, 0), last_poll(K, -1);
   std::vector<long long> iters(K, 0);
   // paths in flight per group: what its buffers hold, but no more than the
   // jobs the ring lets start
@@ -1086,7 +1095,7 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
   HM_TRY(check_launch("stream start", err));
   // A path lives at most max_vertex + 1 iterations and every group holds at
   // least as many slots as pixels (slots >= cnt), so a group drains within
-  // passes x (max_vertex + 1) iterations; the live count is read one batch
+  // passes x (max_vertex + 1) iterations; the scheduler state is read one batch
   // late, which adds up to two batches. Past twice that bound the schedule is
   // reported as stuck.
   for (int g = 0; g < K; ++g) {
@@ -1147,18 +1156,21 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
       iters[g] += kBatch;
       HM_TRY(check_launch("stream iteration", err));
       const int s = 2 * g + (batch & 1);
-      HM_HIP(hipMemcpyAsync(&live_host[s], pb.counts + wave_count(cur[g]), sizeof(int), hipMemcpyDeviceToHost, st),
+      // passes accumulated, paths and jobs left
+      HM_HIP(hipMemcpyAsync(&live_host[2 * s], ctl + (size_t)g * kStreamCtl + kStreamHalf * (calls[g] & 1) + 1,
+                            2 * sizeof(long long), hipMemcpyDeviceToHost, st),
              err);
       HM_HIP(hipEventRecord(live_ev[s], st), err);
+      last_poll[g] = s;
     }
     if (!any) break;
     if (batch > 0) {
-      // the previous batch's counts, read while this batch runs
+      // the previous batch's state, read while this batch runs
       for (int g = 0; g < K; ++g) {
         if (!live[g]) continue;
         const int s = 2 * g + ((batch - 1) & 1);
         HM_HIP(hipEventSynchronize(live_ev[s]), err);
-        if (live_host[s] == 0) {
+        if (live_host[2 * s + 1] == 0) {
           live[g] = 0;  // drained: never an error, however late
           continue;
         }
@@ -1167,6 +1179,16 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
           return kEDevice;
         }
       }
+    }
+  }
+  // a drained group's last batch accumulated what was finished before it
+  for (int g = 0; g < K; ++g) {
+    if (last_poll[g] < 0) continue;
+    HM_HIP(hipEventSynchronize(live_ev[last_poll[g]]), err);
+    if (live_host[2 * last_poll[g]] != passes) {
+      err = "streaming schedule: " + std::to_string(live_host[2 * last_poll[g]]) + " of " + std::to_string(passes) +
+            " passes accumulated";
+      return kEDevice;
     }
   }
   if (tape)

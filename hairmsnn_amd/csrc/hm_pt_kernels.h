@@ -220,13 +220,14 @@ static_assert(8 + kStreamRing <= kStreamHalf && 2 * kStreamHalf <= kStreamCtl, "
 // once all its jobs are done. The pixels are split into K groups (64-pixel
 // chunks dealt round-robin, the last one possibly partial), group g on pbs[g]
 // and streams[g] with ctl +
-// g * kStreamCtl; live_host (pinned, 2K ints) and live_ev (2K events) poll the
-// live-path counts. slots_cap: paths that each group's buffers hold (at least
+// g * kStreamCtl; live_host (pinned, 4K words) and live_ev (2K events) poll the
+// groups' progress. slots_cap: paths that each group's buffers hold (at least
 // the image's pixels). A timer records group 0's launches. The last pass's
 // radiance is left in ring entry (passes - 1) % kStreamRing.
 int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_t* streams, int K,
                   const PassConfig& cfg, int passes, int slots_cap, float4* accum, float4* average, float4* ring,
-                  long long* ctl, int* live_host, hipEvent_t* live_ev, std::string& err, StreamTape* tape = nullptr);
+                  long long* ctl, long long* live_host, hipEvent_t* live_ev, std::string& err,
+                  StreamTape* tape = nullptr);
 // Pixels of stream group g of K over npx pixels, and the pixel of a group's
 // i-th pixel.
 int stream_group_slots(int npx, int g, int K);

@@ -186,6 +186,34 @@ def test_streaming_schedule_two_groups(gpu, calls, groups):
     np.testing.assert_array_equal(imgs["stream"], imgs["passes"])
 
 
+@pytest.mark.parametrize("name,size,path_v2,groups,calls", [("c1_curly.json", (256, 256), 40, 1, (20, 2)),
+                                                            ("c1_curly.json", (256, 256), 40, 2, (64, 2)),
+                                                            ("c1_curly.json", (128, 128), 2, 1, (96, 2)),
+                                                            ("c1_curly.json", (128, 128), 8, 1, (17, 64)),
+                                                            ("c0_hairball.json", (64, 64), 3, 1, (200, 1))])
+def test_streaming_schedule_longer_than_its_ring(gpu, name, size, path_v2, groups, calls):
+    """Calls of more passes than the radiance ring holds, on images small
+    enough that all the ring's passes start together: their last paths then end
+    in one iteration (at the vertex limit), which leaves the wavefront empty
+    while jobs remain. Every pass is traced all the same: the image, the last
+    pass and the image after a following call are the per-pass schedule's, bit
+    for bit. 256 x 256 at 64 passes is above the 2^20 jobs from which two
+    groups are used."""
+    cfg = scene_cfg(name, *size, path_v2=path_v2)
+    got = {}
+    with gpu.Scene(json_text=cfg) as sc:
+        sc.set_pass_concurrency(groups)
+        for sched in ("passes", "stream"):
+            sc.set_pt_schedule(sched)
+            sc.pt_reset()
+            got[sched] = []
+            for n in calls:
+                sc.pt_passes(n)
+                got[sched] += [sc.image(0).copy(), sc.last_pass().copy()]
+    for a, b in zip(got["stream"], got["passes"]):
+        np.testing.assert_array_equal(a, b)
+
+
 def test_exr_environment_equals_procedural(gpu, tmp_path):
     """lights.environment.exr (loadEnvTexture, model.cpp:158-180): the
     procedural C0 environment written to a ZIP-compressed FLOAT EXR renders
