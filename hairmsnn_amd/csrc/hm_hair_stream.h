@@ -33,13 +33,17 @@
 
 namespace hm {
 
-// 2^t from the hardware, the rounding of x * log2(e) added back.
+// 2^t from the hardware, the rounding of x * log2(e) added back (finite t: at
+// -inf the rounding would be a difference of infinities).
 HM_D float fast_exp(float x) {
   const float t = x * 1.44269504f;
   const float r = fmaf(x, 1.92596299e-8f, fmaf(x, 1.44269504f, -t));
   const float e = __builtin_amdgcn_exp2f(t);
   return fmaf(e, r * 0.693147181f, e);
 }
+// exp of -x that may be infinite or overflow in t: 0 from 104 on, as in FP32
+// (the maximum keeps a NaN).
+HM_D float fast_exp_down(float x) { return fast_exp(__builtin_elementwise_maximum(-x, -104.f)); }
 HM_D float fast_log(float x) {
   const float l = __builtin_amdgcn_logf(x);
   return fmaf(l, 0.693147181f, l * -1.90465433e-9f);
@@ -115,7 +119,7 @@ HM_D HairWo stream_prepare(const HairConsts& hc, V3 wo, float h, V3 sigma_a) {
   w.gamma_t = fast_asin(clampf(sin_gamma_t, -1.f, 1.f));
   const float fac = 2.f * fast_sqrt((1.f - sin_gamma_t) * (1.f + sin_gamma_t)) *
                     fast_rsq((1.f - sin_theta_t) * (1.f + sin_theta_t));
-  const V3 T = v3(fast_exp(-sigma_a.x * fac), fast_exp(-sigma_a.y * fac), fast_exp(-sigma_a.z * fac));
+  const V3 T = v3(fast_exp_down(sigma_a.x * fac), fast_exp_down(sigma_a.y * fac), fast_exp_down(sigma_a.z * fac));
   const float xd = 1.f - w.co * cos_gamma_o;
   const float xd2 = xd * xd;
   const float F = hc.f0 + (1.f - hc.f0) * (xd2 * xd2 * xd);
@@ -154,7 +158,7 @@ HM_D float stream_np(const HairConsts& hc, float phi, int p, float gamma_o, floa
   const float c = fmaf(-2.f * (float)p, gamma_t, 2.f * gamma_o);
   const float m = (float)p + 2.f * rintf((phi + c) * (0.5f / kPi) - 0.5f * (float)p);
   const float dphi = fmaf(-m, 3.14159274f, phi) + fmaf(m, 8.74227766e-8f, c);
-  const float e = fast_exp(-fabsf(dphi) * hc.inv_s);
+  const float e = fast_exp_down(fabsf(dphi) * hc.inv_s);
   const float d = 1.f + e;
   return e * (hc.inv_s * hc.trim_norm) * fast_rcp(d * d);
 }

@@ -126,3 +126,32 @@ def test_streams_at_the_edges_of_their_formulas(gpu, case, beta):
     assert np.quantile(np.linalg.norm(wi32 - wi64, axis=1)[same], 0.95) <= 2e-5
     e = np.abs(sp32[same] - sp64[same]) / sp64[same]
     assert np.median(e) <= tol
+
+
+@pytest.mark.parametrize("beta", [0.3, 0.08])
+def test_streams_with_opaque_fibres_and_draws_at_the_ends(gpu, beta):
+    """An absorption that is infinite, or overflows over the fibre's length,
+    transmits nothing, as in FP64; and draws of exactly 0 and 1 (the cdf at
+    beta 0.08 reaches 0 and 1 in FP32) sample the lobes' ends. Directions: the
+    azimuth is off by a rounding of pi at most (2^-22), the inclination's
+    sine and cosine products by four of 2^-24. Values: as in
+    test_streams_at_the_edges_of_their_formulas."""
+    q = bsdf_queries(258, seed=5)
+    q[:, 7] = np.resize(np.float32([np.inf, 1e38, 3e38, 100.0, 2000.0, 1e20]), 258)
+    q[::3, 8] = np.inf
+    q[::5, 7:10] = np.inf
+    u = uniforms(258, 4, 6)
+    u[:, 3] = np.resize(np.float32([0.0, 1.0, 2.0**-24]), 258)
+    u[::7, 1] = np.resize(np.float32([0.0, 1.0]), u[::7].shape[0])
+    prm = ol.hair_params(beta, beta, ALPHA_2DEG)
+    s = np.sqrt(np.pi / 8) * (0.265 * beta + 1.194 * beta**2)
+    v = 0.25 * (0.726 * beta + 0.812 * beta**2) ** 2
+    tol = 2.0**-23 * (3 * np.pi / s + 4 / v) + 1e-6
+    f32, p32 = gpu.hair_bsdf_eval(q, beta, beta, ALPHA_2DEG)
+    for g, o in zip((f32, p32), ol.hair_eval(q, prm, 0)):
+        assert np.all(np.isfinite(g)) and np.linalg.norm(g - o) <= tol * np.linalg.norm(o)
+    wi64, _, _, l64 = ol.hair_sample(q, u, prm, 0)
+    wi32, sf32, sp32, l32 = gpu.hair_bsdf_sample(q, u, beta, beta, ALPHA_2DEG)
+    assert np.all(np.isfinite(wi32)) and np.all(np.isfinite(sf32)) and np.all(np.isfinite(sp32))
+    np.testing.assert_array_equal(l32, l64)
+    assert np.abs(wi32 - wi64).max() <= 2.0**-22 * np.pi + 4 * 2.0**-24 + 1e-6
