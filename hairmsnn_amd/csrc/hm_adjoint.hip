@@ -288,7 +288,7 @@ int hmsnn_adjoint_render(hmsnn_ctx* ctx, int spp, const float* dl_dimg, double* 
   Context& c = ctx->c;
   if (!c.scene.has_hair) return fail(HMSNN_EINVAL, "scene has no hair");
   std::string err;
-  int rc = c.ensure_path_buffers(false, err);
+  int rc = c.ensure_image(err);
   if (rc) return fail(rc, err);
   const size_t npx = (size_t)c.scene.width * c.scene.height;
   const size_t ns = (size_t)c.hair.num_strands;

@@ -111,8 +111,7 @@ Context::~Context() {
   if (stream) (void)hipStreamSynchronize(stream);
   for (Flight& f : extra) {
     if (f.stream) (void)hipStreamSynchronize(f.stream);
-    for (void* p : f.allocs) dev_free(p);
-    f.allocs.clear();
+    f.release();
     if (f.stream) (void)hipStreamDestroy(f.stream);
     f.stream = nullptr;
   }
@@ -128,6 +127,8 @@ Context::~Context() {
   nrc_release(nrc);
   nrc = nullptr;
   free_path_buffers();
+  dev_free(accum);
+  dev_free(average);
   dev_free(scene_points);
   dev_free(seg_dev);
   dev_free(crv_dev);
@@ -146,9 +147,7 @@ void Context::free_path_buffers() {
   for (void* p : pb_allocs) dev_free(p);
   pb_allocs.clear();
   pb = PathBuffers{};
-  dev_free(accum);
-  dev_free(average);
-  accum = average = nullptr;
+  pb_slots = 0;
 }
 
 // Allocates one set of path buffers for n slots (recording every allocation
@@ -216,38 +215,48 @@ int alloc_path_buffers(PathBuffers& pb, std::vector<void*>& allocs, size_t n, bo
   return kOk;
 }
 
-int Context::ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots, bool rays_only) {
-  const int npx = scene.width * scene.height;
-  const int want = std::max(rays_only ? npx : stream_slots(npx, 1), min_slots);
-  if (pb.ray_o && (!msnn_mode || pb_msnn) && pb_slots >= want) return kOk;
-  free_path_buffers();
-  const size_t n = (size_t)want;
-  pb_slots = want;
-  spill_levels = stack_levels();
-  HM_TRY(alloc_path_buffers(pb, pb_allocs, n, msnn_mode, spill_levels, trace_blocks * kTraceBlock, stream, err));
-  pb_msnn = msnn_mode;
-  const size_t f4 = sizeof(float4) * (size_t)npx;
-  HM_TRY(dev_alloc((void**)&accum, f4, err));
-  HM_TRY(dev_alloc((void**)&average, f4, err));
-  HM_HIP(hipMemsetAsync(accum, 0, f4, stream), err);
-  HM_HIP(hipMemsetAsync(average, 0, f4, stream), err);
-  accum_id = 0;
+int Context::ensure_image(std::string& err) {
+  const size_t bytes = sizeof(float4) * (size_t)scene.width * scene.height;
+  for (float4** p : {&accum, &average}) {
+    if (*p) continue;
+    HM_TRY(dev_alloc((void**)p, bytes, err));
+    HM_HIP(hipMemsetAsync(*p, 0, bytes, stream), err);
+    accum_id = 0;
+  }
   return kOk;
 }
 
-// Path-tracing buffers for flights 1 .. count - 1 (flight 0 is pb).
-int Context::ensure_flights(int count, std::string& err) {
+int Context::ensure_path_buffers(std::string& err, int slots) {
+  HM_TRY(ensure_image(err));
+  const int want = std::max(scene.width * scene.height, slots);
+  if (pb_slots >= want) return kOk;
+  free_path_buffers();
+  const int rc = alloc_path_buffers(pb, pb_allocs, (size_t)want, false, stack_levels(), trace_blocks * kTraceBlock,
+                                    stream, err);
+  if (rc) {
+    free_path_buffers();  // a set with arrays missing must not look complete
+    return rc;
+  }
+  pb_slots = want;
+  return kOk;
+}
+
+// Path-tracing buffers of at least `slots` paths for flights 1 .. count - 1
+// (flight 0 is pb).
+int Context::ensure_flights(int count, int slots, std::string& err) {
   if (!acc_event) HM_HIP(hipEventCreateWithFlags(&acc_event, hipEventDisableTiming), err);
-  const int want = stream_slots(scene.width * scene.height, kStreamGroups);
   for (int f = 1; f < count; ++f) {
     Flight& fl = extra[f - 1];
     if (!fl.stream) HM_HIP(hipStreamCreateWithFlags(&fl.stream, hipStreamNonBlocking), err);
-    if (fl.slots >= want) continue;
-    for (void* p : fl.allocs) dev_free(p);
-    fl.allocs.clear();
-    HM_TRY(alloc_path_buffers(fl.pb, fl.allocs, (size_t)want, false, stack_levels(),
-                              trace_blocks * kTraceBlock, fl.stream, err));
-    fl.slots = want;
+    if (fl.slots >= slots) continue;
+    fl.release();
+    const int rc = alloc_path_buffers(fl.pb, fl.allocs, (size_t)slots, false, stack_levels(),
+                                      trace_blocks * kTraceBlock, fl.stream, err);
+    if (rc) {
+      fl.release();
+      return rc;
+    }
+    fl.slots = slots;
   }
   return kOk;
 }
@@ -787,30 +796,38 @@ int hmsnn_pt_reset(hmsnn_ctx* ctx) {
 
 namespace hm {
 
-// Streaming schedule: passes first_pass .. first_pass + passes - 1 of every
-// pixel accumulated into acc / avg (the context's image, or scratch buffers of
-// a caller that only wants the radiance ring); the context stream waits for
-// every group. The ring then holds the last (up to) 16 passes' radiance.
 int stream_groups(const Context& c, int passes) {
   const long long jobs = (long long)c.scene.width * c.scene.height * passes;
   return jobs < kTwoGroupJobs ? 1 : c.max_groups;
 }
 
+// What the streaming schedule needs for a call of `passes` passes; slots: the
+// paths that each group's buffers hold.
+static int stream_prepare(Context& c, int passes, int& slots, std::string& err) {
+  const int n = c.scene.width * c.scene.height, K = stream_groups(c, passes);
+  slots = stream_slots(n, K);
+  HM_TRY(c.ensure_path_buffers(err, slots));
+  HM_TRY(c.ensure_flights(K, slots, err));
+  for (hipEvent_t& e : c.live_ev)
+    if (!e) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
+  if (!c.live_host)
+    HM_HIP(hipHostMalloc((void**)&c.live_host, 4 * Context::kMaxFlights * sizeof(long long)), err);
+  if (!c.stream_ring) HM_TRY(dev_alloc((void**)&c.stream_ring, sizeof(float4) * kStreamRing * (size_t)n, err));
+  if (!c.stream_ctl)
+    HM_TRY(dev_alloc((void**)&c.stream_ctl, sizeof(long long) * kStreamCtl * Context::kMaxFlights, err));
+  return kOk;
+}
+
+// Streaming schedule: passes first_pass .. first_pass + passes - 1 of every
+// pixel accumulated into acc / avg (the context's image, or scratch buffers of
+// a caller that only wants the radiance ring); the context stream waits for
+// every group. The ring then holds the last (up to) 16 passes' radiance.
 int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* avg, PassTimer* timer,
                   std::string& err, StreamTape* tape) {
-  HM_TRY(c.ensure_path_buffers(false, err));
-  const int n = c.scene.width * c.scene.height;
   if (passes <= 0) return kOk;
   const int K = stream_groups(c, passes);
-  HM_TRY(c.ensure_flights(K, err));
-  if (!c.live_host) {
-    HM_HIP(hipHostMalloc((void**)&c.live_host, 4 * Context::kMaxFlights * sizeof(long long)), err);
-    for (hipEvent_t& e : c.live_ev) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
-  }
-  if (!c.stream_ring) {
-    HM_TRY(dev_alloc((void**)&c.stream_ring, sizeof(float4) * kStreamRing * (size_t)n, err));
-    HM_TRY(dev_alloc((void**)&c.stream_ctl, sizeof(long long) * kStreamCtl * Context::kMaxFlights, err));
-  }
+  int slots = 0;
+  HM_TRY(stream_prepare(c, passes, slots, err));
   // every group's stream starts after the work queued so far (including
   // the other schedule's last accumulation)
   if (c.acc_pending) HM_HIP(hipStreamWaitEvent(c.stream, c.acc_event, 0), err);
@@ -826,8 +843,8 @@ int stream_passes(Context& c, int first_pass, int passes, float4* acc, float4* a
   PassConfig cfg = c.pt_pass_config();
   cfg.accum_id = first_pass;
   cfg.timer = timer;
-  HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, stream_slots(n, K), acc, avg, c.stream_ring, c.stream_ctl,
-                       c.live_host, c.live_ev, err, tape));
+  HM_TRY(pt_run_stream(c.view, pbs, sts, K, cfg, passes, slots, acc, avg, c.stream_ring, c.stream_ctl, c.live_host,
+                       c.live_ev, err, tape));
   // the context stream waits for every group
   for (int g = 1; g < K; ++g) {
     HM_HIP(hipEventRecord(c.acc_event, sts[g]), err);
@@ -845,7 +862,7 @@ extern "C" {
 // through acc_event so they happen in pass order (the image is the one a
 // single stream makes), and the context stream waits for the last one.
 static int run_pt_passes(Context& c, int passes, std::string& err, PassTimer* timer = nullptr) {
-  HM_TRY(c.ensure_path_buffers(false, err));
+  HM_TRY(c.ensure_image(err));
   SceneView v = c.view;
   v.bvh.nodes = c.bvh.nodes_w;
   const int n = c.scene.width * c.scene.height;
@@ -859,7 +876,8 @@ static int run_pt_passes(Context& c, int passes, std::string& err, PassTimer* ti
   }
   c.last_streamed = false;
   const int K = std::max(1, std::min(c.num_flights, Context::kMaxFlights));
-  HM_TRY(c.ensure_flights(K, err));
+  HM_TRY(c.ensure_path_buffers(err));
+  HM_TRY(c.ensure_flights(K, n, err));
   hipEvent_t start = nullptr;
   HM_HIP(hipEventCreateWithFlags(&start, hipEventDisableTiming), err);
   HM_HIP(hipEventRecord(start, c.stream), err);
@@ -952,7 +970,7 @@ int hmsnn_pt_trace_stats(hmsnn_ctx* ctx, int passes, double out[6]) {
   if (!ctx || passes <= 0 || !out) return fail(HMSNN_EINVAL, "hmsnn_pt_trace_stats: bad arguments");
   Context& c = ctx->c;
   std::string err;
-  int rc = c.ensure_path_buffers(false, err);
+  int rc = c.ensure_path_buffers(err);
   if (rc) return fail(rc, err);
   hipError_t e = hipMemsetAsync(c.stats_dev, 0, sizeof(unsigned long long) * 8, c.stream);
   if (e != hipSuccess) return fail(HMSNN_EDEVICE, hipGetErrorString(e));
@@ -980,7 +998,8 @@ int hmsnn_pt_time_passes(hmsnn_ctx* ctx, int passes, double out[5]) {
   if (!ctx || passes <= 0 || !out) return fail(HMSNN_EINVAL, "hmsnn_pt_time_passes: bad arguments");
   Context& c = ctx->c;
   std::string err;
-  int rc = c.ensure_path_buffers(false, err);
+  int slots = 0;  // (allocations stay out of the times)
+  int rc = c.pt_schedule == 0 ? stream_prepare(c, passes, slots, err) : c.ensure_path_buffers(err);
   if (rc) return fail(rc, err);
   // records per vertex iteration: extend, shade, shadow (+ finish when streaming)
   const int per_pass = 4 * (c.scene.path_v2 + 1);
@@ -1027,7 +1046,7 @@ int hmsnn_trace_rays_dev(hmsnn_ctx* ctx, const float* rays, int n, int any_hit, 
   if (!ctx || n < 0 || (n > 0 && (!rays || !prim))) return fail(HMSNN_EINVAL, "hmsnn_trace_rays_dev: bad arguments");
   Context& c = ctx->c;
   std::string err;
-  int rc = c.ensure_path_buffers(false, err, 0, true);
+  int rc = c.ensure_path_buffers(err);
   if (rc) return fail(rc, err);
   rc = trace_rays(c.view, rays, n, any_hit, prim, t, u, c.pb.spill, c.pb.spill_stride, c.pb.spill_levels,
                   c.ray_blocks, nullptr, c.stream, err);

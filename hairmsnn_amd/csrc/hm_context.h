@@ -27,6 +27,12 @@ struct Flight {
   PathBuffers pb{};
   std::vector<void*> allocs;
   int slots = 0;
+  void release() {
+    for (void* p : allocs) dev_free(p);
+    allocs.clear();
+    pb = PathBuffers{};
+    slots = 0;
+  }
 };
 
 // One set of path buffers for n slots (msnn_mode adds the training-path
@@ -74,14 +80,13 @@ struct Context {
   // path-tracer state
   PathBuffers pb{};
   std::vector<void*> pb_allocs;
-  bool pb_msnn = false;
+  int pb_slots = 0;             // paths that pb holds (0: not allocated)
   float4* accum = nullptr;
   float4* average = nullptr;
   int accum_id = 0;
   int seed_offset = 0;  // hmsnn_set_seed_offset
   int trace_blocks = 2048;  // largest traversal grid: stack spill is sized for it
   int ray_blocks = 1024;    // grid of the ray streams (kRayBlocksPerCu per CU)
-  int spill_levels = 0;
   unsigned long long* stats_dev = nullptr;
 
   MsnnState* msnn = nullptr;
@@ -105,7 +110,7 @@ struct Context {
   // vertex tape of the adjoint, grown on demand
   std::vector<void*> tape_allocs;
   VertexTape tape{};
-  int ensure_flights(int count, std::string& err);
+  int ensure_flights(int count, int slots, std::string& err);
   PathBuffers& flight_pb(int f) { return f == 0 ? pb : extra[f - 1].pb; }
   hipStream_t flight_stream(int f) { return f == 0 ? stream : extra[f - 1].stream; }
   // HairMSNN scene samples on the hair (3 floats each), made once per scene
@@ -114,11 +119,10 @@ struct Context {
 
   ~Context();
   int init(std::string& err);
-  // Path state for at least a frame's and min_slots paths, and for a stream
-  // group's unless only rays are traced; msnn_mode adds the training-path
-  // arrays.
-  int ensure_path_buffers(bool msnn_mode, std::string& err, int min_slots = 0, bool rays_only = false);
-  int pb_slots = 0;
+  // The image (running sum and mean), cleared when it is made.
+  int ensure_image(std::string& err);
+  // The image, and path state for at least a frame's and `slots` paths.
+  int ensure_path_buffers(std::string& err, int slots = 0);
   void free_path_buffers();
   PassConfig pt_pass_config() const;
   // global stack-spill levels beyond the LDS part for the deepest tree traversed

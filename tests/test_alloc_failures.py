@@ -1,0 +1,77 @@
+"""What the contexts do when the device has no memory left, on the CPU: the
+library runs on tests/fake_hip.c (host memory, launches that do nothing), which
+fails allocations on request. The script runs in a process of its own."""
+import json
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parent.parent
+
+PRELUDE = '''
+import ctypes as C, json, sys
+fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # before the library: its symbols are found first
+fake.fake_bytes.restype = C.c_size_t
+fake.fake_limit.argtypes = [C.c_size_t]
+fake.fake_live.restype = C.c_long
+sys.path.insert(0, sys.argv[2])
+import hairmsnn_amd as hm
+from hairmsnn_amd._lib import load
+lib = load()
+cfg = json.load(open(sys.argv[2] + "/hairmsnn_amd/scenes/c0_hairball.json"))
+cfg["integrator"].update(width=16, height=8)
+cfg["hair"]["procedural"].update(strands=1, segments=1)  # a tree of one leaf needs no kernel's output
+def scene(w=16, h=8, **hair):
+    cfg["integrator"].update(width=w, height=h)
+    return hm.Scene(json_text=cfg)
+def call(f, *a):
+    try:
+        f(*a)
+        return ""
+    except hm._lib.HmsnnError as e:
+        return str(e)
+'''
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    so = tmp_path_factory.mktemp("fake") / "libfakehip.so"
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", str(so), str(ROOT / "tests" / "fake_hip.c")], check=True)
+
+    def run(script: str):
+        r = subprocess.run([sys.executable, "-c", PRELUDE + script, str(so), str(ROOT)], capture_output=True, text=True,
+                           timeout=300)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return json.loads(r.stdout.strip().splitlines()[-1])
+    return run
+
+
+@pytest.mark.parametrize("entry", ["trace_stats", "pt_passes"])
+def test_failed_allocation_leaves_no_partial_buffers(fake, entry):
+    """Every allocation of a first render fails in turn: the call reports it,
+    and the same call afterwards makes everything that was missing (a set of
+    path buffers with null arrays would fault in the kernels). The launches do
+    nothing here, so a streamed call ends by reporting that no pass was
+    accumulated."""
+    out = fake(f'''
+done = "" if "{entry}" == "trace_stats" else "0 of 1 passes accumulated"
+base = scene(); before = fake.fake_live(); e = call(base.{entry}, 1); whole = fake.fake_live() - before
+assert (done in e) if done else not e, e
+base.close()
+bad = []
+for k in range(whole):
+    sc = scene(); before = fake.fake_live()
+    fake.fake_fail_after(k)
+    first = call(sc.{entry}, 1)
+    fake.fake_fail_after(-1)
+    again = call(sc.{entry}, 1)
+    got = fake.fake_live() - before
+    if "ENOMEM" not in first or ((done not in again) if done else again) or got != whole: bad.append([k, first, again, got])
+    sc.close()
+print(json.dumps(dict(whole=whole, bad=bad, left=fake.fake_live())))
+''')
+    assert out["whole"] > 40
+    assert out["bad"] == []
+    assert out["left"] == 0
