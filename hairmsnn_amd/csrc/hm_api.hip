@@ -802,12 +802,22 @@ int stream_groups(const Context& c, int passes) {
 }
 
 // What the streaming schedule needs for a call of `passes` passes; slots: the
-// paths that each group's buffers hold.
+// paths that each group's buffers hold. Without the memory for as many as the
+// schedule would use, this context halves them, down to a frame's, for good.
 static int stream_prepare(Context& c, int passes, int& slots, std::string& err) {
   const int n = c.scene.width * c.scene.height, K = stream_groups(c, passes);
-  slots = stream_slots(n, K);
-  HM_TRY(c.ensure_path_buffers(err, slots));
-  HM_TRY(c.ensure_flights(K, slots, err));
+  for (;;) {
+    slots = std::min(stream_slots(n, K, passes), c.slots_limit);
+    int rc = c.ensure_path_buffers(err, slots);
+    if (!rc) rc = c.ensure_flights(K, slots, err);
+    if (!rc) break;
+    if (rc != kENoMem || slots <= n) return rc;
+    c.slots_limit = std::max(n, slots / 2);
+    c.free_path_buffers();
+    for (Flight& fl : c.extra) fl.release();
+    err.clear();
+    (void)hipGetLastError();
+  }
   for (hipEvent_t& e : c.live_ev)
     if (!e) HM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming), err);
   if (!c.live_host)

@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <climits>
 #include <memory>
 #include <string>
 #include <vector>
@@ -81,6 +82,7 @@ struct Context {
   PathBuffers pb{};
   std::vector<void*> pb_allocs;
   int pb_slots = 0;             // paths that pb holds (0: not allocated)
+  int slots_limit = INT_MAX;    // paths of a stream group's buffers at most (memory was short)
   float4* accum = nullptr;
   float4* average = nullptr;
   int accum_id = 0;

@@ -202,11 +202,11 @@ struct StreamTape {
   VertexTape tape[kStreamGroups];
   const long long* count[kStreamGroups];
 };
-// Paths that the buffers of one of K stream groups hold for an image of npx
-// pixels.
-inline int stream_slots(int npx, int K) {
+// Paths that the buffers of one of K stream groups hold for `passes` passes of
+// an image of npx pixels.
+inline int stream_slots(int npx, int K, int passes) {
   const long long share = kStreamPaths / K;
-  return (int)std::max<long long>(npx, std::min<long long>(share, (long long)kStreamRing * npx));
+  return (int)std::max<long long>(npx, std::min<long long>(share, (long long)std::min(kStreamRing, passes) * npx));
 }
 // Scheduler counters per stream group (64-bit).
 constexpr int kStreamCtl = 64;

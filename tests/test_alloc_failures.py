@@ -75,3 +75,31 @@ print(json.dumps(dict(whole=whole, bad=bad, left=fake.fake_live())))
     assert out["whole"] > 40
     assert out["bad"] == []
     assert out["left"] == 0
+
+
+def test_path_buffers_follow_the_call_and_the_memory(fake):
+    """A call of one pass makes buffers for a frame's paths, not for the ring's
+    16 passes, in either schedule; a longer call grows them; and where memory
+    is short it takes fewer paths (half as many, down to a frame's) instead of
+    failing. Per path the buffers are 300 to 400 bytes, the ring and the image
+    288 bytes a pixel."""
+    out = fake('''
+n = 256 * 128
+def used(sc, passes):
+    e = call(sc.pt_passes, passes)
+    assert "of %d passes accumulated" % passes in e, e
+    return (fake.fake_bytes() - base) / n
+r = {}
+sc = scene(256, 128); base = fake.fake_bytes(); r["one"] = used(sc, 1); r["all"] = used(sc, 40); r["again"] = used(sc, 1); sc.close()
+sc = scene(256, 128); base = fake.fake_bytes(); sc.set_pt_schedule("passes"); sc.set_pass_concurrency(1); sc.pt_passes(1)
+r["passes"] = (fake.fake_bytes() - base) / n; sc.close()
+sc = scene(256, 128); base = fake.fake_bytes(); sc.trace_stats(1); spill = fake.fake_bytes() - base
+fake.fake_limit(fake.fake_bytes() + n * (288 + 400 * 5)); r["short"] = used(sc, 16); fake.fake_limit(0); r["kept"] = used(sc, 16); sc.close()
+r["left"] = fake.fake_live()
+print(json.dumps(r))
+''')
+    print(out)
+    assert out["left"] == 0
+    assert out["one"] < 288 + 400 + 400 and out["passes"] < 32 + 400 + 400
+    assert out["all"] > out["one"] + 15 * 300 and out["again"] == out["all"]
+    assert out["one"] < out["short"] < out["all"] / 2 and out["kept"] == out["short"]

@@ -190,12 +190,13 @@ def test_streaming_schedule_two_groups(gpu, calls, groups):
                                                             ("c1_curly.json", (256, 256), 40, 2, (64, 2)),
                                                             ("c1_curly.json", (128, 128), 2, 1, (96, 2)),
                                                             ("c1_curly.json", (128, 128), 8, 1, (17, 64)),
-                                                            ("c0_hairball.json", (64, 64), 3, 1, (200, 1))])
+                                                            ("c0_hairball.json", (64, 64), 3, 1, (200, 1)),
+                                                            ("c0_hairball.json", (64, 64), 40, 1, (1, 3, 40))])
 def test_streaming_schedule_longer_than_its_ring(gpu, name, size, path_v2, groups, calls):
     """Calls of more passes than the radiance ring holds, on images small
     enough that all the ring's passes start together: their last paths then end
     in one iteration (at the vertex limit), which leaves the wavefront empty
-    while jobs remain. Every pass is traced all the same: the image, the last
+    while jobs remain. And calls that grow the path buffers between them. Every pass is traced all the same: the image, the last
     pass and the image after a following call are the per-pass schedule's, bit
     for bit. 256 x 256 at 64 passes is above the 2^20 jobs from which two
     groups are used."""
