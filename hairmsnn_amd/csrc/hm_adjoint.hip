@@ -24,6 +24,9 @@
 // segments. The tape is sequential memory, 2 GB there, on a GPU of 288 GB.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <cmath>
+
 #include "../../include/hmsnn.h"
 #include "hm_api_util.h"
 #include "hm_context.h"
@@ -183,17 +186,29 @@ __global__ void __launch_bounds__(256, 2) k_adjoint(SceneView sc, AdjArgs a, Ver
 }
 
 // Records a path is expected to leave (its hair vertices and its last, missed
-// ray); a run that leaves more is repeated with a larger tape. Passes per run:
-// as many as a tape of kTapeBytes is expected to hold.
-constexpr int kTapePerPath = 10;
+// ray): what the context's last run left and an eighth more (tape_per_path), at
+// least kTapePerPath. A run that leaves more than its tape holds is repeated
+// with a larger one, or, where that would pass kTapeBytes, as two runs of half
+// the passes; only a single pass may take more, and gives the tape back when
+// the call ends.
+constexpr double kTapePerPath = 10.0;
 constexpr size_t kTapeBytes = (size_t)8 << 30;
+
+void tape_release(Context& c) {
+  for (void* p : c.tape_allocs) dev_free(p);
+  c.tape_allocs.clear();
+  c.tape = VertexTape{};
+}
+
+// Records for `paths` paths.
+long long tape_records(const Context& c, long long paths) {
+  return (long long)std::ceil(std::max(kTapePerPath, c.tape_per_path) * (double)paths) + 64;
+}
 
 // Makes the context's tape hold at least `records`.
 int tape_ensure(Context& c, long long records, std::string& err) {
   if (c.tape.cap >= records) return kOk;
-  for (void* p : c.tape_allocs) dev_free(p);
-  c.tape_allocs.clear();
-  c.tape = VertexTape{};
+  tape_release(c);
   const size_t n = (size_t)records;
   auto A = [&](void** p, size_t bytes) -> int {
     HM_TRY(dev_alloc(p, bytes, err));
@@ -226,9 +241,11 @@ VertexTape tape_share(const VertexTape& t, int g, int K) {
 int adjoint_passes(Context& c, const AdjArgs& a, int p0, int np, float4* tmp_acc, std::string& err) {
   const size_t npx = (size_t)c.scene.width * c.scene.height;
   const int K = stream_groups(c, np);
-  long long want = kTapePerPath * (long long)npx * np + 64;
+  const long long paths = (long long)npx * np;
+  long long want = tape_records(c, paths);
   for (;;) {
-    const int rc = tape_ensure(c, want, err);
+    const bool fits = np == 1 || (size_t)want * kTapeRecordBytes <= kTapeBytes;
+    const int rc = fits ? tape_ensure(c, want, err) : kENoMem;
     if (rc && np > 1) {  // no room: half the passes at a time
       err.clear();
       (void)hipGetLastError();
@@ -245,6 +262,7 @@ int adjoint_passes(Context& c, const AdjArgs& a, int p0, int np, float4* tmp_acc
     HM_HIP(hipStreamSynchronize(c.stream), err);
     long long most = 0;
     for (int g = 0; g < K; ++g) most = std::max(most, count[g]);
+    c.tape_per_path = 1.125 * (double)(K * most) / (double)paths;
     if (most > st.tape[0].cap) {
       want = K * (most + most / 8);
       continue;
@@ -333,12 +351,17 @@ int hmsnn_adjoint_render(hmsnn_ctx* ctx, int spp, const float* dl_dimg, double* 
   a.g_px = d_px;
   float4* tmp_acc = nullptr;
   rc = dev_alloc((void**)&tmp_acc, 2 * sizeof(float4) * (size_t)npx, err);
-  const size_t pass_bytes = (size_t)kTapePerPath * kTapeRecordBytes * npx;
-  const int chunk = (int)std::max<size_t>(1, std::min<size_t>(kStreamRing, kTapeBytes / pass_bytes));
-  for (int p0 = 0; !rc && p0 < spp; p0 += chunk)
-    rc = adjoint_passes(c, a, p0, std::min(chunk, spp - p0), tmp_acc, err);
+  for (int p0 = 0; !rc && p0 < spp;) {
+    // as many passes as a tape of kTapeBytes is expected to hold
+    const size_t pass_bytes = (size_t)tape_records(c, (long long)npx) * kTapeRecordBytes;
+    const int chunk = (int)std::max<size_t>(1, std::min<size_t>(kStreamRing, kTapeBytes / pass_bytes));
+    const int np = std::min(chunk, spp - p0);
+    rc = adjoint_passes(c, a, p0, np, tmp_acc, err);
+    p0 += np;
+  }
   (void)hipStreamSynchronize(c.stream);
   dev_free(tmp_acc);
+  if ((size_t)c.tape.cap * kTapeRecordBytes > kTapeBytes) tape_release(c);
   if (!rc) {
     double gg[4];
     e = hipMemcpyAsync(gg, d_gg, sizeof(gg), hipMemcpyDeviceToHost, c.stream);

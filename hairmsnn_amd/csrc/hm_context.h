@@ -112,6 +112,7 @@ struct Context {
   // vertex tape of the adjoint, grown on demand
   std::vector<void*> tape_allocs;
   VertexTape tape{};
+  double tape_per_path = 0.0;  // records per path the last run left, and an eighth
   int ensure_flights(int count, int slots, std::string& err);
   PathBuffers& flight_pb(int f) { return f == 0 ? pb : extra[f - 1].pb; }
   hipStream_t flight_stream(int f) { return f == 0 ? stream : extra[f - 1].stream; }

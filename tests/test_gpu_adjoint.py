@@ -259,17 +259,23 @@ def test_c3_on_c1_geometry_central_differences(gpu):
     assert bad <= 2
 
 
-def test_long_paths_outgrow_the_first_tape(gpu):
-    """Lossless hair seen from inside: the paths leave more vertices than the
-    vertex tape is first sized for (10 per path), so the first call repeats its
-    trace with a larger tape. Its gradients are the sums of the passes' own
-    (seed offsets 0..5, on the grown tape). Bound: the same FP32 terms summed in
-    another order, about 3e5 of them with 2^-24 each, random signs."""
+def inside_lossless_cfg(w, h):
+    """Lossless hair seen from inside: more vertices a path than the vertex tape
+    is first sized for (10)."""
     cfg = json.loads((SCENES / "c0_hairball.json").read_text())
-    cfg["integrator"].update({"width": 64, "height": 64})
+    cfg["integrator"].update({"width": w, "height": h})
     cfg["hair"]["sigma_a"] = [0.0, 0.0, 0.0]
     cfg["hair"]["procedural"].update({"strands": 40_000, "radius": 0.02})
     cfg["camera"].update({"from": [0.0, -1.2, 0.0], "to": [0.0, -3.0, 0.0]})
+    return cfg
+
+
+def test_long_paths_outgrow_the_first_tape(gpu):
+    """The paths leave more vertices than the vertex tape is first sized for, so
+    the first call repeats its trace with a larger tape. Its gradients are the sums of the passes' own
+    (seed offsets 0..5, on the grown tape). Bound: the same FP32 terms summed in
+    another order, about 3e5 of them with 2^-24 each, random signs."""
+    cfg = inside_lossless_cfg(64, 64)
     rng = np.random.default_rng(3)
     d = rng.normal(size=(64, 64, 3)).astype(np.float32)
     with gpu.Scene(json_text=cfg) as sc:
@@ -283,3 +289,55 @@ def test_long_paths_outgrow_the_first_tape(gpu):
     for whole, parts in ((gs, [x[0] for x in one]), (gg, [x[1] for x in one]), (gp, [x[2] for x in one])):
         tot = np.sum([p.astype(np.float64) for p in parts], axis=0)
         assert np.linalg.norm(whole - tot) <= 3e-5 * np.linalg.norm(tot)
+
+
+def test_tape_stays_within_its_bound(gpu):
+    """Sixteen passes whose tape would take more than 8 GiB (1024 x 512, over 15
+    records of 81 bytes a path) run as fewer passes at a time: the context keeps
+    8 GiB of tape and its path buffers (400 bytes for each of 4M paths) and ring
+    at most, and the per-strand gradients are the sums of the passes' own.
+    Bound: FP64 sums of the same FP32 terms, each term's own rounding (2^-24)
+    the same on both sides; the two scalings of dL/dI round differently
+    (2^-24)."""
+    import ctypes
+
+    def free_bytes():
+        f, t = ctypes.c_size_t(), ctypes.c_size_t()
+        assert gpu._lib.load().hipMemGetInfo(ctypes.byref(f), ctypes.byref(t)) == 0  # of the library's HIP runtime
+        return f.value
+
+    w, h, spp = 1024, 512, 16
+    rng = np.random.default_rng(4)
+    d = rng.normal(size=(h, w, 3)).astype(np.float32)
+    with gpu.Scene(json_text=inside_lossless_cfg(w, h)) as sc:
+        rays = sc.trace_stats(1)["closest_rays"] / (w * h)
+        assert rays * w * h * spp * 81 > 9 << 30, rays
+        free = free_bytes()
+        gs, gg = sc.adjoint(d, spp)
+        kept = free - free_bytes()
+        tot = np.zeros_like(gs)
+        for k in range(spp):
+            sc.set_seed_offset(k)
+            tot += sc.adjoint(d / spp, 1)[0]
+    print(f"{rays:.1f} rays a path, {kept / 2**30:.2f} GiB kept")
+    assert kept <= (8 << 30) + (4 << 20) * 400 + w * h * 16 * 20 + (64 << 20)
+    assert np.linalg.norm(gs - tot) <= 1e-6 * np.linalg.norm(tot) and np.isfinite(gg).all()
+
+
+def test_two_stream_groups_give_the_same_gradients(gpu):
+    """At 2^20 paths the tracer may deal the pixels to two groups, each with its
+    half of the tape, which the first call outgrows: the gradients are the one
+    group's. Bounds: per strand the same FP32 terms in FP64 sums (1e-12, the
+    order alone); globals and pixels FP32 sums in another order (as in
+    test_long_paths_outgrow_the_first_tape)."""
+    cfg = inside_lossless_cfg(256, 256)
+    rng = np.random.default_rng(5)
+    d = rng.normal(size=(256, 256, 3)).astype(np.float32)
+    got = []
+    for groups in (1, 2):
+        with gpu.Scene(json_text=cfg) as sc:
+            sc.set_pass_concurrency(groups)
+            got.append([sc.adjoint(d, 16, per_pixel=True), sc.adjoint(d, 16, per_pixel=True)])
+    for call in (0, 1):
+        for one, two, tol in zip(got[0][call], got[1][call], (1e-12, 3e-5, 3e-5)):
+            assert np.linalg.norm(two.astype(np.float64) - one) <= tol * np.linalg.norm(one)
