@@ -837,7 +837,7 @@ int hmsnn_msnn_save_weights(hmsnn_ctx* ctx, const char* path) {
 int hmsnn_msnn_get_image(hmsnn_ctx* ctx, int which, float* rgba) {
   if (!ctx || !rgba || which < 0 || which > 2) return fail(HMSNN_EINVAL, "hmsnn_msnn_get_image: bad arguments");
   Context& c = ctx->c;
-  if (!c.msnn) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
+  if (!c.msnn || !c.msnn->ready) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
   // which: 0 final, 1 short path, 2 network
   const int slot = which == 0 ? 2 : (which == 1 ? 0 : 1);
   const size_t bytes = sizeof(float4) * (size_t)c.scene.width * c.scene.height;
@@ -861,7 +861,7 @@ int hmsnn_msnn_get_buffer(hmsnn_ctx* ctx, int which, void* host, size_t bytes) {
   if (!ctx || !host) return fail(HMSNN_EINVAL, "hmsnn_msnn_get_buffer: bad arguments");
   Context& c = ctx->c;
   MsnnState* m = c.msnn;
-  if (!m) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
+  if (!m || !m->ready) return fail(HMSNN_EINVAL, "call hmsnn_msnn_begin first");
   if (m->frame == 0) return fail(HMSNN_EINVAL, "no frame rendered yet");
   const size_t npx = (size_t)c.scene.width * c.scene.height, nt = (size_t)m->n_train;
   const int f = m->frame - 1, B = m->warm_batch;

@@ -536,7 +536,7 @@ int hmsnn_nrc_frames(hmsnn_ctx* ctx, int frames, hmsnn_nrc_stats* stats) {
 int hmsnn_nrc_get_image(hmsnn_ctx* ctx, float* rgba) {
   if (!ctx || !rgba) return fail(HMSNN_EINVAL, "hmsnn_nrc_get_image: bad arguments");
   Context& c = ctx->c;
-  if (!c.nrc) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
+  if (!c.nrc || !c.nrc->ready) return fail(HMSNN_EINVAL, "call hmsnn_nrc_begin first");
   const size_t bytes = sizeof(float4) * (size_t)c.scene.width * c.scene.height;
   hipError_t e = hipMemcpyAsync(rgba, c.nrc->avg, bytes, hipMemcpyDeviceToHost, c.stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c.stream);

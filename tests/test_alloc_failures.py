@@ -1,5 +1,5 @@
-"""What the contexts do when the device has no memory left, on the CPU: the
-library runs on tests/fake_hip.c (host memory, launches that do nothing), which
+"""What the contexts do when the device has no memory left, and after a begin
+that failed, on the CPU: the library runs on tests/fake_hip.c (host memory, launches that do nothing), which
 fails allocations on request. The script runs in a process of its own."""
 import json
 import subprocess
@@ -103,3 +103,25 @@ print(json.dumps(r))
     assert out["one"] < 288 + 400 + 400 and out["passes"] < 32 + 400 + 400
     assert out["all"] > out["one"] + 15 * 300 and out["again"] == out["all"]
     assert out["one"] < out["short"] < out["all"] / 2 and out["kept"] == out["short"]
+
+
+@pytest.mark.parametrize("kind", ["msnn", "nrc"])
+def test_failed_begin_shows_no_earlier_image(fake, kind):
+    """The renderers keep their buffers from one begin to the next. A begin that
+    fails (the weight file is gone) refuses the image afterwards, as on a new
+    context, instead of returning the earlier run's; the next good one works."""
+    begin = "sc.msnn_begin(1)" if kind == "msnn" else "sc.nrc_begin()"
+    out = fake(f'''
+import os, tempfile
+w = os.path.join(tempfile.mkdtemp(), "w.json")
+sc = scene(); {begin}; sc.{kind}_save_weights(w); sc.close()
+cfg["tcnn"] = {{"config": "unused.json", "init_train": False, "init_weights": w}}
+sc = scene(); {begin}; first = call(sc.{kind}_image)
+os.rename(w, w + "x")
+bad = call(lambda: {begin}); image = call(sc.{kind}_image)
+os.rename(w + "x", w); {begin}; last = call(sc.{kind}_image); sc.close()
+print(json.dumps(dict(first=first, bad=bad, image=image, last=last, left=fake.fake_live())))
+''')
+    print(out)
+    assert not out["first"] and not out["last"] and out["left"] == 0
+    assert "EIO" in out["bad"] and "EINVAL" in out["image"]
