@@ -138,7 +138,6 @@ struct TraceStack {
   // Whether every active lane has room for three more entries in LDS (and
   // none in memory), decided for the whole wave.
   HM_D bool room3() const { return __ballot(off >= kLevel * (kStackLds - 2)) == 0; }
-  HM_D bool in_lds() const { return __ballot(off >= kLevel * (kStackLds + 1)) == 0; }
   // Writes v to the next entry and keeps it if `keep` (room3 holds).
   HM_D void put(int v, bool keep) {
     *at(off) = v;
@@ -337,92 +336,27 @@ HM_D void closest_leaf(const BvhView& bvh, const RayInv& r, TraceStack& st, Clos
   if (!s.cur) s.cur = st.empty() ? kNone : st.pop();
 }
 
-template <bool kCount, class Leaf = SegLeaf>
+// A whole query by one lane: the closest hit before (best_t, best_id), or, with
+// `first`, the first one found.
+template <bool kCount, class Leaf>
 HM_D void trace_closest(const BvhView& bvh, const RayInv& r, TraceStack& st, float& best_t, int& best_id,
-                        float& best_u, TraceCounters& cnt, const Leaf& leaf_test = Leaf{}) {
+                        float& best_u, bool first, TraceCounters& cnt, const Leaf& leaf_test) {
   ClosestState s;
   s.best_t = best_t;
   s.best_id = best_id;
   s.best_u = best_u;
   closest_begin(bvh, st, s);
   for (int left = trace_cap(bvh); s.cur != kNone && left > 0; --left) {
-    if (s.cur < 0) closest_leaf<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
-    else closest_node<kCount>(bvh, r, st, s, cnt);
+    if (s.cur < 0) {
+      closest_leaf<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
+      if (first && s.best_id != best_id) break;
+    } else {
+      closest_node<kCount>(bvh, r, st, s, cnt);
+    }
   }
   best_t = s.best_t;
   best_id = s.best_id;
   best_u = s.best_u;
-}
-
-// Any hit with t > 0 over hair segments (binary visibility); children are
-// taken in slot order.
-struct AnyState {
-  int cur;
-  bool hit;
-};
-
-HM_D void any_begin(const BvhView& bvh, TraceStack& st, AnyState& s) {
-  st.clear();
-  s.cur = bvh.num_segs > 0 ? 0 : kNone;
-  s.hit = false;
-}
-
-template <bool kCount>
-HM_D void any_node(const BvhView& bvh, const RayInv& r, TraceStack& st, AnyState& s, TraceCounters& cnt) {
-  if (kCount) cnt.nodes++;
-  const float tinf = __builtin_inff();
-  float t[4];
-  int c[4];
-  node_boxes(bvh, r, s.cur, tinf, t, c);
-  int next = kNone;
-  if (st.room3()) {
-    next = t[3] < tinf ? c[3] : kNone;
-#pragma unroll
-    for (int k = 2; k >= 0; --k) {
-      const bool h = t[k] < tinf;
-      st.put(next, h && next != kNone);
-      next = h ? c[k] : next;
-    }
-    if (next == kNone && !st.empty()) next = st.pop_lds();
-  } else {
-#pragma unroll
-    for (int k = 3; k >= 0; --k) {
-      if (t[k] < tinf) {
-        if (next != kNone) st.push(next);
-        next = c[k];
-      }
-    }
-    if (next == kNone && !st.empty()) next = st.pop();
-  }
-  s.cur = next;
-}
-
-template <bool kCount, class Leaf>
-HM_D void any_leaf(const BvhView& bvh, const RayInv& r, TraceStack& st, AnyState& s, TraceCounters& cnt,
-                   const Leaf& leaf_test) {
-  const int code = ~s.cur, leaf = code & kLeafPosMask;
-  if (kCount) cnt.segs++;
-  float t, u;
-  int id;
-  if (leaf_test(bvh, r, leaf, &t, &u, &id)) {
-    s.hit = true;
-    s.cur = kNone;
-  } else {
-    s.cur = leaf_rest(code);
-    if (!s.cur) s.cur = st.empty() ? kNone : st.pop();
-  }
-}
-
-template <bool kCount, class Leaf = SegLeaf>
-HM_D bool trace_any(const BvhView& bvh, const RayInv& r, TraceStack& st, TraceCounters& cnt,
-                    const Leaf& leaf_test = Leaf{}) {
-  AnyState s;
-  any_begin(bvh, st, s);
-  for (int left = trace_cap(bvh); s.cur != kNone && left > 0; --left) {
-    if (s.cur < 0) any_leaf<kCount, Leaf>(bvh, r, st, s, cnt, leaf_test);
-    else any_node<kCount>(bvh, r, st, s, cnt);
-  }
-  return s.hit;
 }
 
 #endif  // __HIPCC__

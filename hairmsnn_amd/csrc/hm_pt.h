@@ -534,52 +534,6 @@ struct ShadowSink {
   }
 };
 
-// Closest hit against the head sphere and the hair BVH. The sphere is tested
-// first so its distance prunes the hair traversal; equal distances go to hair.
-// kCurves: the hair BVH holds round Catmull-Rom segments (sc.curves), a
-// separate instantiation so the linear-segment traversal keeps its registers.
-template <bool kCount, bool kCurves = false>
-HM_D void closest_hit(const SceneView& sc, V3 o, V3 d, TraceStack& st, float& t, int& prim, float& u,
-                      TraceCounters& cnt) {
-  t = __builtin_inff();
-  prim = kPrimMiss;
-  u = 0.f;
-  bool sphere_hit = false;
-  if (sc.sphere.enabled) {
-    float ts;
-    if (intersect_sphere(o, d, v3(sc.sphere.cx, sc.sphere.cy, sc.sphere.cz), sc.sphere.r, &ts)) {
-      t = ts;
-      sphere_hit = true;
-    }
-  }
-  const RayInv r = make_ray(o.x, o.y, o.z, d.x, d.y, d.z);
-  int tri = 0x7fffffff;
-  if (sc.mesh.num > 0) {
-    float bu = 0.f;
-    trace_closest<kCount, TriLeaf>(sc.mesh.bvh, r, st, t, tri, bu, cnt, TriLeaf{sc.mesh.tri});
-  }
-  int id = 0x7fffffff;
-  if constexpr (kCurves)
-    trace_closest<kCount, CurveLeaf>(sc.bvh, r, st, t, id, u, cnt, CurveLeaf{sc.curves, sc.curve_caps});
-  else
-    trace_closest<kCount>(sc.bvh, r, st, t, id, u, cnt);
-  if (id != 0x7fffffff) prim = id;
-  else if (tri != 0x7fffffff) prim = kPrimMesh0 - tri;
-  else if (sphere_hit) prim = kPrimSphere;
-}
-
-template <bool kCount, bool kCurves = false>
-HM_D bool occluded(const SceneView& sc, V3 o, V3 d, TraceStack& st, TraceCounters& cnt) {
-  if (sc.sphere.enabled) {
-    float ts;
-    if (intersect_sphere(o, d, v3(sc.sphere.cx, sc.sphere.cy, sc.sphere.cz), sc.sphere.r, &ts)) return true;
-  }
-  const RayInv r = make_ray(o.x, o.y, o.z, d.x, d.y, d.z);
-  if (sc.mesh.num > 0 && trace_any<kCount, TriLeaf>(sc.mesh.bvh, r, st, cnt, TriLeaf{sc.mesh.tri})) return true;
-  if constexpr (kCurves) return trace_any<kCount, CurveLeaf>(sc.bvh, r, st, cnt, CurveLeaf{sc.curves, sc.curve_caps});
-  return trace_any<kCount>(sc.bvh, r, st, cnt);
-}
-
 // ---- ray streams: one wave traces a list of rays -----------------------------
 //
 // What bounds traversal is how many of a wave's lanes do useful work: with
@@ -592,8 +546,10 @@ HM_D bool occluded(const SceneView& sc, V3 o, V3 d, TraceStack& st, TraceCounter
 // wave's next rays, from a position in a scalar register: no atomics. And
 // each iteration executes either the node step or the primitive step, whichever
 // enough lanes are ready for (the Leaf's kNodes); the others wait. A ray's own
-// steps and their order are those of trace_closest / trace_any, so its result
-// does not depend on the schedule.
+// steps and their order do not depend on the schedule, and neither does its
+// result. A head mesh is searched when a lane takes a ray, before its hair
+// steps, and its distance then prunes them (as the head sphere's does; equal
+// distances go to the hair).
 //
 // A launch takes the next wavefront's closest-hit rays and the light rays of
 // the vertices just shaded together: they do not depend on each other, and
@@ -649,9 +605,9 @@ HM_D bool leaf_turn(unsigned long long at_leaf, unsigned long long at_node) {
 
 // Hits of n_closest + n_any rays: load(i, o, d) gives ray i; the first
 // n_closest are closest-hit queries (store_hit(i, t, prim, u), the sphere and
-// the head mesh included, as closest_hit), the others any-hit ones
-// (store_any(i, hit)). An any-hit query runs the same steps and ends at its
-// first hit. cnt: counters of the closest and of the any-hit rays.
+// the head mesh included), the others any-hit ones (store_any(i, hit)). An
+// any-hit query runs the same steps and ends at its first hit, in the mesh or
+// the hair. cnt: counters of the closest and of the any-hit rays.
 template <bool kCount, class Leaf, class Load, class StoreHit, class StoreAny>
 HM_D void trace_stream(const SceneView& sc, TraceStack& st, int n_closest, int n_any, const Leaf& leaf,
                        TraceCounters cnt[2], Load load, StoreHit store_hit, StoreAny store_any) {
@@ -692,7 +648,7 @@ HM_D void trace_stream(const SceneView& sc, TraceStack& st, int n_closest, int n
           if (sc.mesh.num > 0 && !(any && other != kPrimMiss)) {
             float bu = 0.f;
             int tri = kNone;
-            trace_closest<kCount, TriLeaf>(sc.mesh.bvh, r, st, s.best_t, tri, bu, cnt[any], TriLeaf{sc.mesh.tri});
+            trace_closest<kCount>(sc.mesh.bvh, r, st, s.best_t, tri, bu, any, cnt[any], TriLeaf{sc.mesh.tri});
             if (tri != kNone) other = kPrimMesh0 - tri;
           }
           closest_begin(sc.bvh, st, s);

@@ -197,3 +197,23 @@ def test_ray_stream_lengths_bit_exact(gpu, n):
     np.testing.assert_array_equal(t[hit], t_c[hit])
     np.testing.assert_array_equal(u[hit], u_c[hit])
     np.testing.assert_array_equal(any_hit, hit.astype(np.int32))
+
+
+def test_any_hit_with_a_head_mesh(gpu, tmp_path):
+    """Shadow rays against an OBJ head under the hair stop at their first hit,
+    in the mesh or in the hair: occluded exactly where the closest-hit query
+    finds something."""
+    from tests.objfile import icosphere, write_obj
+    p = tmp_path / "head.obj"
+    write_obj(p, *icosphere(4, radius=0.95))
+    cfg = json.loads((SCENES / "c0_hairball.json").read_text())
+    cfg["integrator"].update({"width": 128, "height": 128})
+    cfg["surface"] = {"geometry": str(p)}
+    with gpu.Scene(json_text=cfg) as sc:
+        rays = make_rays(sc.segments(), 30_001, 31)
+        prim, t, _ = sc.trace_rays(rays)
+        occ = sc.trace_rays(rays, any_hit=True)
+    head = prim < -2
+    print(f"mesh {head.mean():.3f} hair {(prim >= 0).mean():.3f}")
+    assert head.mean() > 0.1 and (prim >= 0).mean() > 0.1 and (prim == -1).mean() > 0.1
+    np.testing.assert_array_equal(occ, (prim != -1).astype(np.int32))
