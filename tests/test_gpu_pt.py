@@ -134,25 +134,29 @@ def test_converges_to_fp64_oracle(gpu):
     assert abs(gm - om) < 4 * se_m
 
 
-@pytest.mark.parametrize("name,groups,calls,size", [("c0_hairball.json", 1, (5, 3), (64, 64)),
-                                                    ("c0_hairball.json", 3, (5, 3), (64, 64)),
-                                                    ("c1_curly.json", 4, (5, 3), (64, 64)),
-                                                    ("c0_hairball.json", 4, (40, 19), (64, 64)),
-                                                    ("c0_hairball.json", 4, (6, 2), (48, 40))])
-def test_streaming_schedule_equals_pass_schedule(gpu, name, groups, calls, size):
+@pytest.mark.parametrize("name,limit,calls,size", [("c0_hairball.json", 1, (5, 3), (64, 64)),
+                                                   ("c1_curly.json", 4, (5, 3), (64, 64)),
+                                                   ("c0_hairball.json", 1, (40, 19), (64, 64)),
+                                                   ("c0_hairball.json", 4, (6, 2), (48, 40)),
+                                                   ("c1_curly.json", 2, (16, 9), (512, 256)),
+                                                   ("c0_hairball.json", 4, (16, 3, 40), (512, 256))])
+def test_streaming_schedule_equals_pass_schedule(gpu, name, limit, calls, size):
     """The streaming schedule (slots take (pass, pixel) jobs in pass order over
-    a compacted wavefront, two paths in flight per pixel of each of `groups`
-    streams; finished radiance waits in a 16-pass ring until its pass is
-    complete) accumulates each pixel's passes in pass order, so its image is
-    the per-pass schedule's bit for bit, across calls, seed offsets, calls
-    longer than the ring and groups of unequal size (48 x 40: 30 chunks of
-    64 pixels over 4 groups)."""
+    a compacted wavefront; finished radiance waits in a 16-pass ring until its
+    pass is complete) accumulates each pixel's passes in pass order, so its
+    image is the per-pass schedule's bit for bit, across calls, seed offsets and
+    calls longer than the ring. set_pass_concurrency(limit): one group of pixels
+    below 2^20 jobs (the 64 x 64 and 48 x 40 rows, whatever the limit, and the
+    call of 3 in the last row), two from there on where the limit allows it
+    (512 x 256 from 8 passes on; scenes hold a multiple of 128 pixels, so two
+    groups of 64-pixel chunks are equal). The per-pass schedule keeps `limit`
+    passes in flight."""
     cfg = scene_cfg(name, *size)
     imgs, lasts = {}, {}
     for sched in ("passes", "stream"):
         with gpu.Scene(json_text=cfg) as sc:
             sc.set_pt_schedule(sched)
-            sc.set_pass_concurrency(groups)
+            sc.set_pass_concurrency(limit)
             sc.set_seed_offset(3)
             sc.pt_reset()
             for n in calls:
@@ -168,12 +172,11 @@ def test_streaming_schedule_equals_pass_schedule(gpu, name, groups, calls, size)
 @pytest.mark.parametrize("calls", [(15,), (16,), (3, 33)])
 def test_streaming_schedule_two_groups(gpu, calls, groups):
     """Calls on both sides of the 2^20 jobs from which the streaming schedule
-    deals its pixels to two groups where it may (128 x 513 has 1026 chunks of 64 pixels,
-    16 passes are the first call above), with the buffers of a small image
-    holding every pass the ring allows: the per-pass schedule's image, bit for
-    bit."""
+    deals its pixels to two groups where it may (128 x 513 has 1026 chunks of 64
+    pixels, 16 passes are the first call above): the per-pass schedule's image
+    and last pass, bit for bit."""
     cfg = scene_cfg("c0_hairball.json", 128, 513)
-    imgs = {}
+    imgs, lasts = {}, {}
     for sched in ("passes", "stream"):
         with gpu.Scene(json_text=cfg) as sc:
             sc.set_pt_schedule(sched)
@@ -183,7 +186,9 @@ def test_streaming_schedule_two_groups(gpu, calls, groups):
             for n in calls:
                 sc.pt_passes(n)
             imgs[sched] = sc.image(0).copy()
+            lasts[sched] = sc.last_pass().copy()
     np.testing.assert_array_equal(imgs["stream"], imgs["passes"])
+    np.testing.assert_array_equal(lasts["stream"], lasts["passes"])
 
 
 @pytest.mark.parametrize("name,size,path_v2,groups,calls", [("c1_curly.json", (256, 256), 40, 1, (20, 2)),
