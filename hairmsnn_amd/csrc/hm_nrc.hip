@@ -90,9 +90,13 @@ struct NrcState {
   // share them (20 frames of 256 x 256: 11.8 ms one by one on four slots, 4.4
   // ms at 8 to a pass, 3.5 ms at 16, 4.0 ms at 32). Two slots overlap one
   // pass's last depths with the next one's first; a call of at least
-  // kSplitPaths paths is two passes or more for that (8 frames of 512 x 512:
-  // 24.4 ms one by one, 11.4 ms in one pass, 10.8 ms in two; 9.7 ms since short
-  // ray lists spread over all waves).
+  // kSplitPaths paths is two passes or more for that. On the headline groom,
+  // one pass against two: a quarter of a million paths 5.6 and 5.6 ms, half a
+  // million 6.9 and 6.6, one million (384 x 384, 8 frames) 8.9 and 8.3, two
+  // million (512 x 512, 8 frames) 11.4 and 10.8, three 15.0 and 14.1, four 18.4
+  // and 17.2. The line is higher than where two begin to win because a process
+  // whose streams leave the two slots one hardware queue loses more than that
+  // (two million paths: 15.6 ms), and smaller calls have less to win.
   static constexpr int kSlots = 2, kBatch = 16;
   static constexpr int kBatchPaths = 4 << 20, kSplitPaths = 2 << 20;
   NrcSlot slots[kSlots];
@@ -259,7 +263,7 @@ int nrc_alloc_slot(Context& c, const NrcState& m, NrcSlot& sl, int frames, std::
     sl.allocs.push_back(*p);
     return kOk;
   };
-  HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
+  if (!sl.st) HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
   for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
     HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
   HM_TRY(alloc_path_buffers(sl.pb, sl.allocs, npx, true, c.stack_levels(), c.trace_blocks * kTraceBlock, sl.st, err));
@@ -290,11 +294,15 @@ int nrc_batch(Context& c, NrcState& m, int frames) {
     if (sl.frames >= want) continue;
     NrcSlot grown;
     std::string err;
+    grown.st = sl.st;  // the stream stays, and with it the hardware queue it got
     if (nrc_alloc_slot(c, m, grown, want, err)) {
+      if (sl.st) grown.st = nullptr;
       grown.release();
       (void)hipGetLastError();
       break;
     }
+    if (sl.st) (void)hipStreamSynchronize(sl.st);
+    sl.st = nullptr;
     sl.release();
     sl = std::move(grown);
     if (m.last_slot == k) m.last_slot = -1;

@@ -168,13 +168,14 @@ constexpr int kStreamRing = 16;
 // Stream groups: one, and two where the caller asks for concurrency
 // (hmsnn_set_pass_concurrency) and there are kTwoGroupJobs jobs. Two groups'
 // launches fill each other's tails where their streams have a hardware queue
-// each (16 passes of the headline frame 63 ms against 67, a 640 x 363 frame of
-// round curves 15.6 against 16.2), which depends on every stream the process
-// has made: in one that had rendered other scenes before, the same two groups
-// took 70 to 74 and 21 to 23 ms, and 256 x 256 at 16 passes 3.4 to 3.8 ms
-// against 2.5. More than two only share the queues. Below kTwoGroupJobs two
-// shorter wavefronts drain in as many launches each (128 x 128, 4 passes: 1.28
-// against 1.48 ms; 256 x 256, 16 passes: level).
+// each (16 passes of the headline frame 62.3 ms against 65.4), which depends on
+// every stream the process has made: in one that had rendered other scenes
+// before, the same two groups took 70 to 74 ms, and 256 x 256 at 16 passes 3.4
+// to 3.8 ms against 2.5. More than two only share the queues. One group against
+// two with a queue each, headline groom: 0.12 M jobs 5.67 and 5.73 ms, 0.25 M
+// 6.17 and 6.22, 0.5 M 7.49 and 7.31, 1 M 9.52 and 9.13, 2 M 13.0 and 12.8, 6 M
+// 29.0 and 27.7; a sparse ball of 64 K jobs 1.28 and 1.48. The line is where the
+// gain passes the spread between processes.
 constexpr int kStreamGroups = 2;
 constexpr long long kTwoGroupJobs = 1 << 20;
 // Paths in flight over all groups. A launch ends with its longest rays, so

@@ -4,6 +4,7 @@ and, for HBM traffic, the per-kernel JSON that bench.py reads.
     python -m hairmsnn_amd.profile_summary trace RUN.db
     python -m hairmsnn_amd.profile_summary calls RUN.db KERNEL [KERNEL ...]
     python -m hairmsnn_amd.profile_summary pmc RUN.db
+    python -m hairmsnn_amd.profile_summary valu RUN.db --json out.json
     python -m hairmsnn_amd.profile_summary flops RUN.db [RUN.db ...] --json out.json
     python -m hairmsnn_amd.profile_summary traffic --fetch F.db --write W.db \
         --copy-fetch CF.db --copy-write CW.db --copy-mib 1024 --json out.json
@@ -19,7 +20,10 @@ reads and writes that many bytes), giving HBM bytes per launch. flops:
 FP32 VALU operations per launch (SQ_INSTS_VALU_FLOPS_FP32 and its
 transcendental counterpart count per wave instruction, so x 64 lanes) and
 matrix-core operations (SQ_INSTS_VALU_MFMA_MOPS_* x 512), with the rate over
-each launch's mean duration.
+each launch's mean duration. valu: the share of the SIMDs' cycles in which
+vector instructions issue (SQ_ACTIVE_INST_VALU, in quarter-wave quads of four
+cycles, over GRBM_GUI_ACTIVE / 8 XCDs x SIMDs) and the lanes active in them
+(SQ_THREAD_CYCLES_VALU / 64 of that), over a kernel's launches.
 """
 from __future__ import annotations
 
@@ -177,6 +181,23 @@ def cmd_pmc(a) -> None:
         print(f"| {k} | {int(v['_launches'])} | {v['_us']:.1f} | {vals} |")
 
 
+def cmd_valu(a) -> None:
+    out = {}
+    print("| kernel | launches | avg us | VALU busy % | lanes active % |")
+    print("|---|---:|---:|---:|---:|")
+    cs = counters(a.db)
+    for k, v in sorted(cs.items(), key=lambda kv: -kv[1]["_us"] * kv[1]["_launches"])[: a.top]:
+        act, gui = v.get("SQ_ACTIVE_INST_VALU", 0.0), v.get("GRBM_GUI_ACTIVE", 0.0)
+        if not act or not gui:
+            continue
+        busy = 4.0 * act / (gui / 8.0 * a.simds)
+        lanes = v["SQ_THREAD_CYCLES_VALU"] / (64.0 * act)
+        out[k] = {"launches": int(v["_launches"]), "valu_busy": busy, "lanes_active": lanes}
+        print(f"| {k} | {int(v['_launches'])} | {v['_us']:.1f} | {100 * busy:.1f} | {100 * lanes:.1f} |")
+    if a.json:
+        Path(a.json).write_text(json.dumps({"workload": a.workload, "kernels": out}, indent=1) + "\n")
+
+
 def cmd_flops(a) -> None:
     per: dict[str, dict[str, float]] = {}
     for db in a.dbs:
@@ -267,6 +288,12 @@ def main(argv=None) -> None:
     p = sub.add_parser("pmc")
     p.add_argument("db")
     p.add_argument("--top", type=int, default=12)
+    va = sub.add_parser("valu")
+    va.add_argument("db")
+    va.add_argument("--json")
+    va.add_argument("--workload", default="")
+    va.add_argument("--simds", type=int, default=1024)
+    va.add_argument("--top", type=int, default=12)
     fl = sub.add_parser("flops")
     fl.add_argument("dbs", nargs="+")
     fl.add_argument("--json")
@@ -287,7 +314,7 @@ def main(argv=None) -> None:
     f.add_argument("--top", type=int, default=12)
     a = ap.parse_args(argv)
     {"trace": cmd_trace, "calls": cmd_calls, "pmc": cmd_pmc, "flops": cmd_flops, "traffic": cmd_traffic,
-     "mfma": cmd_mfma}[a.cmd](a)
+     "mfma": cmd_mfma, "valu": cmd_valu}[a.cmd](a)
 
 
 if __name__ == "__main__":

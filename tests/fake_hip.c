@@ -4,10 +4,12 @@
 #include <stdlib.h>
 #include <string.h>
 
-static long live, fail_after = -1;
+static long live, fail_after = -1, streams;
 static size_t bytes_live, bytes_limit;
 
 long fake_live(void) { return live; }
+/* streams created so far */
+long fake_streams(void) { return streams; }
 size_t fake_bytes(void) { return bytes_live; }
 /* the allocation after the next n fails, once (n < 0: none) */
 void fake_fail_after(long n) { fail_after = n; }
@@ -43,7 +45,7 @@ int hipMemsetAsync(void* d, int v, size_t n, void* st) { memset(d, v, n); return
 static int handle(void** p) { *p = (void*)1; return 0; }
 int hipEventCreate(void** e) { return handle(e); }
 int hipEventCreateWithFlags(void** e, unsigned f) { return handle(e); }
-int hipStreamCreateWithFlags(void** s, unsigned f) { return handle(s); }
+int hipStreamCreateWithFlags(void** s, unsigned f) { streams++; return handle(s); }
 int hipEventDestroy(void* e) { return 0; }
 int hipEventElapsedTime(float* ms, void* a, void* b) { *ms = 0; return 0; }
 int hipEventRecord(void* e, void* s) { return 0; }

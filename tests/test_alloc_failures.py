@@ -1,6 +1,8 @@
-"""What the contexts do when the device has no memory left, and after a begin
-that failed, on the CPU: the library runs on tests/fake_hip.c (host memory, launches that do nothing), which
-fails allocations on request. The script runs in a process of its own."""
+"""What the contexts do with their buffers and streams, on the CPU: when the
+device has no memory left, after a begin that failed, when they grow. The
+library runs on tests/fake_hip.c (host memory, launches that do nothing), which
+fails allocations on request and counts them. Each script runs in a process of
+its own."""
 import json
 import subprocess
 import sys
@@ -125,3 +127,17 @@ print(json.dumps(dict(first=first, bad=bad, image=image, last=last, left=fake.fa
     print(out)
     assert not out["first"] and not out["last"] and out["left"] == 0
     assert "EIO" in out["bad"] and "EINVAL" in out["image"]
+
+
+def test_nrc_slots_keep_their_stream_when_they_grow(fake):
+    """Calls of more frames make larger slots. They stay on the stream they had:
+    which hardware queue a stream shares is settled when it is made, and a
+    second stream on the first one's queue cost up to 1.4 times. A growth that
+    finds no memory leaves the slot and its stream as they were."""
+    out = fake('''
+sc = scene(); sc.nrc_begin(); sc.nrc_frames(1); a = fake.fake_streams()
+sc.nrc_frames(3); sc.nrc_frames(9); b = fake.fake_streams()
+fake.fake_fail_after(5); sc.nrc_frames(16); fake.fake_fail_after(-1); sc.nrc_frames(2); sc.close()
+print(json.dumps(dict(a=a, b=b, left=fake.fake_live())))
+''')
+    assert out["a"] == out["b"] and out["left"] == 0
