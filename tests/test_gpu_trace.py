@@ -217,3 +217,49 @@ def test_any_hit_with_a_head_mesh(gpu, tmp_path):
     print(f"mesh {head.mean():.3f} hair {(prim >= 0).mean():.3f}")
     assert head.mean() > 0.1 and (prim >= 0).mean() > 0.1 and (prim == -1).mean() > 0.1
     np.testing.assert_array_equal(occ, (prim != -1).astype(np.int32))
+
+
+@pytest.mark.parametrize("offset,scale", [(0.0, 1e-3), (300.0, 1.0), (-1e5, 50.0), (2e6, 3e4)])
+def test_grooms_off_the_origin_bit_exact(gpu, tmp_path, offset, scale):
+    """The 8-bit child boxes are steps from each node's corner, widened by the
+    rounding of coordinates and distances: a groom far from the origin or of
+    another scale, with rays from nearby and from afar, still finds what the
+    brute-force search finds, bit for bit."""
+    from tests.hairfile import write_hair
+    rng = np.random.default_rng(13)
+    strands = []
+    for k in range(150):
+        root = rng.normal(size=3)
+        root /= np.linalg.norm(root)
+        t = np.linspace(0, 1, 9)[:, None]
+        curl = 0.05 * np.stack([np.cos(9 * t[:, 0] + k), np.sin(9 * t[:, 0] + k), np.zeros(9)], -1)
+        strands.append((root * (1 + 0.6 * t) + curl) * scale + offset * np.array([1.0, -0.7, 0.3]))
+    p = tmp_path / "far.hair"
+    write_hair(p, strands, d_thickness=0.05 * scale)
+    cfg = json.loads((SCENES / "c0_hairball.json").read_text())
+    cfg["integrator"].update({"width": 128, "height": 128})
+    cfg["hair"] = {"geometry": str(p), "primitive": "linear", "tessellation": 2, "sigma_a": [0.06, 0.1, 0.2],
+                   "beta_m": 0.3, "beta_n": 0.3, "alpha": 2.0}
+    with gpu.Scene(json_text=cfg) as sc:
+        seg = sc.segments()
+        n = 6000
+        c = 0.5 * (seg[:, 0:3].min(0) + seg[:, 0:3].max(0)).astype(np.float64)
+        rays = np.zeros((n, 8), np.float32)
+        dist = np.where(np.arange(n) % 2 == 0, 4.0, 400.0)[:, None] * scale
+        o = c + unit_sphere(rng, n) * dist
+        tgt = c + unit_sphere(rng, n) * rng.uniform(0, 1.6, (n, 1)) * scale
+        rays[:, 0:3] = o
+        rays[:, 4:7] = (tgt - o) / np.linalg.norm(tgt - o, axis=1, keepdims=True)
+        k = n // 5  # from a point of a segment, parallel to an axis
+        rays[:k, 0:3] = seg[rng.integers(0, seg.shape[0], k), 0:3]
+        rays[:k, 4:7] = np.eye(3)[rng.integers(0, 3, k)] * rng.choice([-1.0, 1.0], (k, 1))
+        prim, t, u = sc.trace_rays(rays)
+        occ = sc.trace_rays(rays, any_hit=True)
+    prim_b, t_b, u_b = ol.intersect(seg, rays, use_bvh=False)
+    hit = prim_b >= 0
+    print(f"offset {offset} scale {scale}: hit fraction {hit.mean():.3f}")
+    assert 0.1 < hit.mean() < 0.95
+    np.testing.assert_array_equal(prim, prim_b)
+    np.testing.assert_array_equal(t[hit], t_b[hit])
+    np.testing.assert_array_equal(u[hit], u_b[hit])
+    np.testing.assert_array_equal(occ, hit.astype(np.int32))
