@@ -17,7 +17,10 @@ visited x 64 B + segments tested x 32 B + ray in / hit out (48 B closest,
 per vertex 56 B of path state read, per continuing vertex 60 B more read
 (hit, RNG, throughput, segment) and 92 B moved into the next wavefront, per
 finished path 36 B, per shadow ray 52 B written. HBM traffic per launch comes
-from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs summarised in profiles/.
+from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs summarised in profiles/. The
+rate is that of the algorithmic bytes, most of which the caches serve; what
+bounds the traversal is the issue of vector instructions (`bound`, with the
+counters behind it).
 
 CPU baseline: the C++ oracle (FP32 twin of the reference integrator, OpenMP)
 on a bounded crop of the same scene, run on this machine's host cores.
@@ -55,6 +58,7 @@ PASS_KERNELS = {"extend": "k_trace<false, true, false> (closest hits)", "shade":
 # FP32 VALU operations per launch (rocprofv3 SQ_INSTS_VALU_FLOPS_FP32 x 64
 # lanes) of the pass kernels and of the BSDF streams, for the VALU FLOP rates
 FLOPS_JSON = ROOT / "profiles" / "pt_c1_1024_flops.json"
+VALU_JSON = ROOT / "profiles" / "pt_c1_1024_valu.json"
 KERNEL_FLOPS_JSON = ROOT / "profiles" / "bsdf_mlp_flops.json"
 VALU_FP32_PEAK_TFLOPS = 157.3
 
@@ -386,6 +390,16 @@ def mlp_train_rate(hm, n: int = 1 << 16, reps: int = 20) -> dict:
     return {"records": n, "ms": dt * 1e3, "TFLOP/s": tf, "peak_TFLOP/s": 2500.0, "frac": tf / 2500.0}
 
 
+def valu_counters() -> dict:
+    """Share of the SIMDs' cycles that issue vector instructions and of the
+    lanes active in them, of the traversal kernel (a rocprofv3 counter run of
+    this workload)."""
+    if not VALU_JSON.exists():
+        return {}
+    k = json.loads(VALU_JSON.read_text())["kernels"].get("k_trace<false, true, false>", {})
+    return {"valu_busy": k.get("valu_busy"), "valu_lanes_active": k.get("lanes_active")}
+
+
 def main() -> None:
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -398,7 +412,9 @@ def main() -> None:
     ap.add_argument("--schedule", choices=("stream", "passes"), default="stream",
                     help="path-tracing schedule: stream (a pixel's next pass starts when its path ends) or passes "
                          "(one wavefront per pass, --pass-concurrency of them in flight)")
-    ap.add_argument("--pass-concurrency", type=int, default=4, help="passes in flight with --schedule passes")
+    ap.add_argument("--pass-concurrency", type=int, default=0,
+                    help="passes in flight with --schedule passes, stream groups at most with --schedule stream "
+                         "(default: the library's own, 4 and 1)")
     ap.add_argument("--copy-mib", type=int, default=0,
                     help="instead of the benchmark, run 8 device-to-device copies of this many MiB (the known-size "
                          "kernel that calibrates rocprofv3 FETCH_SIZE / WRITE_SIZE)")
@@ -447,9 +463,18 @@ def main() -> None:
     # counting pass (not timed): algorithmic traversal bytes
     stats = sc.trace_stats(1)
     log(f"trace stats (1 pass): {stats}")
-    # warmup
+    # per-kernel timing with HIP events on the stream each kernel runs on, every
+    # launch running alone (streaming: one stream; passes: one pass in flight);
+    # it also makes the path buffers of a long call, which stays out of the
+    # timed region then
     sc.set_pt_schedule(args.schedule)
-    sc.set_pass_concurrency(args.pass_concurrency)
+    sc.set_pass_concurrency(1)
+    passes_t = max(2, min(16, args.steps))
+    sc.pt_reset()
+    sc.time_passes(1)
+    kt = sc.time_passes(passes_t)
+    # warmup
+    sc.set_pass_concurrency(args.pass_concurrency or (4 if args.schedule == "passes" else 1))
     sc.pt_reset()
     sc.pt_passes(args.warmup)
     # timed region: K passes, synchronised on both sides
@@ -461,12 +486,6 @@ def main() -> None:
     value = paths_per_step * args.steps / wall
     log(f"{args.steps} passes in {wall:.3f} s -> {value / 1e6:.2f} M paths/s")
 
-    # per-kernel timing with HIP events on the stream each kernel runs on, every
-    # launch running alone (streaming: one stream; passes: one pass in flight)
-    sc.set_pass_concurrency(1)
-    passes_t = max(2, min(16, args.steps))
-    kt = sc.time_passes(passes_t)
-    sc.set_pass_concurrency(args.pass_concurrency)
     launches = max(kt["extend_launches"], 1)
     launches_pass = launches / passes_t
     V, P, S = stats["closest_rays"], float(paths_per_step), stats["any_rays"]
@@ -476,20 +495,21 @@ def main() -> None:
                   + P * SHADE_DONE_BYTES + S * SHADE_SHADOW_BYTES),
         "shadow": stats["any_nodes"] * NODE_BYTES + stats["any_segs"] * SEG_BYTES + S * ANY_RAY_BYTES,
     }
-    traffic_k = {}
-    if TRAFFIC_JSON.exists():
-        traffic_k = json.loads(TRAFFIC_JSON.read_text()).get("kernels", {})
-    flops_k = {}
-    if FLOPS_JSON.exists():
-        flops_k = json.loads(FLOPS_JSON.read_text()).get("kernels", {})
+    def counted(path: Path, kname: str, key: str):
+        """A counter run's amount per launch of this run: its mean over all
+        launches of its passes, by passes (shorter calls launch more often)."""
+        d = json.loads(path.read_text()) if path.exists() else {}
+        k = d.get("kernels", {}).get(kname)
+        return k[key] * k["launches"] / d["passes"] / launches_pass if k and d.get("passes") else None
+
     per_kernel = {}
     for k, kname in PASS_KERNELS.items():
         ms_pass = kt[f"{k}_ms"] / passes_t
         ms_launch = ms_pass / launches_pass
         b_launch = alg_pass[k] / launches_pass
         ach = b_launch / (ms_launch * 1e-3) / 1e9
-        tr = traffic_k.get(kname, {}).get("traffic_bytes_per_launch")
-        fl = flops_k.get(kname, {}).get("valu_flops_per_launch")
+        tr = counted(TRAFFIC_JSON, kname, "traffic_bytes_per_launch")
+        fl = counted(FLOPS_JSON, kname, "valu_flops_per_launch")
         per_kernel[k] = {"kernel": kname, "ms_per_pass": ms_pass, "ms_per_launch": ms_launch,
                          "bytes_per_launch": b_launch, "achieved": ach, "frac": ach / HBM_PEAK_GBS, "traffic": tr,
                          "traffic_GBps": tr / (ms_launch * 1e-3) / 1e9 if tr else None,
@@ -523,9 +543,11 @@ def main() -> None:
             "segments": int(sc.info["num_segments"]), "bvh_depth": int(sc.info["bvh_depth"]),
         },
         "roofline": {
-            "bound": "hbm", "achieved": d["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "bound": "valu", "bound_source": "profiles/pt_c1_1024_valu.md", **valu_counters(),
+            "rate": "algorithmic bytes against the HBM peak", "achieved": d["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": d["frac"], "traffic": d["traffic"], "kernel": d["kernel"],
-            "traffic_source": "rocprofv3 FETCH_SIZE/WRITE_SIZE, profiles/pt_c1_1024_hbm_traffic.md",
+            "traffic_source": "rocprofv3 FETCH_SIZE/WRITE_SIZE, profiles/pt_c1_1024_hbm_traffic.md (of "
+                              "k_trace counted over launches of both kinds of rays)",
             "bytes_per_launch": d["bytes_per_launch"], "ms_per_launch": d["ms_per_launch"],
             "nodes_per_ray": stats["closest_nodes"] / max(stats["closest_rays"], 1),
             "segs_per_ray": stats["closest_segs"] / max(stats["closest_rays"], 1),

@@ -218,7 +218,8 @@ def cmd_flops(a) -> None:
             print(f"| {k} | {int(v['_launches'])} | {us:.1f} | {valu / 1e9:.3f} | {valu / (us * 1e-6) / 1e12:.1f} | "
                   f"{mfma / 1e9:.3f} | {mfma / (us * 1e-6) / 1e12:.1f} |")
     if a.json:
-        Path(a.json).write_text(json.dumps({"workload": a.workload, "kernels": out}, indent=1) + "\n")
+        Path(a.json).write_text(json.dumps({"workload": a.workload, "passes": a.passes, "kernels": out}, indent=1)
+                                + "\n")
 
 
 def cmd_traffic(a) -> None:
@@ -250,7 +251,7 @@ def cmd_traffic(a) -> None:
             print(f"| {k} | {int(fetch[k]['_launches'])} | {us:.1f} | {fr / 1024:.1f} | {rb / 1e6:.1f} | "
                   f"{wr / 1024:.1f} | {wb / 1e6:.1f} | {(rb + wb) / (us * 1e-6) / 1e9:.0f} |")
     if a.json:
-        Path(a.json).write_text(json.dumps({"workload": a.workload, "fetch_scale": fetch_scale,
+        Path(a.json).write_text(json.dumps({"workload": a.workload, "passes": a.passes, "fetch_scale": fetch_scale,
                                             "write_scale": write_scale, "kernels": out}, indent=1) + "\n")
 
 
@@ -298,6 +299,7 @@ def main(argv=None) -> None:
     fl.add_argument("dbs", nargs="+")
     fl.add_argument("--json")
     fl.add_argument("--workload", default="")
+    fl.add_argument("--passes", type=int, default=0, help="rendering passes of the run, kept in the JSON")
     fl.add_argument("--top", type=int, default=12)
     mm = sub.add_parser("mfma")
     for n in ("--trace", "--fetch", "--write", "--mfma"):
@@ -311,6 +313,7 @@ def main(argv=None) -> None:
     f.add_argument("--copy-mib", type=int, required=True)
     f.add_argument("--json")
     f.add_argument("--workload", default="")
+    f.add_argument("--passes", type=int, default=0, help="rendering passes of the run, kept in the JSON")
     f.add_argument("--top", type=int, default=12)
     a = ap.parse_args(argv)
     {"trace": cmd_trace, "calls": cmd_calls, "pmc": cmd_pmc, "flops": cmd_flops, "traffic": cmd_traffic,
