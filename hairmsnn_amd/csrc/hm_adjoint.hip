@@ -138,9 +138,9 @@ HM_D void adj_vertex(const SceneView& sc, const AdjArgs& a, V3 o, V3 d, float t,
 }
 
 // Bound by its vector arithmetic (the dual-number evaluations carry six
-// tangents): 3.4 ms for the 13 M records of one of two groups. Two waves per
-// SIMD keep its registers (1, 2, 3 and 4 waves: 42.7, 40.9, 42.4 and 42.2 ms
-// for the whole 512 x 512, 16-pass step).
+// tangents): 6.7 ms for the 20 M records (4.85 a path) of a 512 x 512, 16-pass
+// step. Two waves per SIMD keep its registers (1, 2, 3 and 4 waves: 42.7, 40.9,
+// 42.4 and 42.2 ms for the whole step).
 __global__ void __launch_bounds__(256, 2) k_adjoint(SceneView sc, AdjArgs a, VertexTape tape,
                                                                    const long long* count) {
   const int npx = sc.width * sc.height;
