@@ -88,17 +88,15 @@ struct NrcState {
   // Frames of one pass: a pass's 40 depths are bound by their longest rays'
   // chains, about 0.14 ms each at any path count past the tenth, so frames
   // share them (20 frames of 256 x 256: 11.8 ms one by one on four slots, 4.4
-  // ms at 8 to a pass, 3.5 ms at 16, 4.0 ms at 32). Two slots overlap one
-  // pass's last depths with the next one's first; a call of at least
-  // kSplitPaths paths is two passes or more for that. On the headline groom,
-  // one pass against two: a quarter of a million paths 5.6 and 5.6 ms, half a
-  // million 6.9 and 6.6, one million (384 x 384, 8 frames) 8.9 and 8.3, two
-  // million (512 x 512, 8 frames) 11.4 and 10.8, three 15.0 and 14.1, four 18.4
-  // and 17.2. The line is higher than where two begin to win because a process
-  // whose streams leave the two slots one hardware queue loses more than that
-  // (two million paths: 15.6 ms), and smaller calls have less to win.
+  // ms at 8 to a pass, 3.5 ms at 16, 4.0 ms at 32). A call of more than
+  // kBatch frames or kBatchPaths paths is several passes, on two slots that
+  // overlap one pass's last depths with the next one's first. Splitting smaller
+  // calls for that overlap is not worth it: 8 frames of 512 x 512 took 9.6 ms
+  // in two passes and 10.1 in one, but the first ones of a scene 23.4 against
+  // 20.5 (the second slot's buffers), and 14.5 where the two slots' streams got
+  // one hardware queue; half a million paths 6.6 and 6.9, a quarter level.
   static constexpr int kSlots = 2, kBatch = 16;
-  static constexpr int kBatchPaths = 4 << 20, kSplitPaths = 2 << 20;
+  static constexpr int kBatchPaths = 4 << 20;
   NrcSlot slots[kSlots];
   int next_slot = 0, last_slot = -1, last_frame = 0;  // the last frame: its slot and place there
   // shared, used in frame order on the context stream
@@ -255,7 +253,8 @@ float nrc_lr_at(float base, int step) {
   return base * std::pow(0.33f, (float)((step - 4000) / 4000 + 1));
 }
 
-// Buffers, stream and events of a slot for passes of `frames` frames.
+// Buffers and events of a slot, which has its stream, for passes of `frames`
+// frames.
 int nrc_alloc_slot(Context& c, const NrcState& m, NrcSlot& sl, int frames, std::string& err) {
   const size_t npx = (size_t)m.frame_size * frames, tpx = (size_t)m.n_tpx * frames;
   auto S = [&](void** p, size_t bytes) -> int {
@@ -263,7 +262,6 @@ int nrc_alloc_slot(Context& c, const NrcState& m, NrcSlot& sl, int frames, std::
     sl.allocs.push_back(*p);
     return kOk;
   };
-  if (!sl.st) HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
   for (hipEvent_t* e : {&sl.ev_gb, &sl.ev_done, &sl.ev_copy})
     HM_HIP(hipEventCreateWithFlags(e, hipEventDisableTiming), err);
   HM_TRY(alloc_path_buffers(sl.pb, sl.allocs, npx, true, c.stack_levels(), c.trace_blocks * kTraceBlock, sl.st, err));
@@ -287,8 +285,7 @@ int nrc_alloc_slot(Context& c, const NrcState& m, NrcSlot& sl, int frames, std::
 // (nrc_setup made one for single frames). No slot has work in flight.
 int nrc_batch(Context& c, NrcState& m, int frames) {
   const int cap = std::clamp(NrcState::kBatchPaths / m.frame_size, 1, NrcState::kBatch);
-  const int least = frames > 1 && (long long)frames * m.frame_size >= NrcState::kSplitPaths ? 2 : 1;
-  const int batches = std::max(least, (frames - 1) / cap + 1), want = (frames - 1) / batches + 1;
+  const int batches = (frames - 1) / cap + 1, want = (frames - 1) / batches + 1;
   for (int k = 0; k < std::min(NrcState::kSlots, batches); ++k) {
     NrcSlot& sl = m.slots[k];
     if (sl.frames >= want) continue;
@@ -296,12 +293,13 @@ int nrc_batch(Context& c, NrcState& m, int frames) {
     std::string err;
     grown.st = sl.st;  // the stream stays, and with it the hardware queue it got
     if (nrc_alloc_slot(c, m, grown, want, err)) {
-      if (sl.st) grown.st = nullptr;
+      (void)hipStreamSynchronize(grown.st);
+      grown.st = nullptr;
       grown.release();
       (void)hipGetLastError();
       break;
     }
-    if (sl.st) (void)hipStreamSynchronize(sl.st);
+    (void)hipStreamSynchronize(sl.st);
     sl.st = nullptr;
     sl.release();
     sl = std::move(grown);
@@ -318,6 +316,13 @@ int nrc_alloc(Context& c, NrcState& m, std::string& err) {
     m.allocs.push_back(*p);
     return kOk;
   };
+  // The slots' passes overlap only on hardware queues of their own, and which
+  // one a stream gets is settled when it is made: two streams made in a row
+  // mostly get different ones (two of 24 histories of scenes opened, rendered
+  // and closed before did not; seven where the second stream was made with its
+  // slot's first pass. One queue for both costs two passes of 4M paths 19.4 ms
+  // against 15.4).
+  for (NrcSlot& sl : m.slots) HM_HIP(hipStreamCreateWithFlags(&sl.st, hipStreamNonBlocking), err);
   HM_TRY(nrc_alloc_slot(c, m, m.slots[0], 1, err));
   HM_TRY(A((void**)&m.cache, sizeof(float) * 3 * (size_t)m.n_query));
   HM_TRY(A((void**)&m.gb_rad, sizeof(float4) * (size_t)npx));

@@ -130,10 +130,9 @@ print(json.dumps(dict(first=first, bad=bad, image=image, last=last, left=fake.fa
 
 
 def test_nrc_slots_keep_their_stream_when_they_grow(fake):
-    """Calls of more frames make larger slots. They stay on the stream they had:
-    which hardware queue a stream shares is settled when it is made, and a
-    second stream on the first one's queue cost up to 1.4 times. A growth that
-    finds no memory leaves the slot and its stream as they were."""
+    """Calls of more frames make larger slots. They stay on the streams made at
+    the begin, which mostly have a hardware queue each. A growth that finds no
+    memory leaves the slot and its stream as they were."""
     out = fake('''
 sc = scene(); sc.nrc_begin(); sc.nrc_frames(1); a = fake.fake_streams()
 sc.nrc_frames(3); sc.nrc_frames(9); b = fake.fake_streams()
