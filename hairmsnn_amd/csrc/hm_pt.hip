@@ -1172,6 +1172,7 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
         HM_HIP(hipEventSynchronize(live_ev[s]), err);
         if (live_host[2 * s + 1] == 0) {
           live[g] = 0;  // drained: never an error, however late
+          if (live_host[2 * s] == passes) last_poll[g] = -1;  // and all in the image
           continue;
         }
         if (iters[g] > max_iters) {
@@ -1181,7 +1182,8 @@ int pt_run_stream(const SceneView& sc, PathBuffers* const* pbs, const hipStream_
       }
     }
   }
-  // a drained group's last batch accumulated what was finished before it
+  // where a group drained in its batch's last iteration, the next batch has
+  // accumulated what that one finished
   for (int g = 0; g < K; ++g) {
     if (last_poll[g] < 0) continue;
     HM_HIP(hipEventSynchronize(live_ev[last_poll[g]]), err);

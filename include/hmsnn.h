@@ -203,8 +203,8 @@ int hmsnn_set_pt_schedule(hmsnn_ctx* ctx, int schedule);
 int hmsnn_pt_reset(hmsnn_ctx* ctx);
 /* Traces `passes` more samples per pixel into the accumulation buffers.
  * Asynchronous on the context's stream; hmsnn_ctx_synchronize waits. (The
- * streaming schedule polls its progress, returns once every pass is in the
- * image, and with HMSNN_EDEVICE if one is not.) */
+ * streaming schedule polls its progress, returns when every pass is in the
+ * image, and HMSNN_EDEVICE if one is not.) */
 int hmsnn_pt_passes(hmsnn_ctx* ctx, int passes);
 int hmsnn_ctx_synchronize(hmsnn_ctx* ctx);
 /* Samples accumulated so far (the reference's accumId). */
